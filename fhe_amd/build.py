@@ -22,9 +22,9 @@ ARCH = "gfx950"
 
 HOST_SOURCES = ["params.cpp"]
 HIP_SOURCES = ["ntt.hip", "ckks_kernels.hip", "ks_fused.hip", "automorphism.hip",
-               "elementwise.hip", "crypt.hip", "tensor_fused.hip",
+               "elementwise.hip", "crypt.hip",
                "encode.hip", "probe.hip", "context.hip", "engine.hip",
-               "wire.hip", "ks_wide.hip", "uneven_kernels.hip", "uneven.hip",
+               "wire.hip", "uneven_kernels.hip", "uneven.hip",
                "advanced.hip", "serve.hip", "noalloc.hip", "bk_kernels.hip",
                "bootstrap_key.hip"]
 # per-source flags: the encoder's double arithmetic must round every product

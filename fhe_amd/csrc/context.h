@@ -120,10 +120,6 @@ struct fhe_context {
   size_t workspace_bytes = 0;
   // lazy transforms where results are canonicalized before use
   bool lazy_key_switch = true;
-  // ModUp fused with the first NTT pass of the extended limbs
-  bool fuse_modup = false;
-  // input NTT second pass + tensor + trio INTT first pass in one kernel
-  bool fuse_tensor = false;
   // ModUp staged through the Garner digits (digits kernel + extension fused
   // with the first NTT pass)
   bool staged_modup = true;
@@ -139,14 +135,6 @@ struct fhe_context {
   hipEvent_t fork_event = nullptr, join_event = nullptr;
   // small-prime key products accumulated without guards, reduced once
   bool ks_lazy_accumulate = true;
-  // small-prime key products summed unreduced (96 bits), reduced once:
-  // about 10% fewer VALU instructions in the key inner product, but it
-  // issues them at a lower rate (measured slower), so off by default
-  bool ks_wide_accumulate = false;
-  // key inner product loads the next partition's tile ahead
-  bool ks_prefetch = false;
-  // waves per SIMD targeted by the key inner product's register allocation
-  int ks_occupancy = 2;
   // second growable device buffer (Garner digits of the staged ModUp)
   void *aux = nullptr;
   size_t aux_bytes = 0;
@@ -315,11 +303,25 @@ struct fhe_context {
     pending.clear();
   }
 
+  // Whether key switching at moduli_id takes the fused path, which holds
+  // every partition's extended limbs at once.  Below N = 2^16 it is left for
+  // chains so long that these would take more than kMaxExtLimbs limbs per
+  // ciphertext, and by callers with a fixed workspace (fused_key_switch).
+  static constexpr int kMaxExtLimbs = 1024;
+  bool fused_key_switch = true;
+  bool ks_fused(int moduli_id) const {
+    if (!fhe::ks_fused_supported(tables))
+      return false;
+    if (tables.log_n == 16)
+      return true;
+    return fused_key_switch && params.partition_count(moduli_id) *
+                                       (params.limbs_at(moduli_id) +
+                                        params.alpha) <= kMaxExtLimbs;
+  }
   // extended polynomials held at once by key switching: every partition on
   // the fused path, one at a time otherwise
   int ext_slots(int moduli_id) const {
-    return fhe::ks_fused_supported(tables) ? params.partition_count(moduli_id)
-                                           : 1;
+    return ks_fused(moduli_id) ? params.partition_count(moduli_id) : 1;
   }
 
   void require_not_capturing(const char *what) const {
@@ -685,7 +687,7 @@ struct fhe_context {
                   int64_t *ext, int64_t *acc, const int64_t *own = nullptr,
                   int64_t own_stride = 0, bool signed_input = false,
                   int64_t *digits = nullptr) {
-    if (fhe::ks_fused_supported(tables)) {
+    if (ks_fused(moduli_id)) {
       if (!own_limbs || int(params.partitions(moduli_id, key_moduli_id)
                                 .size()) > fhe::kMaxFusedParts)
         own = nullptr;
@@ -725,7 +727,7 @@ struct fhe_context {
                      ext_limbs, moduli_id, fhe::kInttExitReduce, stream);
   }
 
-  // The key-independent half of key switching on the fused path (N = 2^16):
+  // The key-independent half of key switching on the fused path (N = 2^13 .. 2^16):
   // ModUp of every partition and the first forward NTT pass of every
   // extended limb into ext [count][parts][ext][N] (CKKSCore::decompose,
   // src/ckks/core_key_switch.cpp:434-460, up to its second NTT pass).
@@ -782,15 +784,6 @@ struct fhe_context {
       });
       return;
     }
-    if (fuse_modup && fhe::modup_ntt_fused_supported(tables, max_size, np)) {
-      stage("modup_ntt_high(ext)", [&] {
-        fhe::launch_modup_ntt_fused(tables, src, src_stride, ext, count, limbs,
-                                    moduli_id, starts.data(), sizes.data(),
-                                    is_signed, np, cst, stride,
-                                    lazy_key_switch, stream);
-      });
-      return;
-    }
     for (int p = 0; p < np; p++)
       stage("modup", [&] {
         fhe::launch_modup(tables, src, src_stride,
@@ -833,8 +826,7 @@ struct fhe_context {
       fhe::launch_ks_inner_product_fused(
           tables, ext, key, key_chain, key_offset, parts[0].key_index, np, acc,
           count, ext_limbs, moduli_id, lazy_key_switch, own, own_stride,
-          starts.data(), sizes.data(), ks_lazy_accumulate, ks_wide_accumulate,
-          ks_prefetch, ks_occupancy, stream);
+          starts.data(), sizes.data(), ks_lazy_accumulate, stream);
     });
     stage("intt_pass_high(acc)", [&] {
       fhe::ntt_inverse_second(tables, acc, acc, int64_t(count) * 2 * ext_limbs,

@@ -166,26 +166,20 @@ int fhe_context_set_option(fhe_context *ctx, const char *name, int value) {
       ctx->lazy_key_switch = value != 0;
     else if (n == "staged_modup")
       ctx->staged_modup = value != 0;
-    else if (n == "fuse_modup")
-      ctx->fuse_modup = value != 0;
-    else if (n == "fuse_tensor")
-      ctx->fuse_tensor = value != 0;
     else if (n == "own_limbs")
       ctx->own_limbs = value != 0;
     else if (n == "overlap_trio")
       ctx->overlap_trio = value < 0 ? 0 : value > 2 ? 2 : value;
-    else if (n == "ks_occupancy")
-      ctx->ks_occupancy = value;
-    else if (n == "ks_prefetch")
-      ctx->ks_prefetch = value != 0;
     else if (n == "ks_lazy_accumulate")
       ctx->ks_lazy_accumulate = value != 0;
-    else if (n == "ks_wide_accumulate")
-      ctx->ks_wide_accumulate = value != 0;
     else if (n == "split_variants")
       ctx->tables.split_variants = value != 0 ? 1 : 0;
     else
-      require(false, "unknown option " + n);
+      // names of pipelines that the defaults have replaced: no effect
+      require(n == "fuse_modup" || n == "fuse_tensor" ||
+                  n == "ks_occupancy" || n == "ks_prefetch" ||
+                  n == "ks_wide_accumulate",
+              "unknown option " + n);
   });
 }
 
@@ -374,8 +368,7 @@ void hmult_relin_rescale_into(fhe_context *ctx, int count, int moduli_id,
         ctx->lazy_key_switch ? fhe::LazySpec{3, 2} : fhe::LazySpec();
     const bool overlap =
         ctx->overlap_trio && ctx->lazy_key_switch &&
-        fhe::ntt_parts_supported(ctx->tables) &&
-        !(ctx->fuse_tensor && fhe::tensor_fused_supported(ctx->tables));
+        fhe::ntt_parts_supported(ctx->tables);
     // once the side stream has forked, every exit (an exception included)
     // makes the main stream wait for it, so later work on the workspace is
     // ordered after the side-stream INTT
@@ -388,78 +381,56 @@ void hmult_relin_rescale_into(fhe_context *ctx, int count, int moduli_id,
           (void)hipStreamWaitEvent(ctx->stream, ctx->join_event, 0);
       }
     } join_guard{ctx, joined};
-    if (ctx->fuse_tensor && fhe::tensor_fused_supported(ctx->tables)) {
-      ctx->stage("ntt_pass_high(inputs)", [&] {
-        fhe::ntt_forward_first(ctx->tables, a, an, duo_l, limbs, moduli_id,
-                               ctx->tables.r2, ctx->stream, first_poly);
-        fhe::ntt_forward_first(ctx->tables, b, bn, duo_l, limbs, moduli_id,
-                               ctx->tables.r2, ctx->stream, first_poly);
+    ctx->stage("ntt(inputs)", [&] {
+      fhe::ntt_forward(ctx->tables, a, an, duo_l, limbs, moduli_id,
+                       ctx->tables.r2, ctx->stream, first_poly);
+      fhe::ntt_forward(ctx->tables, b, bn, duo_l, limbs, moduli_id,
+                       ctx->tables.r2, ctx->stream, first_poly);
+    });
+    ctx->stage("tensor", [&] {
+      fhe::launch_tensor(ctx->tables, an, bn, trio, count, limbs, moduli_id,
+                         ctx->stream);
+    });
+    if (overlap) {
+      // d0, d1 (lazy) on the side stream, forked once the trio is written
+      // (overlap_trio 1) or once d2's INTT is done (2, alongside the key
+      // switching of d2); d2 (exact, feeds ModUp) here
+      fhe::LazySpec lazy_part = d01, exact_part = d01;
+      lazy_part.part = 2;
+      exact_part.part = 1;
+      auto fork = [&] {
+        hip_check(hipEventRecord(ctx->fork_event, ctx->stream), "event");
+        hip_check(hipStreamWaitEvent(ctx->side, ctx->fork_event, 0),
+                  "event");
+        fhe::ntt_inverse(ctx->tables, trio, trio_c, trio_l, limbs,
+                         moduli_id, fhe::kInttExit, ctx->side, lazy_part);
+        hip_check(hipEventRecord(ctx->join_event, ctx->side), "event");
+        joined = false;
+      };
+      if (ctx->overlap_trio == 1)
+        fork();
+      ctx->stage("intt(trio)", [&] {
+        fhe::ntt_inverse(ctx->tables, trio, trio_c, trio_l, limbs,
+                         moduli_id, fhe::kInttExit, ctx->stream,
+                         exact_part);
       });
-      ctx->stage("tensor_r16", [&] {
-        fhe::launch_tensor_fused(ctx->tables, an, bn, trio, count, limbs,
-                                 moduli_id, ctx->lazy_key_switch,
-                                 ctx->stream);
-      });
-      ctx->stage("intt_pass_high(trio)", [&] {
-        fhe::ntt_inverse_second(ctx->tables, trio, trio, trio_l, limbs,
-                                moduli_id, fhe::kInttExit, ctx->stream, d01);
-      });
+      if (ctx->overlap_trio != 1)
+        fork();
     } else {
-      ctx->stage("ntt(inputs)", [&] {
-        fhe::ntt_forward(ctx->tables, a, an, duo_l, limbs, moduli_id,
-                         ctx->tables.r2, ctx->stream, first_poly);
-        fhe::ntt_forward(ctx->tables, b, bn, duo_l, limbs, moduli_id,
-                         ctx->tables.r2, ctx->stream, first_poly);
+      ctx->stage("intt(trio)", [&] {
+        fhe::ntt_inverse(ctx->tables, trio, trio_c, trio_l, limbs,
+                         moduli_id, fhe::kInttExit, ctx->stream, d01);
       });
-      ctx->stage("tensor", [&] {
-        fhe::launch_tensor(ctx->tables, an, bn, trio, count, limbs, moduli_id,
-                           ctx->stream);
-      });
-      if (overlap) {
-        // d0, d1 (lazy) on the side stream, forked once the trio is written
-        // (overlap_trio 1) or once d2's INTT is done (2, alongside the key
-        // switching of d2); d2 (exact, feeds ModUp) here
-        fhe::LazySpec lazy_part = d01, exact_part = d01;
-        lazy_part.part = 2;
-        exact_part.part = 1;
-        auto fork = [&] {
-          hip_check(hipEventRecord(ctx->fork_event, ctx->stream), "event");
-          hip_check(hipStreamWaitEvent(ctx->side, ctx->fork_event, 0),
-                    "event");
-          fhe::ntt_inverse(ctx->tables, trio, trio_c, trio_l, limbs,
-                           moduli_id, fhe::kInttExit, ctx->side, lazy_part);
-          hip_check(hipEventRecord(ctx->join_event, ctx->side), "event");
-          joined = false;
-        };
-        if (ctx->overlap_trio == 1)
-          fork();
-        ctx->stage("intt(trio)", [&] {
-          fhe::ntt_inverse(ctx->tables, trio, trio_c, trio_l, limbs,
-                           moduli_id, fhe::kInttExit, ctx->stream,
-                           exact_part);
-        });
-        if (ctx->overlap_trio != 1)
-          fork();
-      } else {
-        ctx->stage("intt(trio)", [&] {
-          fhe::ntt_inverse(ctx->tables, trio, trio_c, trio_l, limbs,
-                           moduli_id, fhe::kInttExit, ctx->stream, d01);
-        });
-      }
     }
-    const bool fused_trio = ctx->fuse_tensor &&
-                            fhe::tensor_fused_supported(ctx->tables);
-    const int64_t *coef = fused_trio ? trio : trio_c;
-    ctx->key_switch(count, moduli_id, key, key_moduli_id, coef + 2 * limbs * N,
-                    3 * limbs * N, ext, acc,
-                    fused_trio ? nullptr : trio + 2 * limbs * N,
-                    3 * limbs * N, false, digits);
+    ctx->key_switch(count, moduli_id, key, key_moduli_id,
+                    trio_c + 2 * limbs * N, 3 * limbs * N, ext, acc,
+                    trio + 2 * limbs * N, 3 * limbs * N, false, digits);
     if (overlap) {
       joined = true;
       hip_check(hipStreamWaitEvent(ctx->stream, ctx->join_event, 0), "event");
     }
     ctx->stage("moddown_relin_rescale", [&] {
-      fhe::launch_moddown_relin_rescale(ctx->tables, acc, coef, out, count,
+      fhe::launch_moddown_relin_rescale(ctx->tables, acc, trio_c, out, count,
                                         limbs, moduli_id, ctx->stream);
     });
 }
@@ -1127,7 +1098,7 @@ int fhe_rotate_batch(fhe_context *ctx, int count, int moduli_id,
     const int64_t acc_l = int64_t(count) * 2 * ext_limbs;
     int64_t *ws = ctx->scratch(size_t(duo_l + ext_l + acc_l) * N * 8);
     int64_t *sw = ws, *ext = sw + duo_l * N, *acc = ext + ext_l * N;
-    const bool hoist = fhe::ks_fused_supported(ctx->tables);
+    const bool hoist = ctx->ks_fused(moduli_id);
     // CKKSEngine::rotate_batch (src/ckks/engine_rotate.cpp:262-300): one
     // decomposition of c1, then the key-dependent part per key
     if (hoist)

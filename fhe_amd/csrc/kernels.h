@@ -57,7 +57,7 @@ void ntt_forward_second(const DeviceTables &t, const int64_t *src,
                         int moduli_id, hipStream_t stream,
                         LazySpec lazy = LazySpec());
 
-// Fused key-switching core for N = 2^16: for each tile of each extended limb
+// Fused key-switching core for N = 2^13 .. 2^16: for each tile of each extended limb
 // and ciphertext, the low-bit forward NTT pass of every partition's
 // extended polynomial, the key inner product over all partitions
 // (src/ckks/core_key_switch.cpp:318-336) and the low-bit inverse NTT pass of
@@ -71,9 +71,7 @@ void launch_ks_inner_product_fused(const DeviceTables &t, const int64_t *ext,
                                    int ext_limbs, int moduli_id, bool lazy,
                                    const int64_t *own, int64_t own_stride,
                                    const int *starts, const int *sizes,
-                                   bool lazy_accumulate, bool wide_accumulate,
-                                   bool prefetch, int occupancy,
-                                   hipStream_t stream);
+                                   bool lazy_accumulate, hipStream_t stream);
 
 // out = mont_mult(a, b) elementwise (src/montgomery/unit.cpp:5-10).
 void launch_mont_mult(const DeviceTables &t, const int64_t *a,
@@ -107,23 +105,10 @@ void launch_modup(const DeviceTables &t, const int64_t *x, int64_t x_stride,
                   int ext_shoup_offset, bool non_negative, bool lazy,
                   hipStream_t stream);
 
-// ModUp of every partition fused with the first forward NTT pass of every
-// extended limb (N = 2^16, partitions of at most 4 limbs): ext
-// [count][parts][ext][N] receives what launch_modup followed by
-// ntt_forward_first would write (the same representatives with lazy = false,
-// the same residues otherwise).  starts / sizes / is_signed: per partition.
 constexpr int kMaxFusedParts = 32;
-bool modup_ntt_fused_supported(const DeviceTables &t, int max_partition_size,
-                               int parts);
-void launch_modup_ntt_fused(const DeviceTables &t, const int64_t *x,
-                            int64_t x_stride, int64_t *ext, int count,
-                            int limbs, int moduli_id, const int *starts,
-                            const int *sizes, const bool *is_signed, int parts,
-                            const int64_t *constants, int constants_stride,
-                            bool lazy, hipStream_t stream);
 
-// ModUp staged through the Garner digits (N = 2^16, partitions of at most
-// 4 limbs): digits [count][parts][maxz][N] (maxz = partition size rounded up
+// ModUp staged through the Garner digits (N = 2^13 .. 2^16, partitions of at
+// most 8 limbs): digits [count][parts][maxz][N] (maxz = partition size rounded up
 // to a power of two) then ext [count][parts][ext][N] after the first forward
 // NTT pass, as launch_modup + ntt_forward_first would give (the same
 // representatives without lazy; with lazy, for non-negative partitions, the
@@ -138,16 +123,6 @@ void launch_staged_modup(const DeviceTables &t, const int64_t *x,
                          const int64_t *constants, int constants_stride,
                          int ext_shoup_offset, bool lazy, bool skip_own,
                          hipStream_t stream);
-
-// Second forward NTT pass of both input duos, tensor and first inverse NTT
-// pass of the trio in one kernel (N = 2^16).  a, b: [count][2][limbs][N]
-// after ntt_forward_first; trio: [count][3][limbs][N] for
-// ntt_inverse_second.  With lazy, a0 / b0 / z0 / z1 use the lazy arithmetic
-// (LazySpec{2, 1} for the first passes, {3, 2} for the last).
-bool tensor_fused_supported(const DeviceTables &t);
-void launch_tensor_fused(const DeviceTables &t, const int64_t *a,
-                         const int64_t *b, int64_t *trio, int count, int limbs,
-                         int moduli_id, bool lazy, hipStream_t stream);
 
 // Key inner product for one partition: acc[c][h] (+)= ext[c] * key_h
 // (src/ckks/core_key_switch.cpp:318-336).  Each key limb is read once for

@@ -54,14 +54,34 @@ extern "C" int fhe_hmult_relin_rescale_noalloc(fhe_context *ctx, int count,
     require(count > 0, "Multiply: empty batch");
     ctx->check_moduli(moduli_id, 3, "Multiply");
     ctx->check_key(moduli_id, key_moduli_id, "Multiply");
-    const int64_t ws = hmult_workspace_words(ctx, count, moduli_id);
-    const int64_t digits = ctx->ks_digits_words(count, moduli_id);
-    require(size_t(ws + digits) <= kScratchWords,
+    // the one-partition-at-a-time form needs the least workspace where it
+    // runs (N != 2^16); batches it holds are accepted, and run in the fused
+    // form in as many parts as the fused form's workspace asks for, or, when
+    // that holds not even one pair, one partition at a time
+    const bool fused = ctx->fused_key_switch;
+    struct Restore {
+      fhe_context *ctx;
+      bool fused;
+      ~Restore() { ctx->fused_key_switch = fused; }
+    } restore{ctx, fused};
+    auto words = [&](int n) {
+      return hmult_workspace_words(ctx, n, moduli_id) +
+             ctx->ks_digits_words(n, moduli_id);
+    };
+    ctx->fused_key_switch = false;
+    const int64_t least = words(count);
+    require(size_t(least) <= kScratchWords,
             "Multiply (no allocation): the batch needs " +
-                std::to_string((ws + digits) * 8) +
+                std::to_string(least * 8) +
                 " bytes of workspace, above the " +
                 std::to_string(kScratchBytes) +
                 "-byte scratch; split the batch");
+    ctx->fused_key_switch = fused;
+    int part = std::min<int64_t>(count, kScratchWords / words(1));
+    if (part == 0) {
+      ctx->fused_key_switch = false;
+      part = count;
+    }
     require(ctx->modup_cache.count({moduli_id, key_moduli_id}) != 0,
             "Multiply (no allocation): no ModUp constants for this key "
             "level (contexts prepare those of the maximum key-switching "
@@ -74,8 +94,14 @@ extern "C" int fhe_hmult_relin_rescale_noalloc(fhe_context *ctx, int count,
     }
     require(base != nullptr, "Multiply (no allocation): no scratch address "
                              "for this device");
-    hmult_relin_rescale_into(ctx, count, moduli_id, a, b, key, key_moduli_id,
-                             out, base, base + ws);
+    const int64_t in = int64_t(2) * ctx->params.limbs_at(moduli_id) * ctx->n();
+    const int64_t res = in - 2 * ctx->n();
+    for (int c = 0; c < count; c += part) {
+      const int n = std::min(part, count - c);
+      hmult_relin_rescale_into(
+          ctx, n, moduli_id, a + c * in, b + c * in, key, key_moduli_id,
+          out + c * res, base, base + hmult_workspace_words(ctx, n, moduli_id));
+    }
     ctx->check_launch("Multiply");
   });
 }

@@ -142,14 +142,14 @@ __global__ __launch_bounds__(kBlock) void ntt_pass_kernel(PassArgs a,
   }
 }
 
-// Register-resident 8-bit pass (r16_limb_pass, ntt_r16.h) on limb l of
+// Register-resident L-bit pass (r16_limb_pass, ntt_r16.h) on limb l of
 // polynomial `poly` of the batch.
-template <bool INV, bool COLS, int A>
+template <int L, bool INV, bool COLS, int A>
 __device__ __forceinline__ void r16_pass(const PassArgs &a,
                                          const DeviceTables &t, int64_t *lds,
                                          int64_t poly, int tile, int l) {
   const int64_t limb = (poly * a.limbs + l) << t.log_n;
-  r16_limb_pass<INV, COLS, A>(a.src + limb, a.dst + limb, a.moduli_id + l,
+  r16_limb_pass<L, INV, COLS, A>(a.src + limb, a.dst + limb, a.moduli_id + l,
                               tile, a.low_bit, a.pre, a.post, a.last != 0, t,
                               lds);
 }
@@ -165,11 +165,11 @@ struct PolySelect {
   int l0;      // first limb of the launch
 };
 
-template <bool INV, bool COLS, int A>
+template <int L, bool INV, bool COLS, int A>
 __global__ __launch_bounds__(kBlock) void ntt_radix16_kernel(
     PassArgs a, DeviceTables t, PolySelect sel, int tiles_per_limb,
     int swizzle) {
-  __shared__ int64_t lds[kR16Lds];
+  __shared__ int64_t lds[kR16Lds<L>];
   // block -> (limb l, tile, polynomial), polynomial fastest so blocks sharing
   // a prime's twiddles run together; with swizzle each of the 8 XCDs (blocks
   // are dealt round-robin to XCDs) gets one contiguous range of that order.
@@ -184,16 +184,16 @@ __global__ __launch_bounds__(kBlock) void ntt_radix16_kernel(
   const int l = sel.l0 + int(rest / tiles_per_limb);
   const int64_t poly =
       (j / sel.count) * sel.period + sel.offset + (j % sel.count);
-  r16_pass<INV, COLS, A>(a, t, lds, poly, tile, l);
+  r16_pass<L, INV, COLS, A>(a, t, lds, poly, tile, l);
 }
 
 // The same pass with the arithmetic chosen per block: polynomials whose index
 // modulo a.lazy_period is below a.lazy_count take the lazy arithmetic of
 // their prime's size class, the others the exact one (one launch for all).
-template <bool INV, bool COLS>
+template <int L, bool INV, bool COLS>
 __global__ __launch_bounds__(kBlock) void ntt_radix16_mixed_kernel(
     PassArgs a, DeviceTables t, int polys, int tiles_per_limb, int swizzle) {
-  __shared__ int64_t lds[kR16Lds];
+  __shared__ int64_t lds[kR16Lds<L>];
   int64_t w = blockIdx.x;
   if (swizzle) {
     const int64_t per = int64_t(gridDim.x) >> 3;
@@ -205,16 +205,23 @@ __global__ __launch_bounds__(kBlock) void ntt_radix16_mixed_kernel(
   const int l = int(rest / tiles_per_limb);
   const bool lazy = a.lazy_period > 0 && (poly % a.lazy_period) < a.lazy_count;
   if (!lazy)
-    r16_pass<INV, COLS, kExact>(a, t, lds, poly, tile, l);
+    r16_pass<L, INV, COLS, kExact>(a, t, lds, poly, tile, l);
   else if (t.q[a.moduli_id + l] < kLazySmallBound)
-    r16_pass<INV, COLS, kLazySmall>(a, t, lds, poly, tile, l);
+    r16_pass<L, INV, COLS, kLazySmall>(a, t, lds, poly, tile, l);
   else
-    r16_pass<INV, COLS, kLazyLarge>(a, t, lds, poly, tile, l);
+    r16_pass<L, INV, COLS, kLazyLarge>(a, t, lds, poly, tile, l);
 }
 
-// Split log_n into the bit ranges of at most two passes (each <= 12 bits).
-void split_bits(int log_n, int &first, int &second) {
-  if (log_n <= 12) {
+// Split log_n into the bit ranges of at most two passes (each <= 12 bits),
+// the first one's bits first: the high bits of a forward transform, the low
+// bits of an inverse one.  The radix-16 sizes use the same two ranges in
+// both directions (the fused kernels run the low forward pass and the low
+// inverse pass on one tile).
+void split_bits(int log_n, bool inverse, int &first, int &second) {
+  if (r16_supported(log_n)) {
+    first = inverse ? r16_low_bits(log_n) : r16_high_bits(log_n);
+    second = log_n - first;
+  } else if (log_n <= 12) {
     first = log_n;
     second = 0;
   } else {
@@ -223,128 +230,116 @@ void split_bits(int log_n, int &first, int &second) {
   }
 }
 
-void launch_pass(bool inverse, const PassArgs &a, const DeviceTables &t,
-                 hipStream_t stream) {
-  if (a.bits == 8 && t.log_n >= 12) {
-    const int64_t total_limbs = a.total_subs >> (t.log_n - 8);
-    const int polys = int(total_limbs / a.limbs);
-    const int tiles = int(int64_t(1) << (t.log_n - 12));
-    const bool cols = a.low_bit > 0;
-    auto launch = [&](int arith, PolySelect sel, int limbs_in_launch) {
-      const int64_t blocks = int64_t(sel.polys) * tiles * limbs_in_launch;
-      if (blocks == 0)
-        return;
-      const int swizzle = (blocks % 8 == 0) ? 1 : 0;
-#define FHE_R16(I, C, A)                                                       \
-  hipLaunchKernelGGL((ntt_radix16_kernel<I, C, A>), dim3(unsigned(blocks)),   \
-                     dim3(kBlock), 0, stream, a, t, sel, tiles, swizzle)
-#define FHE_R16_A(I, C)                                                        \
-  do {                                                                         \
-    if (arith == kExact)                                                       \
-      FHE_R16(I, C, kExact);                                                   \
-    else if (arith == kLazySmall)                                              \
-      FHE_R16(I, C, kLazySmall);                                               \
-    else                                                                       \
-      FHE_R16(I, C, kLazyLarge);                                               \
-  } while (0)
-      if (inverse) {
-        if (cols)
-          FHE_R16_A(true, true);
-        else
-          FHE_R16_A(true, false);
-      } else {
-        if (cols)
-          FHE_R16_A(false, true);
-        else
-          FHE_R16_A(false, false);
-      }
-#undef FHE_R16_A
-#undef FHE_R16
-    };
-    if (!t.split_variants) {
-      const int64_t blocks = total_limbs * tiles;
-      const int swizzle = (blocks % 8 == 0) ? 1 : 0;
-#define FHE_R16M(I, C)                                                         \
-  hipLaunchKernelGGL((ntt_radix16_mixed_kernel<I, C>), dim3(unsigned(blocks)),\
-                     dim3(kBlock), 0, stream, a, t, polys, tiles, swizzle)
-      if (inverse) {
-        if (cols)
-          FHE_R16M(true, true);
-        else
-          FHE_R16M(true, false);
-      } else {
-        if (cols)
-          FHE_R16M(false, true);
-        else
-          FHE_R16M(false, false);
-      }
-#undef FHE_R16M
+// One radix-16 pass of L bits (low index bits unless COLS).
+template <int L, bool INV, bool COLS>
+void launch_r16_pass(const PassArgs &a, const DeviceTables &t,
+                     hipStream_t stream) {
+  const int64_t total_limbs = a.total_subs >> (t.log_n - L);
+  const int polys = int(total_limbs / a.limbs);
+  const int tiles = int(int64_t(1) << (t.log_n - 12));
+  if (!t.split_variants) {
+    const int64_t blocks = total_limbs * tiles;
+    hipLaunchKernelGGL((ntt_radix16_mixed_kernel<L, INV, COLS>),
+                       dim3(unsigned(blocks)), dim3(kBlock), 0, stream, a, t,
+                       polys, tiles, blocks % 8 == 0 ? 1 : 0);
+    return;
+  }
+  auto launch = [&](int arith, PolySelect sel, int limbs_in_launch) {
+    const int64_t blocks = int64_t(sel.polys) * tiles * limbs_in_launch;
+    if (blocks == 0)
       return;
+    const dim3 grid{unsigned(blocks), 1, 1};
+    const int swizzle = blocks % 8 == 0 ? 1 : 0;
+    if (arith == kExact)
+      hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, kExact>), grid,
+                         dim3(kBlock), 0, stream, a, t, sel, tiles, swizzle);
+    else if (arith == kLazySmall)
+      hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, kLazySmall>), grid,
+                         dim3(kBlock), 0, stream, a, t, sel, tiles, swizzle);
+    else
+      hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, kLazyLarge>), grid,
+                         dim3(kBlock), 0, stream, a, t, sel, tiles, swizzle);
+  };
+  const int period = a.lazy_period > 0 ? a.lazy_period : 1;
+  const int lazy_count = a.lazy_period > 0 ? a.lazy_count : 0;
+  // polynomials in whole periods (every caller passes whole periods)
+  if (polys % period != 0)
+    throw std::invalid_argument(
+        "NTT: the polynomial count is not a whole number of lazy periods");
+  const int periods = polys / period;
+  // exact polynomials: all limbs in one launch
+  if (lazy_count < period && a.lazy_part != 2)
+    launch(kExact,
+           PolySelect{periods * (period - lazy_count), period,
+                      period - lazy_count, lazy_count, 0},
+           a.limbs);
+  // lazy polynomials: one launch per run of limbs of one prime class
+  if (lazy_count > 0 && a.lazy_part != 1) {
+    int l = 0;
+    while (l < a.limbs) {
+      const bool small = t_host_q_small(t, a.moduli_id + l);
+      int e = l + 1;
+      while (e < a.limbs && t_host_q_small(t, a.moduli_id + e) == small)
+        e++;
+      launch(small ? kLazySmall : kLazyLarge,
+             PolySelect{periods * lazy_count, period, lazy_count, 0, l},
+             e - l);
+      l = e;
     }
-    const int period = a.lazy_period > 0 ? a.lazy_period : 1;
-    const int lazy_count = a.lazy_period > 0 ? a.lazy_count : 0;
-    // polynomials in whole periods (every caller passes whole periods)
-    if (polys % period != 0)
-      throw std::invalid_argument(
-          "NTT: the polynomial count is not a whole number of lazy periods");
-    const int periods = polys / period;
-    // exact polynomials: all limbs in one launch
-    if (lazy_count < period && a.lazy_part != 2)
-      launch(kExact,
-             PolySelect{periods * (period - lazy_count), period,
-                        period - lazy_count, lazy_count, 0},
-             a.limbs);
-    // lazy polynomials: one launch per run of limbs of one prime class
-    if (lazy_count > 0 && a.lazy_part != 1) {
-      int l = 0;
-      while (l < a.limbs) {
-        const bool small = t_host_q_small(t, a.moduli_id + l);
-        int e = l + 1;
-        while (e < a.limbs && t_host_q_small(t, a.moduli_id + e) == small)
-          e++;
-        launch(small ? kLazySmall : kLazyLarge,
-               PolySelect{periods * lazy_count, period, lazy_count, 0, l},
-               e - l);
-        l = e;
-      }
-    }
+  }
+}
+
+template <bool INV>
+void launch_pass(const PassArgs &a, const DeviceTables &t,
+                 hipStream_t stream) {
+  const bool cols = a.low_bit > 0;
+  if (t.log_n >= 13 && a.bits == 8) {
+    if (cols)
+      launch_r16_pass<8, INV, true>(a, t, stream);
+    else
+      launch_r16_pass<8, INV, false>(a, t, stream);
+    return;
+  }
+  if (t.log_n >= 13 && a.bits == 7) {
+    if (cols)
+      launch_r16_pass<7, INV, true>(a, t, stream);
+    else
+      launch_r16_pass<7, INV, false>(a, t, stream);
+    return;
+  }
+  if (t.log_n >= 13 && a.bits == 6 && cols) {
+    launch_r16_pass<6, INV, true>(a, t, stream);
     return;
   }
   const int C = kTile >> a.bits;
   const unsigned blocks = unsigned((a.total_subs + C - 1) / C);
-  if (inverse)
-    hipLaunchKernelGGL(ntt_pass_kernel<true>, dim3(blocks), dim3(kBlock), 0,
-                       stream, a, t);
-  else
-    hipLaunchKernelGGL(ntt_pass_kernel<false>, dim3(blocks), dim3(kBlock), 0,
-                       stream, a, t);
+  hipLaunchKernelGGL(ntt_pass_kernel<INV>, dim3(blocks), dim3(kBlock), 0,
+                     stream, a, t);
 }
 
 } // namespace
 
 bool ntt_parts_supported(const DeviceTables &t) {
-  int l1, l2;
-  split_bits(t.log_n, l1, l2);
-  return t.split_variants && l1 == 8 && l2 == 8;
+  return t.split_variants && r16_supported(t.log_n);
 }
 
 void ntt_forward(const DeviceTables &t, const int64_t *src, int64_t *dst,
                  int64_t total_limbs, int limbs, int moduli_id,
                  const int64_t *pre, hipStream_t stream, LazySpec lazy) {
   int l1, l2;
-  split_bits(t.log_n, l1, l2);
+  split_bits(t.log_n, false, l1, l2);
   // first pass: the high bits (stages 0 .. l1-1)
   PassArgs a{src,     dst,      total_limbs << (t.log_n - l1),
              limbs,   moduli_id, t.log_n - l1,
              l1,      pre,       kInttRaw,
              l2 == 0, lazy.period, lazy.count, lazy.part};
-  launch_pass(false, a, t, stream);
+  launch_pass<false>(a, t, stream);
   if (l2 > 0) {
     PassArgs b2{dst,   dst,      total_limbs << (t.log_n - l2),
                 limbs, moduli_id, 0,
                 l2,    nullptr,   kInttRaw,
                 1,     lazy.period, lazy.count, lazy.part};
-    launch_pass(false, b2, t, stream);
+    launch_pass<false>(b2, t, stream);
   }
 }
 
@@ -352,19 +347,19 @@ void ntt_inverse(const DeviceTables &t, const int64_t *src, int64_t *dst,
                  int64_t total_limbs, int limbs, int moduli_id, int post,
                  hipStream_t stream, LazySpec lazy) {
   int l1, l2;
-  split_bits(t.log_n, l1, l2);
+  split_bits(t.log_n, true, l1, l2);
   // first pass: the low bits (stages with span 1 .. 2^(l1-1))
   PassArgs a{src,     dst,      total_limbs << (t.log_n - l1),
              limbs,   moduli_id, 0,
              l1,      nullptr,   l2 > 0 ? int(kInttRaw) : post,
              l2 == 0, lazy.period, lazy.count, lazy.part};
-  launch_pass(true, a, t, stream);
+  launch_pass<true>(a, t, stream);
   if (l2 > 0) {
     PassArgs b2{dst,   dst,      total_limbs << (t.log_n - l2),
                 limbs, moduli_id, l1,
                 l2,    nullptr,   post,
                 1,     lazy.period, lazy.count, lazy.part};
-    launch_pass(true, b2, t, stream);
+    launch_pass<true>(b2, t, stream);
   }
 }
 
@@ -373,19 +368,19 @@ void ntt_forward_first(const DeviceTables &t, const int64_t *src, int64_t *dst,
                        const int64_t *pre, hipStream_t stream,
                        LazySpec lazy) {
   int l1, l2;
-  split_bits(t.log_n, l1, l2);
+  split_bits(t.log_n, false, l1, l2);
   PassArgs a{src,     dst,      total_limbs << (t.log_n - l1),
              limbs,   moduli_id, t.log_n - l1,
              l1,      pre,       kInttRaw,
              l2 == 0, lazy.period, lazy.count, lazy.part};
-  launch_pass(false, a, t, stream);
+  launch_pass<false>(a, t, stream);
 }
 
 void ntt_forward_second(const DeviceTables &t, const int64_t *src,
                         int64_t *dst, int64_t total_limbs, int limbs,
                         int moduli_id, hipStream_t stream, LazySpec lazy) {
   int l1, l2;
-  split_bits(t.log_n, l1, l2);
+  split_bits(t.log_n, false, l1, l2);
   if (l2 == 0) {
     // single-pass sizes: the first pass was the whole transform
     if (src != dst)
@@ -397,7 +392,7 @@ void ntt_forward_second(const DeviceTables &t, const int64_t *src,
               limbs, moduli_id, 0,
               l2,    nullptr,   kInttRaw,
               1,     lazy.period, lazy.count, lazy.part};
-  launch_pass(false, b2, t, stream);
+  launch_pass<false>(b2, t, stream);
 }
 
 void ntt_inverse_second(const DeviceTables &t, const int64_t *src,
@@ -405,12 +400,12 @@ void ntt_inverse_second(const DeviceTables &t, const int64_t *src,
                         int moduli_id, int post, hipStream_t stream,
                         LazySpec lazy) {
   int l1, l2;
-  split_bits(t.log_n, l1, l2);
+  split_bits(t.log_n, true, l1, l2);
   PassArgs a{src,   dst,      total_limbs << (t.log_n - l2),
              limbs, moduli_id, l1,
              l2,    nullptr,   post,
              1,     lazy.period, lazy.count, lazy.part};
-  launch_pass(true, a, t, stream);
+  launch_pass<true>(a, t, stream);
 }
 
 } // namespace fhe

@@ -1,14 +1,16 @@
-// Register-resident radix-16 rounds of a 256-point (8-bit) NTT pass, shared
-// by the standalone NTT kernel and the fused key-switching kernels.
+// Register-resident radix-16 rounds of an L-bit NTT pass (L = 6, 7 or 8),
+// shared by the standalone NTT kernel and the fused key-switching kernels.
 //
-// A tile holds 16 sub-transforms of 256 points; sub-transform c is owned by
-// the 16 threads with row r = 0..15, each holding 16 points v[m].  Two
-// ownerships are used:
-//   ROWS  j = r + 16 m   (bits 7..4 of j vary inside a thread)
+// A tile holds 4096 points: 2^(12 - L) sub-transforms of 2^L points;
+// sub-transform c is owned by the T = 2^(L - 4) threads with row r = 0..T-1,
+// each holding 16 points v[m].  Two ownerships are used:
+//   ROWS  j = r + T m    (bits L-1..L-4 of j vary inside a thread)
 //   COLS  j = 16 r + m   (bits 3..0 vary inside a thread)
-// The forward pass runs its local bits 7..4 in ROWS and 3..0 in COLS; the
-// inverse pass runs 0..3 in COLS and 4..7 in ROWS.  Twiddle addressing is
-// derived in the ntt.hip header comment.
+// The forward pass runs its local bits L-1..L-4 in ROWS and the others in
+// COLS; the inverse pass runs 0..L-5 in COLS and the last four in ROWS.
+// N = 2^13 splits into passes of 7 low and 6 high bits, 2^14 into 7 and 7,
+// 2^15 into 8 and 7, 2^16 into 8 and 8 (r16_low_bits).  Twiddle addressing
+// is derived in the ntt.hip header comment.
 //
 // Three arithmetics share the loop structure (template parameter A):
 //   kExact      the reference's radix-2 formulas with Montgomery twiddles
@@ -31,6 +33,16 @@
 #include "device.h"
 
 namespace fhe {
+
+// Low (contiguous) and high (strided) index bits of the two radix-16 passes
+// of N = 2^log_n, and the sizes they serve.
+inline bool r16_supported(int log_n) { return log_n >= 13 && log_n <= 16; }
+__host__ __device__ constexpr int r16_low_bits(int log_n) {
+  return (log_n + 1) / 2;
+}
+__host__ __device__ constexpr int r16_high_bits(int log_n) {
+  return log_n - r16_low_bits(log_n);
+}
 
 enum NttArith : int { kExact = 0, kLazySmall = 1, kLazyLarge = 2 };
 
@@ -93,9 +105,9 @@ __device__ __forceinline__ int64_t load_product(int64_t v, int64_t c,
   return y;
 }
 
-// Everything a thread needs to address twiddles in one 8-bit pass: the pass
-// covers index bits [b, b+8) of a limb of 2^log_n points; hi is the
-// sub-transform's index bits above b+8 and r the thread's row.
+// Everything a thread needs to address twiddles in one L-bit pass: the pass
+// covers index bits [b, b+L) of a limb of 2^log_n points; hi is the
+// sub-transform's index bits above b+L and r the thread's row.
 struct R16Pass {
   const int64_t *tw;   // Montgomery twiddles of this prime (kExact)
   const uint64_t *ts;  // {w, w'} pairs of this prime (lazy forms)
@@ -148,32 +160,32 @@ __device__ __forceinline__ void inv_bfly(int64_t &x, int64_t &y,
   y = int64_t(shoup_mult_neg(uint64_t(d), w, wq, s.nq));
 }
 
-// forward local bits 7..4, ROWS ownership
-template <int A = kExact>
+// forward local bits L-1..L-4, ROWS ownership
+template <int L, int A = kExact>
 __device__ __forceinline__ void r16_forward_high(int64_t (&v)[16],
                                                  const R16Pass &s) {
 #pragma unroll
-  for (int u = 7; u >= 4; u--) {
-    const int x = u - 4;
+  for (int x = 3; x >= 0; x--) {
+    const int u = x + L - 4;
     const int stage = s.log_n - 1 - s.b - u;
-    const int64_t tb = (int64_t(1) << stage) - 1 + (s.hi << (7 - u));
+    const int64_t tb = (int64_t(1) << stage) - 1 + (s.hi << (L - 1 - u));
 #pragma unroll
     for (int m = 0; m < 16; m++) {
       if (m & (1 << x))
         continue;
-      fwd_bfly<A>(v[m], v[m + (1 << x)], s, tb + (m >> (u - 3)));
+      fwd_bfly<A>(v[m], v[m + (1 << x)], s, tb + (m >> (x + 1)));
     }
   }
 }
 
-// forward local bits 3..0, COLS ownership
-template <int A = kExact>
+// forward local bits L-5..0, COLS ownership
+template <int L, int A = kExact>
 __device__ __forceinline__ void r16_forward_low(int64_t (&v)[16],
                                                 const R16Pass &s) {
 #pragma unroll
-  for (int u = 3; u >= 0; u--) {
+  for (int u = L - 5; u >= 0; u--) {
     const int stage = s.log_n - 1 - s.b - u;
-    const int64_t tb = (int64_t(1) << stage) - 1 + (s.hi << (7 - u)) +
+    const int64_t tb = (int64_t(1) << stage) - 1 + (s.hi << (L - 1 - u)) +
                        (int64_t(s.r) << (3 - u));
 #pragma unroll
     for (int m = 0; m < 16; m++) {
@@ -184,13 +196,13 @@ __device__ __forceinline__ void r16_forward_low(int64_t (&v)[16],
   }
 }
 
-// inverse local bits 0..3, COLS ownership
-template <int A = kExact>
+// inverse local bits 0..L-5, COLS ownership
+template <int L, int A = kExact>
 __device__ __forceinline__ void r16_inverse_low(int64_t (&v)[16],
                                                 const R16Pass &s) {
 #pragma unroll
-  for (int u = 0; u <= 3; u++) {
-    const int64_t tb = s.n - (s.n >> (s.b + u)) + (s.hi << (7 - u)) +
+  for (int u = 0; u <= L - 5; u++) {
+    const int64_t tb = s.n - (s.n >> (s.b + u)) + (s.hi << (L - 1 - u)) +
                        (int64_t(s.r) << (3 - u));
 #pragma unroll
     for (int m = 0; m < 16; m++) {
@@ -201,19 +213,19 @@ __device__ __forceinline__ void r16_inverse_low(int64_t (&v)[16],
   }
 }
 
-// inverse local bits 4..7, ROWS ownership
-template <int A = kExact>
+// inverse local bits L-4..L-1, ROWS ownership
+template <int L, int A = kExact>
 __device__ __forceinline__ void r16_inverse_high(int64_t (&v)[16],
                                                  const R16Pass &s) {
 #pragma unroll
-  for (int u = 4; u <= 7; u++) {
-    const int x = u - 4;
-    const int64_t tb = s.n - (s.n >> (s.b + u)) + (s.hi << (7 - u));
+  for (int x = 0; x <= 3; x++) {
+    const int u = x + L - 4;
+    const int64_t tb = s.n - (s.n >> (s.b + u)) + (s.hi << (L - 1 - u));
 #pragma unroll
     for (int m = 0; m < 16; m++) {
       if (m & (1 << x))
         continue;
-      inv_bfly<A>(v[m], v[m + (1 << x)], s, tb + (m >> (u - 3)), s.b + u);
+      inv_bfly<A>(v[m], v[m + (1 << x)], s, tb + (m >> (x + 1)), s.b + u);
     }
   }
 }
@@ -230,13 +242,20 @@ __device__ __forceinline__ void r16_forward_settle(int64_t (&v)[16],
     v[m] = guard_u(v[m], s.q2);
 }
 
-// LDS exchange buffer: 16 sub-transforms x 256 points, padded so that both
-// ownerships and the 16 sub-transforms of a row map to distinct banks.
-constexpr int kR16Row = 273;
-constexpr int kR16Lds = 16 * kR16Row;
+// LDS exchange buffer: a tile's sub-transforms in rows of 2^L points, padded
+// so that both ownerships and the sub-transforms of a row spread over the
+// banks.
+template <int L> constexpr int kR16Row = (1 << L) + (1 << (L - 4)) + 1;
+template <int L> constexpr int kR16Lds = (4096 >> L) * kR16Row<L>;
 
-__device__ __forceinline__ int r16_lds(int c, int j) {
-  return c * kR16Row + j + (j >> 4);
+template <int L> __device__ __forceinline__ int r16_lds(int c, int j) {
+  return c * kR16Row<L> + j + (j >> 4);
+}
+
+// Index within its sub-transform of the thread's point m.
+template <int L, bool COLS_OWNED>
+__device__ __forceinline__ int r16_point(int r, int m) {
+  return COLS_OWNED ? 16 * r + m : r + (1 << (L - 4)) * m;
 }
 
 // Orders one wavefront's LDS accesses: a wave's LDS instructions execute in
@@ -247,70 +266,69 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Re-own the thread's 16 points: ROWS -> COLS (to_cols) or COLS -> ROWS.
+// Re-own the thread's 16 points: ROWS -> COLS (TO_COLS) or COLS -> ROWS.
 // Starts with a barrier so the previous use of the buffer has finished.
-// WAVE: the 16 threads sharing c are 16 consecutive threads (c = tid >> 4),
-// hence in one wavefront, and a wavefront barrier replaces the block's.
-template <bool WAVE = false>
+// WAVE: the threads sharing c are consecutive (c = tid / T, T <= 16), hence
+// in one wavefront, and a wavefront barrier replaces the block's.
+template <int L, bool TO_COLS, bool WAVE = false>
 __device__ __forceinline__ void r16_exchange(int64_t (&v)[16], int64_t *lds,
-                                             int c, int r, bool to_cols) {
+                                             int c, int r) {
   if (WAVE)
     wave_lds_sync();
   else
     __syncthreads();
 #pragma unroll
   for (int m = 0; m < 16; m++)
-    lds[r16_lds(c, to_cols ? r + 16 * m : 16 * r + m)] = v[m];
+    lds[r16_lds<L>(c, r16_point<L, !TO_COLS>(r, m))] = v[m];
   if (WAVE)
     wave_lds_sync();
   else
     __syncthreads();
 #pragma unroll
   for (int m = 0; m < 16; m++)
-    v[m] = lds[r16_lds(c, to_cols ? 16 * r + m : r + 16 * m)];
+    v[m] = lds[r16_lds<L>(c, r16_point<L, TO_COLS>(r, m))];
 }
 
 // r16_exchange through a buffer of 32-bit words, half the LDS of the 64-bit
 // exchange (so that twice as many blocks fit on a CU): the low words go
 // through first, then the high words, each between two barriers.
-constexpr int kR16LdsWords = kR16Lds;
-
+template <int L, bool TO_COLS>
 __device__ __forceinline__ void r16_exchange_words(int64_t (&v)[16],
                                                    uint32_t *lds, int c,
-                                                   int r, bool to_cols) {
+                                                   int r) {
   uint32_t lo[16];
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < 16; m++)
-    lds[r16_lds(c, to_cols ? r + 16 * m : 16 * r + m)] = uint32_t(v[m]);
+    lds[r16_lds<L>(c, r16_point<L, !TO_COLS>(r, m))] = uint32_t(v[m]);
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < 16; m++)
-    lo[m] = lds[r16_lds(c, to_cols ? 16 * r + m : r + 16 * m)];
+    lo[m] = lds[r16_lds<L>(c, r16_point<L, TO_COLS>(r, m))];
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < 16; m++)
-    lds[r16_lds(c, to_cols ? r + 16 * m : 16 * r + m)] =
+    lds[r16_lds<L>(c, r16_point<L, !TO_COLS>(r, m))] =
         uint32_t(uint64_t(v[m]) >> 32);
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < 16; m++)
     v[m] = int64_t(
-        (uint64_t(lds[r16_lds(c, to_cols ? 16 * r + m : r + 16 * m)]) << 32) |
+        (uint64_t(lds[r16_lds<L>(c, r16_point<L, TO_COLS>(r, m))]) << 32) |
         lo[m]);
 }
 
-// One register-resident 8-bit pass over one 4096-point tile of one limb:
-// the 16 sub-transforms of the tile are owned by 16 threads each (16 points
-// per thread) and the eight radix-2 stages run as two radix-16 rounds with
-// one LDS exchange between them.  A second exchange is added where the
+// One register-resident L-bit pass over one 4096-point tile of one limb:
+// the sub-transforms of the tile are owned by T threads each (16 points per
+// thread) and the L radix-2 stages run as two rounds (four stages and L - 4)
+// with one LDS exchange between them.  A second exchange is added where the
 // global side of the pass is contiguous and the register ownership is not,
 // so that every global access is coalesced.  src / dst point at the limb
-// (prime p); the pass covers index bits [b, b + 8); COLS is b > 0.  pre
+// (prime p); the pass covers index bits [b, b + L); COLS is b > 0.  pre
 // (forward, per prime) multiplies every loaded value first; post (inverse)
 // is the InttPost epilogue; last = the pass completes a forward transform.
 // OPAQUE: the pass runs inside a persistent loop (opaque_tid).
-template <bool INV, bool COLS, int A, bool OPAQUE = false>
+template <int L, bool INV, bool COLS, int A, bool OPAQUE = false>
 __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
                                               int64_t *dst_limb, int p,
                                               int tile, int b,
@@ -320,12 +338,13 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
   const int log_n = t.log_n;
   const int64_t n = int64_t(1) << log_n;
   const int tid = OPAQUE ? opaque_tid() : int(threadIdx.x);
-  const int c = COLS ? (tid & 15) : (tid >> 4);
-  const int r = COLS ? (tid >> 4) : (tid & 15);
-  const int64_t sp = int64_t(tile) * 16 + c;
+  constexpr int T = 1 << (L - 4), C = 4096 >> L;
+  const int c = COLS ? (tid & (C - 1)) : (tid >> (L - 4));
+  const int r = COLS ? (tid >> (12 - L)) : (tid & (T - 1));
+  const int64_t sp = int64_t(tile) * C + c;
   const int64_t lo = sp & ((int64_t(1) << b) - 1);
   const int64_t hi = sp >> b;
-  const int64_t base = (hi << (b + 8)) + lo;
+  const int64_t base = (hi << (b + L)) + lo;
   const int64_t *src = src_limb + base;
   int64_t *dst = dst_limb + base;
 
@@ -346,10 +365,10 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
   int64_t v[16];
   // load in the ownership of the first round; the contiguous inverse pass
   // loads coalesced ROWS and re-owns through LDS
-  const bool cols_load = INV && COLS;
+  constexpr bool cols_load = INV && COLS;
 #pragma unroll
   for (int m = 0; m < 16; m++)
-    v[m] = src[int64_t(cols_load ? 16 * r + m : r + 16 * m) << b];
+    v[m] = src[int64_t(r16_point<L, cols_load>(r, m)) << b];
   if (pre) {
     const int64_t cst = pre[p];
 #pragma unroll
@@ -357,20 +376,20 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
       v[m] = load_product<A>(v[m], cst, s.q, s.k);
   }
   if (INV && !COLS)
-    r16_exchange<!COLS>(v, lds, c, r, true);
+    r16_exchange<L, true, !COLS>(v, lds, c, r);
 
   if (!INV) {
-    r16_forward_high<A>(v, s);
-    r16_exchange<!COLS>(v, lds, c, r, true);
-    r16_forward_low<A>(v, s);
+    r16_forward_high<L, A>(v, s);
+    r16_exchange<L, true, !COLS>(v, lds, c, r);
+    r16_forward_low<L, A>(v, s);
     if (last)
       r16_forward_settle<A>(v, s);
     if (!COLS)
-      r16_exchange<!COLS>(v, lds, c, r, false); // coalesced contiguous store
+      r16_exchange<L, false, !COLS>(v, lds, c, r); // coalesced contiguous store
   } else {
-    r16_inverse_low<A>(v, s);
-    r16_exchange<!COLS>(v, lds, c, r, false);
-    r16_inverse_high<A>(v, s);
+    r16_inverse_low<L, A>(v, s);
+    r16_exchange<L, false, !COLS>(v, lds, c, r);
+    r16_inverse_high<L, A>(v, s);
     if (post != kInttRaw) {
       const int64_t ninv = t.ninv[p];
       if (A == kExact) {
@@ -396,10 +415,10 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
     }
   }
   // store: ROWS ownership except the strided forward pass (COLS)
-  const bool cols_store = !INV && COLS;
+  constexpr bool cols_store = !INV && COLS;
 #pragma unroll
   for (int m = 0; m < 16; m++)
-    dst[int64_t(cols_store ? 16 * r + m : r + 16 * m) << b] = v[m];
+    dst[int64_t(r16_point<L, cols_store>(r, m)) << b] = v[m];
 }
 
 } // namespace fhe

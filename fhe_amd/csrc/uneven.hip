@@ -157,8 +157,8 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     int64_t key;
     uint32_t unit;
   };
-  auto emit = [&](int stage, std::vector<Keyed> (&by_variant)[4]) {
-    for (int v = 0; v < 4; v++) {
+  auto emit = [&](int stage, std::vector<Keyed> (&by_variant)[3]) {
+    for (int v = 0; v < 3; v++) {
       auto &list = by_variant[v];
       if (list.empty())
         continue;
@@ -177,7 +177,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
   if (relin) {
     // the trio's d2 exact (it feeds ModUp), d0 / d1 lazy
     for (int stage : {int(kStTrioIntt1), int(kStTrioIntt2)}) {
-      std::vector<Keyed> lists[4];
+      std::vector<Keyed> lists[3];
       for (int c = 0; c < count; c++) {
         const UnevenCt &u = plan->host[c];
         for (int poly = 0; poly < 3; poly++)
@@ -193,7 +193,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     }
   }
   {
-    std::vector<Keyed> lists[4];
+    std::vector<Keyed> lists[3];
     for (int c = 0; c < count; c++)
       for (int p = 0; p < plan->host[c].parts; p++)
         for (int ch = 0; ch < chunks; ch++)
@@ -201,7 +201,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     emit(kStDigits, lists);
   }
   {
-    std::vector<Keyed> lists[4];
+    std::vector<Keyed> lists[3];
     for (int c = 0; c < count; c++) {
       const UnevenCt &u = plan->host[c];
       for (int p = 0; p < u.parts; p++)
@@ -221,16 +221,12 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     emit(kStExtend, lists);
   }
   {
-    std::vector<Keyed> lists[4];
+    std::vector<Keyed> lists[3];
     for (int c = 0; c < count; c++) {
       const UnevenCt &u = plan->host[c];
       for (int i = 0; i < u.ext; i++) {
         const int prime = u.moduli_id + i;
-        int v = lazy_variant(P, prime);
-        // small primes of ciphertexts with several partitions: 96-bit sums
-        if (v == fhe::kLazySmall && ctx->ks_wide_accumulate && u.parts > 1 &&
-            u.parts <= fhe::kMaxWideParts)
-          v = 3;
+        const int v = lazy_variant(P, prime);
         for (int t = 0; t < tiles; t++)
           lists[v].push_back({tile_key(prime, t), fhe::unit_pack(c, 0, i, t)});
       }
@@ -238,7 +234,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     emit(kStKs, lists);
   }
   {
-    std::vector<Keyed> lists[4];
+    std::vector<Keyed> lists[3];
     for (int c = 0; c < count; c++) {
       const UnevenCt &u = plan->host[c];
       for (int h = 0; h < 2; h++)
@@ -252,7 +248,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     emit(kStAccIntt2, lists);
   }
   {
-    std::vector<Keyed> lists[4];
+    std::vector<Keyed> lists[3];
     for (int c = 0; c < count; c++)
       for (int h = 0; h < 2; h++)
         for (int ch = 0; ch < chunks; ch++)
@@ -260,7 +256,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     emit(kStModDown, lists);
   }
   if (!relin) {
-    std::vector<Keyed> lists[4];
+    std::vector<Keyed> lists[3];
     const int aut_chunks = int(P.n / (4 * fhe::kBlock));
     for (int c = 0; c < count; c++)
       for (int poly = 0; poly < 2; poly++)
@@ -447,7 +443,7 @@ void uneven_tune(fhe_context *ctx, UnevenPlan *plan, const int64_t *const *src,
 void check_uneven(fhe_context *ctx, int count, const int *moduli_ids,
                   int key_moduli_id, const char *op) {
   require(count > 0, std::string(op) + ": empty batch");
-  require(fhe::ks_fused_supported(ctx->tables),
+  require(ctx->params.log_n == 16,
           std::string(op) + ": uneven-level batches need N = 2^16");
   for (int c = 0; c < count; c++) {
     ctx->check_moduli(moduli_ids[c], 1, op);

@@ -51,14 +51,14 @@ struct UnevenNttArgs {
 template <bool INV, bool COLS, int A>
 __global__ __launch_bounds__(kBlock) void uneven_ntt_kernel(UnevenNttArgs a,
                                                             DeviceTables t) {
-  __shared__ int64_t lds[kR16Lds];
+  __shared__ int64_t lds[kR16Lds<8>];
   for (UnitWalk u(a.list); u.w < u.end; u.w += u.step) {
     const uint32_t unit = a.list.units[u.w];
     const int c = unit_ct(unit), l = unit_limb(unit);
     const UnevenCt &ct = a.cts[c];
     const int stride = a.ext_stride ? ct.ext : ct.limbs;
     const int64_t off = (int64_t(unit_a(unit)) * stride + l) << t.log_n;
-    r16_limb_pass<INV, COLS, A, true>(a.src.p[c] + off,
+    r16_limb_pass<8, INV, COLS, A, true>(a.src.p[c] + off,
                                 const_cast<int64_t *>(a.dst.p[c]) + off,
                                 ct.moduli_id + l, unit_tile(unit), a.b, a.pre,
                                 a.post, a.last != 0, t, lds);
@@ -116,7 +116,7 @@ struct UnevenExtArgs {
 template <int A, int MAXZ, bool SIGNED>
 __global__ __launch_bounds__(kBlock) void uneven_extend_kernel(
     UnevenExtArgs a, DeviceTables t) {
-  __shared__ uint32_t lds[kR16LdsWords];
+  __shared__ uint32_t lds[kR16Lds<8>];
   for (UnitWalk u(a.list); u.w < u.end; u.w += u.step) {
     const uint32_t unit = a.list.units[u.w];
     const int c = unit_ct(unit), part = unit_a(unit);
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(kBlock) void uneven_extend_kernel(
     it.ext_limbs = ct.ext;
     it.moduli_id = ct.moduli_id;
     it.ext_shoup_offset = ct.ext_shoup_offset;
-    ext_item_tile<A, MAXZ, SIGNED, true>(it, t, lds, unit_tile(unit),
+    ext_item_tile<16, A, MAXZ, SIGNED, true>(it, t, lds, unit_tile(unit),
                                    unit_limb(unit));
   }
 }
@@ -178,14 +178,16 @@ struct UnevenKsAddr {
   }
 };
 
-template <int A, bool WIDE>
-__global__ __launch_bounds__(kBlock) void uneven_ks_kernel(UnevenKsArgs a,
+// two waves per SIMD: without the bound the allocation of the large-prime
+// form ends just above 256 registers, at one wave
+template <int A>
+__global__ __launch_bounds__(kBlock, 2) void uneven_ks_kernel(UnevenKsArgs a,
                                                            DeviceTables t) {
-  __shared__ int64_t lds[kR16Lds];
+  __shared__ int64_t lds[kR16Lds<8>];
   for (UnitWalk u(a.list); u.w < u.end; u.w += u.step) {
     const uint32_t unit = a.list.units[u.w];
     const UnevenKsAddr ad(a, unit_ct(unit), t.log_n);
-    ks_item_tile<A, false, WIDE, UnevenKsAddr, true>(
+    ks_item_tile<16, A, UnevenKsAddr, true>(
         ad, t, lds, unit_tile(unit), unit_limb(unit));
   }
 }
@@ -377,19 +379,15 @@ void launch_uneven_ks(const DeviceTables &t, const UnevenCt *cts,
                  own,       acc,           key,
                  key_chain, key_moduli_id, lazy_accumulate ? 1 : 0};
   const dim3 grid(grid_of(list.count, cap));
-  // variant 3: small primes with the 96-bit sums
   if (variant == kExact)
-    hipLaunchKernelGGL((uneven_ks_kernel<kExact, false>), grid, dim3(kBlock),
-                       0, stream, a, t);
+    hipLaunchKernelGGL(uneven_ks_kernel<kExact>, grid, dim3(kBlock), 0,
+                       stream, a, t);
   else if (variant == kLazySmall)
-    hipLaunchKernelGGL((uneven_ks_kernel<kLazySmall, false>), grid,
-                       dim3(kBlock), 0, stream, a, t);
-  else if (variant == kLazyLarge)
-    hipLaunchKernelGGL((uneven_ks_kernel<kLazyLarge, false>), grid,
-                       dim3(kBlock), 0, stream, a, t);
+    hipLaunchKernelGGL(uneven_ks_kernel<kLazySmall>, grid, dim3(kBlock), 0,
+                       stream, a, t);
   else
-    hipLaunchKernelGGL((uneven_ks_kernel<kLazySmall, true>), grid,
-                       dim3(kBlock), 0, stream, a, t);
+    hipLaunchKernelGGL(uneven_ks_kernel<kLazyLarge>, grid, dim3(kBlock), 0,
+                       stream, a, t);
 }
 
 void launch_uneven_moddown(const DeviceTables &t, const UnevenCt *cts,

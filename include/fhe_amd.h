@@ -750,29 +750,23 @@ int fhe_mod_raise(fhe_context *ctx, int count, const int64_t *in,
  *   "lazy_key_switch" 1    lazy transforms where results are canonicalized
  *                          later;
  *   "staged_modup" 1       ModUp through the Garner digits;
- *   "fuse_modup" 0, "fuse_tensor" 0   one-kernel variants (slower);
  *   "own_limbs" 1          partitions' own extended limbs from the NTT-form
  *                          input;
  *   "split_variants" 1     one NTT launch per arithmetic variant;
  *   "ks_lazy_accumulate" 1 small-prime key products summed without
  *                          intermediate reductions, large-prime sums kept
  *                          below 2q with one conditional subtraction;
- *   "ks_wide_accumulate" 0 small primes' key products summed as unreduced
- *                          96-bit values with one Montgomery reduction per
- *                          accumulator (fewer VALU instructions, measured
- *                          slower);
- *   "overlap_trio" 1       N = 2^16 with split_variants: the INTT of d0 and
+ *   "overlap_trio" 1       N >= 2^13 with split_variants: the INTT of d0 and
  *                          d1 in fhe_hmult_relin_rescale runs on a second
  *                          non-blocking stream of the context (default
  *                          priority), joined by an event before ModDown;
  *                          forked once the trio is written (1), or once
  *                          d2's INTT is done (2: beside the key inner
  *                          product, about 1% more throughput, that kernel's
- *                          launches then sharing the device); 0: one stream;
- *   "ks_occupancy" 2       waves per SIMD of the key inner product (3 trades
- *                          registers for occupancy; slower);
- *   "ks_prefetch" 0        the key inner product loads the next partition's
- *                          tile ahead (slower).
+ *                          launches then sharing the device); 0: one stream.
+ * "fuse_modup", "fuse_tensor", "ks_wide_accumulate", "ks_occupancy" and
+ * "ks_prefetch" name pipelines that the defaults have replaced; they are
+ * accepted and have no effect.
  * Synchronizes the context's stream. */
 int fhe_context_set_option(fhe_context *ctx, const char *name, int value);
 
