@@ -217,6 +217,24 @@ struct fhe_context {
     t.root_inverse = upload(params.root_inverse, owned);
     t.root_shoup = upload(params.root_shoup, owned);
     t.root_inverse_shoup = upload(params.root_inverse_shoup, owned);
+    {
+      // the F64 arithmetic's tables from the Shoup pairs' first words
+      const size_t words = size_t(params.prime_count) * params.n;
+      std::vector<double> d(words);
+      for (auto *table : {&params.root_shoup, &params.root_inverse_shoup}) {
+        for (size_t i = 0; i < words; i++)
+          d[i] = double((*table)[2 * i]);
+        (table == &params.root_shoup ? t.root_f64 : t.root_inverse_f64) =
+            upload(d, owned);
+      }
+      std::vector<double> qd(params.prime_count), qi(params.prime_count);
+      for (int i = 0; i < params.prime_count; i++) {
+        qd[i] = double(params.q[i]);
+        qi[i] = 1.0 / qd[i];
+      }
+      t.q_f64 = upload(qd, owned);
+      t.q_inverse_f64 = upload(qi, owned);
+    }
     t.p_inverse = upload(params.p_inverse_mult_r, owned);
     t.p_inverse_shoup = upload(params.p_inverse_shoup, owned);
     t.q_top = upload(params.q_top, owned);
@@ -830,7 +848,7 @@ struct fhe_context {
     });
     stage("intt_pass_high(acc)", [&] {
       fhe::ntt_inverse_second(tables, acc, acc, int64_t(count) * 2 * ext_limbs,
-                              ext_limbs, moduli_id, fhe::kInttExitReduce,
+                              ext_limbs, moduli_id, fhe::kInttKeyReduce,
                               stream, lazy);
     });
   }

@@ -25,6 +25,11 @@ struct DeviceTables {
   // standard-form twiddles with Shoup quotients, [prime][N][2]
   const uint64_t *root_shoup;
   const uint64_t *root_inverse_shoup;
+  // the standard-form twiddles as doubles, [prime][N] (primes below 2^42)
+  const double *root_f64;
+  const double *root_inverse_f64;
+  const double *q_f64;          // the prime and its rounded reciprocal
+  const double *q_inverse_f64;
   const int64_t *p_inverse;     // [alpha][prime_count]
   const uint64_t *p_inverse_shoup; // [alpha][prime_count][2] standard form
   const uint64_t *q_top;        // largest multiple of q below 2^63
@@ -44,7 +49,10 @@ struct DeviceTables {
 enum InttPost : int {
   kInttRaw = 0,       // plain INTT output, lazy in [0, 2q)
   kInttExit = 1,      // * N^-1, leave Montgomery form (to_intt)
-  kInttExitReduce = 2 // as kInttExit, then reduce [0, 2q) -> [0, q)
+  kInttExitReduce = 2, // as kInttExit, then reduce [0, 2q) -> [0, q)
+  // as kInttExitReduce, for the accumulators of the key inner product, which
+  // carry one more factor R in the kF64 arithmetic (ks_tile.h)
+  kInttKeyReduce = 3
 };
 
 constexpr int kBlock = 256;

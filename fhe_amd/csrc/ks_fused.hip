@@ -17,14 +17,15 @@ namespace fhe {
 
 namespace {
 
+// Waves per SIMD of the kF64 key inner product.
+constexpr int kKsF64Waves = 3;
+
 // Block -> (limb i, tile, ciphertext), ciphertext fastest: the blocks of a
 // key tile run together and share its reads through L2; with swizzle each of
 // the 8 XCDs (blocks are dealt round-robin to XCDs) gets one contiguous
 // range of that order.
-template <int LOGN>
-__global__ __launch_bounds__(kBlock) void ks_inner_product_r16_kernel(
-    KsArgs a, DeviceTables t) {
-  __shared__ int64_t lds[kR16Lds<r16_low_bits(LOGN)>];
+template <int LOGN, class F>
+__device__ __forceinline__ void ks_block(const KsArgs &a, F &&item) {
   constexpr int tiles = 1 << (LOGN - 12);
   int64_t w = blockIdx.x;
   if (a.swizzle) {
@@ -33,15 +34,33 @@ __global__ __launch_bounds__(kBlock) void ks_inner_product_r16_kernel(
   }
   const int ct = int(w % a.count);
   const int64_t rest = w / a.count;
-  const int tile = int(rest % tiles);
-  const int i = int(rest / tiles);
-  const KsBatchAddr<LOGN> ad(a, ct);
-  if (!a.lazy)
-    ks_item_tile<LOGN, kExact>(ad, t, lds, tile, i);
-  else if (t.q[a.moduli_id + i] < kLazySmallBound)
-    ks_item_tile<LOGN, kLazySmall>(ad, t, lds, tile, i);
-  else
-    ks_item_tile<LOGN, kLazyLarge>(ad, t, lds, tile, i);
+  item(ct, int(rest % tiles), a.limb0 + int(rest / tiles));
+}
+
+// One arithmetic per launch, over a run of extended limbs of its class.
+template <int LOGN, int A>
+__global__ __launch_bounds__(kBlock, A == kF64 ? kKsF64Waves : 2)
+void ks_inner_product_r16_kernel(KsArgs a, DeviceTables t) {
+  __shared__ int64_t lds[kR16Lds<r16_low_bits(LOGN)>];
+  ks_block<LOGN>(a, [&](int ct, int tile, int i) {
+    const KsBatchAddr<LOGN> ad(a, ct);
+    ks_item_tile<LOGN, A>(ad, t, lds, tile, i);
+  });
+}
+
+// The lazy arithmetic of each limb's class chosen per block: one launch for
+// all limbs.
+template <int LOGN>
+__global__ __launch_bounds__(kBlock, 2) void ks_inner_product_mixed_kernel(
+    KsArgs a, DeviceTables t) {
+  __shared__ int64_t lds[kR16Lds<r16_low_bits(LOGN)>];
+  ks_block<LOGN>(a, [&](int ct, int tile, int i) {
+    const KsBatchAddr<LOGN> ad(a, ct);
+    if (t.q[a.moduli_id + i] < kF64Bound)
+      ks_item_tile<LOGN, kF64>(ad, t, lds, tile, i);
+    else
+      ks_item_tile<LOGN, kLazyLarge>(ad, t, lds, tile, i);
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -149,6 +168,7 @@ struct ExtendArgs {
   int count, parts, ext_limbs, moduli_id, maxz, swizzle;
   int size[kMaxFusedParts];
   int start[kMaxFusedParts];
+  int limb0, limbs_here; // the launch's extended limbs
   int skip_own;          // leave each partition's own limbs unwritten
   uint32_t signed_mask;
 };
@@ -163,6 +183,7 @@ __device__ __forceinline__ void extend_ntt_tile(const ExtendArgs &a,
   it.digits = a.digits + cp * a.maxz * n;
   it.cst = a.cst + int64_t(part) * a.cst_stride;
   it.ext = a.ext + cp * a.ext_limbs * n;
+  it.start = a.start[part];
   it.size = a.size[part];
   it.ext_limbs = a.ext_limbs;
   it.moduli_id = a.moduli_id;
@@ -170,40 +191,98 @@ __device__ __forceinline__ void extend_ntt_tile(const ExtendArgs &a,
   ext_item_tile<LOGN, A, MAXZ, SIGNED>(it, t, lds, tile, i);
 }
 
-// six waves per SIMD for the lazy forms (the allocation alone ends just above
-// 80 registers, at five)
-template <int LOGN, int MAXZ, bool LAZY>
-__global__ __launch_bounds__(kBlock, LAZY && MAXZ <= 4 ? 6 : 2)
-void extend_ntt_r16_kernel(
-    ExtendArgs a, DeviceTables t) {
-  __shared__ uint32_t lds[kR16Lds<r16_high_bits(LOGN)>];
+// Block -> (extended limb, tile, ciphertext and partition), the limb
+// fastest: the 4096-coefficient digit tile is re-read by the blocks of the
+// other limbs through the XCD's L2.
+template <int LOGN, class F>
+__device__ __forceinline__ void extend_block(const ExtendArgs &a, F &&item) {
   constexpr int tiles = 1 << (LOGN - 12);
   int64_t w = blockIdx.x;
   if (a.swizzle) {
     const int64_t per = int64_t(gridDim.x) >> 3;
     w = int64_t(blockIdx.x & 7) * per + (blockIdx.x >> 3);
   }
-  // extended limb fastest, then tile, then (ciphertext, partition)
-  const int i = int(w % a.ext_limbs);
-  const int64_t rest = w / a.ext_limbs;
+  const int i = a.limb0 + int(w % a.limbs_here);
+  const int64_t rest = w / a.limbs_here;
   const int tile = int(rest % tiles);
   const int64_t cp = rest / tiles;
   const int part = int(cp % a.parts);
   // the whole block leaves (before any barrier) for a partition's own limb
   if (a.skip_own && i >= a.start[part] && i < a.start[part] + a.size[part])
     return;
-  const bool sgn = (a.signed_mask >> part) & 1;
-  if (!LAZY) {
-    if (sgn)
+  item(cp, part, tile, i);
+}
+
+// One lazy arithmetic per launch, over a run of extended limbs of its class
+// (no signed partitions).
+template <int LOGN, int MAXZ, int A>
+__global__ __launch_bounds__(kBlock, A == kF64 || MAXZ > 4 ? 4 : 6)
+void extend_ntt_r16_kernel(ExtendArgs a, DeviceTables t) {
+  __shared__ __align__(8) uint32_t lds[kExtendLds<LOGN, A>];
+  extend_block<LOGN>(a, [&](int64_t cp, int part, int tile, int i) {
+    extend_ntt_tile<LOGN, A, MAXZ, false>(a, t, lds, cp, part, tile, i);
+  });
+}
+
+// The arithmetic chosen per block: signed digits take the exact extension,
+// and the transform after it may be lazy all the same.
+template <int LOGN, int MAXZ, bool LAZY>
+__global__ __launch_bounds__(kBlock) void extend_ntt_mixed_kernel(
+    ExtendArgs a, DeviceTables t) {
+  __shared__ __align__(8) uint32_t lds[kExtendLds<LOGN, kF64>];
+  extend_block<LOGN>(a, [&](int64_t cp, int part, int tile, int i) {
+    const bool sgn = (a.signed_mask >> part) & 1;
+    const bool small = t.q[a.moduli_id + i] < kF64Bound;
+    if (LAZY && small) {
+      if (sgn)
+        extend_ntt_tile<LOGN, kF64, MAXZ, true>(a, t, lds, cp, part, tile, i);
+      else
+        extend_ntt_tile<LOGN, kF64, MAXZ, false>(a, t, lds, cp, part, tile, i);
+    } else if (sgn) {
       extend_ntt_tile<LOGN, kExact, MAXZ, true>(a, t, lds, cp, part, tile, i);
-    else
+    } else if (LAZY) {
+      extend_ntt_tile<LOGN, kLazyLarge, MAXZ, false>(a, t, lds, cp, part,
+                                                     tile, i);
+    } else {
       extend_ntt_tile<LOGN, kExact, MAXZ, false>(a, t, lds, cp, part, tile, i);
-  } else if (t.q[a.moduli_id + i] < kLazySmallBound) {
-    extend_ntt_tile<LOGN, kLazySmall, MAXZ, false>(a, t, lds, cp, part, tile, i);
-  } else {
-    extend_ntt_tile<LOGN, kLazyLarge, MAXZ, false>(a, t, lds, cp, part, tile, i);
+    }
+  });
+}
+
+// Calls f with log2 N as a compile-time constant.
+template <class F> void with_log_n(int log_n, F &&f) {
+  switch (log_n) {
+  case 13:
+    f(std::integral_constant<int, 13>());
+    break;
+  case 14:
+    f(std::integral_constant<int, 14>());
+    break;
+  case 15:
+    f(std::integral_constant<int, 15>());
+    break;
+  default:
+    f(std::integral_constant<int, 16>());
   }
 }
+
+// Calls f(first limb, limbs, small) for each run of extended limbs of one
+// prime class.
+template <class F>
+void for_class_runs(const DeviceTables &t, int moduli_id, int limbs, F &&f) {
+  for (int l = 0; l < limbs;) {
+    const bool small = t_host_q_small(t, moduli_id + l);
+    int e = l + 1;
+    while (e < limbs && t_host_q_small(t, moduli_id + e) == small)
+      e++;
+    f(l, e - l, small);
+    l = e;
+  }
+}
+
+// Launches with fewer blocks than this choose the arithmetic per block: a
+// launch more costs them more than the registers of the larger kernel.
+constexpr int64_t kSplitBlocks = 1024;
 
 } // namespace
 
@@ -227,12 +306,10 @@ void launch_staged_modup(const DeviceTables &t, const int64_t *x,
                          hipStream_t stream) {
   int maxz = 1;
   uint32_t mask = 0;
-  bool any_signed = false;
   for (int p = 0; p < parts; p++) {
     while (maxz < sizes[p])
       maxz <<= 1;
     mask |= is_signed[p] ? (uint32_t(1) << p) : 0u;
-    any_signed = any_signed || is_signed[p];
   }
   DigitArgs d{};
   d.x = x;
@@ -264,57 +341,58 @@ void launch_staged_modup(const DeviceTables &t, const int64_t *x,
     e.size[p] = sizes[p];
     e.start[p] = starts[p];
   }
-  // the lazy extension needs canonical digits: only for non-negative ones
-  const bool use_lazy = lazy && !any_signed;
   const int tiles = int((int64_t(1) << t.log_n) >> 12);
-  const int64_t eblocks = int64_t(count) * parts * tiles * e.ext_limbs;
-  e.swizzle = eblocks % 8 == 0 ? 1 : 0;
+  const int64_t per_limb = int64_t(count) * parts * tiles;
   const dim3 dgrid(grid_for((int64_t(count) * parts) << t.log_n));
-  const dim3 egrid{unsigned(eblocks), 1, 1};
   const bool chunked = chunked_ok(t.log_n, {x, digits}) && x_stride % 2 == 0;
-#define FHE_EXTEND(L, W)                                                       \
-  do {                                                                         \
-    if (use_lazy)                                                              \
-      hipLaunchKernelGGL((extend_ntt_r16_kernel<L, W, true>), egrid,           \
-                         dim3(kBlock), 0, stream, e, t);                       \
-    else                                                                       \
-      hipLaunchKernelGGL((extend_ntt_r16_kernel<L, W, false>), egrid,          \
-                         dim3(kBlock), 0, stream, e, t);                       \
-  } while (0)
-#define FHE_STAGED(W)                                                          \
-  do {                                                                         \
-    if (chunked)                                                               \
-      hipLaunchKernelGGL(modup_digits_chunk_kernel<W>,                         \
-                         dim3(unsigned(((int64_t(count) * parts) << t.log_n) / \
-                                       kChunk)),                               \
-                         dim3(kBlock), 0, stream, d, t);                       \
-    else                                                                       \
-      hipLaunchKernelGGL(modup_digits_kernel<W>, dgrid, dim3(kBlock), 0,      \
-                         stream, d, t);                                        \
-    switch (t.log_n) {                                                         \
-    case 13:                                                                   \
-      FHE_EXTEND(13, W);                                                       \
-      break;                                                                   \
-    case 14:                                                                   \
-      FHE_EXTEND(14, W);                                                       \
-      break;                                                                   \
-    case 15:                                                                   \
-      FHE_EXTEND(15, W);                                                       \
-      break;                                                                   \
-    default:                                                                   \
-      FHE_EXTEND(16, W);                                                       \
-    }                                                                          \
-  } while (0)
-  if (maxz == 1)
-    FHE_STAGED(1);
-  else if (maxz == 2)
-    FHE_STAGED(2);
-  else if (maxz == 4)
-    FHE_STAGED(4);
-  else
-    FHE_STAGED(8);
-#undef FHE_STAGED
-#undef FHE_EXTEND
+  // the extensions of the limbs [l, l + n): small per class, or mixed (-1)
+  auto extend = [&](auto logn, auto width, int l, int n, int small) {
+    constexpr int LOGN = decltype(logn)::value, W = decltype(width)::value;
+    e.limb0 = l;
+    e.limbs_here = n;
+    const int64_t blocks = per_limb * n;
+    e.swizzle = blocks % 8 == 0 ? 1 : 0;
+    const dim3 grid{unsigned(blocks), 1, 1};
+    if (small == 1)
+      hipLaunchKernelGGL((extend_ntt_r16_kernel<LOGN, W, kF64>), grid,
+                         dim3(kBlock), 0, stream, e, t);
+    else if (small == 0)
+      hipLaunchKernelGGL((extend_ntt_r16_kernel<LOGN, W, kLazyLarge>), grid,
+                         dim3(kBlock), 0, stream, e, t);
+    else if (lazy)
+      hipLaunchKernelGGL((extend_ntt_mixed_kernel<LOGN, W, true>), grid,
+                         dim3(kBlock), 0, stream, e, t);
+    else
+      hipLaunchKernelGGL((extend_ntt_mixed_kernel<LOGN, W, false>), grid,
+                         dim3(kBlock), 0, stream, e, t);
+  };
+  auto staged = [&](auto logn, auto width) {
+    constexpr int W = decltype(width)::value;
+    if (chunked)
+      hipLaunchKernelGGL(
+          modup_digits_chunk_kernel<W>,
+          dim3(unsigned(((int64_t(count) * parts) << t.log_n) / kChunk)),
+          dim3(kBlock), 0, stream, d, t);
+    else
+      hipLaunchKernelGGL(modup_digits_kernel<W>, dgrid, dim3(kBlock), 0,
+                         stream, d, t);
+    if (lazy && mask == 0 && per_limb * e.ext_limbs >= kSplitBlocks)
+      for_class_runs(t, moduli_id, e.ext_limbs, [&](int l, int n, bool small) {
+        extend(logn, width, l, n, small ? 1 : 0);
+      });
+    else
+      extend(logn, width, 0, e.ext_limbs, -1);
+  };
+  with_log_n(t.log_n, [&](auto logn) {
+    if (maxz == 1)
+      staged(logn, std::integral_constant<int, 1>());
+    else if (maxz == 2)
+      staged(logn, std::integral_constant<int, 2>());
+    else if (maxz == 4)
+      staged(logn, std::integral_constant<int, 4>());
+    else
+      staged(logn, std::integral_constant<int, 8>());
+  });
 }
 
 void launch_ks_inner_product_fused(const DeviceTables &t, const int64_t *ext,
@@ -338,8 +416,6 @@ void launch_ks_inner_product_fused(const DeviceTables &t, const int64_t *ext,
   a.key_chain = key_chain;
   a.key_offset = key_offset;
   a.key_partition0 = key_partition0;
-  a.swizzle = blocks % 8 == 0 ? 1 : 0;
-  a.lazy = lazy ? 1 : 0;
   a.own = own;
   a.own_stride = own_stride;
   a.lazy_acc = lazy_accumulate ? 1 : 0;
@@ -347,24 +423,27 @@ void launch_ks_inner_product_fused(const DeviceTables &t, const int64_t *ext,
     a.start[p] = own ? starts[p] : 0;
     a.size[p] = own ? sizes[p] : 0;
   }
-  const dim3 grid{unsigned(blocks), 1, 1};
-#define FHE_KS(LOGN)                                                           \
-  hipLaunchKernelGGL(ks_inner_product_r16_kernel<LOGN>, grid, dim3(kBlock), 0, \
-                     stream, a, t)
-  switch (t.log_n) {
-  case 13:
-    FHE_KS(13);
-    break;
-  case 14:
-    FHE_KS(14);
-    break;
-  case 15:
-    FHE_KS(15);
-    break;
-  default:
-    FHE_KS(16);
-  }
-#undef FHE_KS
+  with_log_n(t.log_n, [&](auto logn) {
+    constexpr int LOGN = decltype(logn)::value;
+    auto launch = [&](auto *kernel, int l, int n) {
+      a.limb0 = l;
+      const int64_t b = blocks / ext_limbs * n;
+      a.swizzle = b % 8 == 0 ? 1 : 0;
+      hipLaunchKernelGGL(kernel, dim3(unsigned(b)), dim3(kBlock), 0, stream, a,
+                         t);
+    };
+    if (!lazy)
+      launch(ks_inner_product_r16_kernel<LOGN, kExact>, 0, ext_limbs);
+    else if (blocks < kSplitBlocks)
+      launch(ks_inner_product_mixed_kernel<LOGN>, 0, ext_limbs);
+    else
+      for_class_runs(t, moduli_id, ext_limbs, [&](int l, int n, bool small) {
+        if (small)
+          launch(ks_inner_product_r16_kernel<LOGN, kF64>, l, n);
+        else
+          launch(ks_inner_product_r16_kernel<LOGN, kLazyLarge>, l, n);
+      });
+  });
 }
 
 } // namespace fhe

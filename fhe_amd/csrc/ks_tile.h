@@ -33,8 +33,8 @@ struct KsArgs {
   int key_chain;
   int key_offset;      // first key limb aligned with the ciphertext's limb 0
   int key_partition0;  // key partition index of the ciphertext's partition 0
+  int limb0;           // first extended limb of the launch
   int swizzle;
-  int lazy;            // lazy transforms (the ext pass before was lazy too)
   // NTT form of the key-switched polynomial, when the caller has it: limb i
   // of ciphertext c at own + c * own_stride + i * N.  The extended limbs of a
   // partition's own primes are that polynomial's limbs, so their transforms
@@ -44,7 +44,7 @@ struct KsArgs {
   int64_t own_stride;
   int start[kMaxFusedParts];
   int size[kMaxFusedParts];
-  int lazy_acc;        // small primes: accumulate without guards
+  int lazy_acc;        // large primes: sums below 2q with one guard
 };
 
 
@@ -63,11 +63,12 @@ struct KsArgs {
 // products are canonicalized later).
 
 // The (extended limb i, tile) work item of one ciphertext with arithmetic A
-// for the two transforms.  The key products are Montgomery products of
-// operands whose product stays below q * 2^62, accumulated with the
-// reference's guards; on small primes, lazy_acc sums the reduced products
-// and brings the sum under 2q once.  Every form gives the same residues, and
-// the accumulators are canonicalized after the inverse transform.
+// for the two transforms.  The key products of the 64-bit forms are
+// Montgomery products of operands whose product stays below q * 2^62,
+// accumulated with the reference's guards (lazy_acc: one conditional
+// subtraction for kLazyLarge); the kF64 sums need no guards (up to 64 parts
+// of less than 0.55 q each).  Every form gives the same residues, and the
+// accumulators are canonicalized after the inverse transform.
 // LOGN: log2 N.
 // OPAQUE: the tile runs inside a persistent loop (opaque_tid).
 template <int LOGN, int A, class Addr, bool OPAQUE = false>
@@ -84,33 +85,34 @@ __device__ __forceinline__ void ks_item_tile(const Addr &a,
   const int64_t off = sp << L;
 
   R16Pass f;
-  f.tw = t.root + int64_t(p) * n;
-  f.ts = t.root_shoup + int64_t(p) * n * 2;
-  f.n = n;
+  r16_prime<A, false>(f, t, p);
   f.hi = sp;
-  f.log_n = t.log_n;
   f.b = 0;
   f.r = r;
-  f.q = t.q[p];
-  f.k = t.k[p];
-  f.q2 = int64_t(t.q2[p]);
-  f.nq2 = A == kExact ? opaque_neg(f.q2) : 0;  // exact guards only
-  f.nq = A == kExact ? 0 : uint64_t(opaque_neg(int64_t(f.q)));
   const int64_t qq = int64_t(f.q);
 
-  int64_t acc0[16], acc1[16], v[16];
+  R16Value<A> acc0[16], acc1[16], v[16];
   for (int pp = 0; pp < a.parts; pp++) {
+    int64_t w[16];
     // block-uniform: every thread of the block has the same (i, pp)
     if (a.is_own(pp, i)) {
       const int64_t *src = a.own(i, off);
 #pragma unroll
       for (int m = 0; m < 16; m++)
-        v[m] = src[r16_point<L, true>(r, m)];
+        w[m] = src[r16_point<L, true>(r, m)];
+      if constexpr (A == kF64) {
+        f64_load(w, v, f.f);
+      } else {
+#pragma unroll
+        for (int m = 0; m < 16; m++)
+          v[m] = w[m];
+      }
     } else {
       const int64_t *src = a.ext(pp, i, off);
 #pragma unroll
       for (int m = 0; m < 16; m++)
-        v[m] = src[r16_point<L, false>(r, m)];
+        v[m] = __builtin_bit_cast(R16Value<A>,
+                                  src[r16_point<L, false>(r, m)]);
       r16_forward_high<L, A>(v, f);
       r16_exchange<L, true, true>(v, lds, c, r);
       r16_forward_low<L, A>(v, f);
@@ -119,19 +121,21 @@ __device__ __forceinline__ void ks_item_tile(const Addr &a,
     // v[m] is now the NTT value at coefficient off + 16 r + m
     const int64_t *k0 = a.key_tile(pp, i, off) + 16 * r;
     const int64_t *k1 = k0 + int64_t(a.key_chain) * n;
-    if (pp == 0) {
+    if constexpr (A == kF64) {
+      // plain products: the sums carry the key's Montgomery factor R, which
+      // the epilogue of the second inverse pass takes out (kInttKeyReduce)
+#pragma unroll
+      for (int m = 0; m < 16; m++) {
+        const double x0 = f64_mul(v[m], f64_from_int(k0[m]), f.f);
+        const double x1 = f64_mul(v[m], f64_from_int(k1[m]), f.f);
+        acc0[m] = pp == 0 ? x0 : acc0[m] + x0;
+        acc1[m] = pp == 0 ? x1 : acc1[m] + x1;
+      }
+    } else if (pp == 0) {
 #pragma unroll
       for (int m = 0; m < 16; m++) {
         acc0[m] = mont_mult_u(v[m], k0[m], f.q, f.k);
         acc1[m] = mont_mult_u(v[m], k1[m], f.q, f.k);
-      }
-    } else if (A == kLazySmall && a.lazy_acc) {
-      // q < 2^42: the sum of the parts' products (each below 2q) stays far
-      // below 2^63; it is brought back under 2q once, after the loop
-#pragma unroll
-      for (int m = 0; m < 16; m++) {
-        acc0[m] = add64(mont_mult_u(v[m], k0[m], f.q, f.k), acc0[m]);
-        acc1[m] = add64(mont_mult_u(v[m], k1[m], f.q, f.k), acc1[m]);
       }
     } else if (A == kLazyLarge && a.lazy_acc) {
       // sums kept below 2q (one conditional subtraction of 2q): the lazy
@@ -156,31 +160,22 @@ __device__ __forceinline__ void ks_item_tile(const Addr &a,
     }
   }
 
-  if (A == kLazySmall && a.lazy_acc && a.parts > 1) {
-    // acc < 2q * parts: halving guards from 2q * 2^ceil(log2(parts) - 1)
-    int64_t bound = f.q2;
-    while (bound < f.q2 * a.parts)
-      bound <<= 1;
-    for (bound >>= 1; bound >= f.q2; bound >>= 1) {
-#pragma unroll
-      for (int m = 0; m < 16; m++) {
-        acc0[m] = guard_u(acc0[m], bound);
-        acc1[m] = guard_u(acc1[m], bound);
-      }
-    }
-  }
   R16Pass g = f;
-  g.tw = t.root_inverse + int64_t(p) * n;
-  g.ts = t.root_inverse_shoup + int64_t(p) * n * 2;
+  r16_prime<A, true>(g, t, p);
   int64_t *d0 = a.acc(i, off);
   int64_t *d1 = d0 + int64_t(a.ext_limbs) * n;
-  auto inverse = [&](int64_t (&x)[16], int64_t *d) {
+  auto inverse = [&](R16Value<A> (&x)[16], int64_t *d) {
+    if constexpr (A == kF64) {
+#pragma unroll
+      for (int m = 0; m < 16; m++)
+        x[m] = f64_center(x[m], f.f);
+    }
     r16_inverse_low<L, A>(x, g);
     r16_exchange<L, false, true>(x, lds, c, r);
     r16_inverse_high<L, A>(x, g);
 #pragma unroll
     for (int m = 0; m < 16; m++)
-      d[r16_point<L, false>(r, m)] = x[m];
+      d[r16_point<L, false>(r, m)] = __builtin_bit_cast(int64_t, x[m]);
   };
   inverse(acc0, d0);
   inverse(acc1, d1);
@@ -221,10 +216,18 @@ struct ExtItem {
   const int64_t *digits; // this partition's [maxz][N] Garner digits
   const int64_t *cst;    // this partition's ModUp constants
   int64_t *ext;          // this partition's [ext_limbs][N]
-  int size, ext_limbs, moduli_id, ext_shoup_offset;
+  int start, size, ext_limbs, moduli_id, ext_shoup_offset;
 };
 
-// LOGN, OPAQUE: as for ks_item_tile.
+// lds: kExtendLds<LOGN, A> words.  LOGN, OPAQUE: as for ks_item_tile.
+//
+// The 64-bit forms exchange through 32-bit words (half the LDS: six waves per
+// SIMD); kF64 holds about 100 registers, so that four waves fit either way,
+// and takes the 64-bit exchange with half the barriers.
+template <int LOGN, int A>
+constexpr int kExtendLds =
+    kR16Lds<r16_high_bits(LOGN)> * (A == kF64 ? 2 : 1);
+
 template <int LOGN, int A, int MAXZ, bool SIGNED, bool OPAQUE = false>
 __device__ __forceinline__ void ext_item_tile(const ExtItem &a,
                                               const DeviceTables &t,
@@ -238,44 +241,81 @@ __device__ __forceinline__ void ext_item_tile(const ExtItem &a,
   const int size = a.size;
   const int64_t *dg = a.digits + sp;
   R16Pass s;
-  s.tw = t.root + int64_t(p) * n;
-  s.ts = t.root_shoup + int64_t(p) * n * 2;
-  s.n = n;
+  r16_prime<A, false>(s, t, p);
   s.hi = 0;
-  s.log_n = t.log_n;
   s.b = b;
   s.r = r;
-  s.q = t.q[p];
-  s.k = t.k[p];
-  s.q2 = int64_t(t.q2[p]);
-  s.nq2 = A == kExact ? opaque_neg(s.q2) : 0;  // exact guards only
-  s.nq = A == kExact ? 0 : uint64_t(opaque_neg(int64_t(s.q)));
-  int64_t v[16];
+  R16Value<A> v[16];
+  if constexpr (A == kF64 && !SIGNED) {
+    // one digit at a time: sum_j d_j c_j, each product below 0.55 q
+    const uint64_t *es =
+        reinterpret_cast<const uint64_t *>(a.cst + a.ext_shoup_offset) + 2 * i;
 #pragma unroll
-  for (int m = 0; m < 16; m++) {
-    int64_t d[MAXZ];
+    for (int j = 0; j < MAXZ; j++) {
+      if (j < size) {
+        int64_t d[16];
 #pragma unroll
-    for (int j = 0; j < MAXZ; j++)
-      d[j] = j < size ? dg[int64_t(j) * n +
-                           (int64_t(r16_point<L, false>(r, m)) << b)]
-                      : 0;
-    if (A == kExact)
-      v[m] = extend_limb<MAXZ, SIGNED>(d, size, i, a.ext_limbs,
-                                       a.cst + CkksParams::kKsExtOffset, s.q,
-                                       s.k, s.q2);
-    else
-      v[m] = extend_limb_lazy<MAXZ>(
-          d, size, i, a.ext_limbs,
-          reinterpret_cast<const uint64_t *>(a.cst + a.ext_shoup_offset), s.q,
-          s.nq, A == kLazySmall);
+        for (int m = 0; m < 16; m++)
+          d[m] =
+              dg[int64_t(j) * n + (int64_t(r16_point<L, false>(r, m)) << b)];
+        const double cj = double(es[2 * int64_t(j) * a.ext_limbs]);
+        // the digits of primes below 2^42 are below their prime but for the
+        // first, the input itself, which f64_load looks at; those of larger
+        // primes are reduced
+        double x[16];
+        const bool digit_small =
+            t.q[a.moduli_id + a.start + j] < kF64Bound; // block-uniform
+        if (j == 0) {
+          f64_load(d, x, s.f);
+        } else {
+#pragma unroll
+          for (int m = 0; m < 16; m++)
+            x[m] = digit_small ? f64_from_int(d[m]) : f64_from_any(d[m], s.f);
+        }
+#pragma unroll
+        for (int m = 0; m < 16; m++) {
+          const double y = f64_mul(x[m], cj, s.f);
+          v[m] = j == 0 ? y : v[m] + y;
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < 16; m++) {
+      int64_t d[MAXZ];
+#pragma unroll
+      for (int j = 0; j < MAXZ; j++)
+        d[j] = j < size
+                   ? dg[int64_t(j) * n +
+                        (int64_t(r16_point<L, false>(r, m)) << b)]
+                   : 0;
+      int64_t y;
+      if (A == kExact || SIGNED)
+        y = extend_limb<MAXZ, SIGNED>(d, size, i, a.ext_limbs,
+                                      a.cst + CkksParams::kKsExtOffset, s.q,
+                                      s.k, s.q2);
+      else
+        y = extend_limb_lazy<MAXZ>(
+            d, size, i, a.ext_limbs,
+            reinterpret_cast<const uint64_t *>(a.cst + a.ext_shoup_offset),
+            s.q, s.nq, false);
+      if constexpr (A == kF64)
+        v[m] = f64_from_int(y);
+      else
+        v[m] = y;
+    }
   }
   r16_forward_high<L, A>(v, s);
-  r16_exchange_words<L, true>(v, lds, c, r);
+  if constexpr (A == kF64)
+    r16_exchange<L, true>(v, reinterpret_cast<int64_t *>(lds), c, r);
+  else
+    r16_exchange_words<L, true>(v, lds, c, r);
   r16_forward_low<L, A>(v, s);
   int64_t *out = a.ext + int64_t(i) * n + sp;
 #pragma unroll
   for (int m = 0; m < 16; m++)
-    out[int64_t(r16_point<L, true>(r, m)) << b] = v[m];
+    out[int64_t(r16_point<L, true>(r, m)) << b] =
+        __builtin_bit_cast(int64_t, v[m]);
 }
 
 } // namespace fhe

@@ -135,7 +135,7 @@ __global__ __launch_bounds__(kBlock) void ntt_pass_kernel(PassArgs a,
       const int p = a.moduli_id + int(f % a.limbs);
       const uint64_t q = t.q[p], k = t.k[p];
       v = mont_exit(mont_mult_cs(t.ninv[p], v, q, k), q, k);
-      if (a.post == kInttExitReduce)
+      if (a.post != kInttExit)
         v = guard(v, int64_t(q));
     }
     a.dst[f * n + i] = v;
@@ -206,8 +206,8 @@ __global__ __launch_bounds__(kBlock) void ntt_radix16_mixed_kernel(
   const bool lazy = a.lazy_period > 0 && (poly % a.lazy_period) < a.lazy_count;
   if (!lazy)
     r16_pass<L, INV, COLS, kExact>(a, t, lds, poly, tile, l);
-  else if (t.q[a.moduli_id + l] < kLazySmallBound)
-    r16_pass<L, INV, COLS, kLazySmall>(a, t, lds, poly, tile, l);
+  else if (r16_supported(t.log_n) && t.q[a.moduli_id + l] < kF64Bound)
+    r16_pass<L, INV, COLS, kF64>(a, t, lds, poly, tile, l);
   else
     r16_pass<L, INV, COLS, kLazyLarge>(a, t, lds, poly, tile, l);
 }
@@ -253,8 +253,8 @@ void launch_r16_pass(const PassArgs &a, const DeviceTables &t,
     if (arith == kExact)
       hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, kExact>), grid,
                          dim3(kBlock), 0, stream, a, t, sel, tiles, swizzle);
-    else if (arith == kLazySmall)
-      hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, kLazySmall>), grid,
+    else if (arith == kF64)
+      hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, kF64>), grid,
                          dim3(kBlock), 0, stream, a, t, sel, tiles, swizzle);
     else
       hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, kLazyLarge>), grid,
@@ -277,11 +277,15 @@ void launch_r16_pass(const PassArgs &a, const DeviceTables &t,
   if (lazy_count > 0 && a.lazy_part != 1) {
     int l = 0;
     while (l < a.limbs) {
-      const bool small = t_host_q_small(t, a.moduli_id + l);
+      // (the generic second pass of N = 2^17 takes no doubles)
+      auto is_small = [&](int limb) {
+        return r16_supported(t.log_n) && t_host_q_small(t, a.moduli_id + limb);
+      };
+      const bool small = is_small(l);
       int e = l + 1;
-      while (e < a.limbs && t_host_q_small(t, a.moduli_id + e) == small)
+      while (e < a.limbs && is_small(e) == small)
         e++;
-      launch(small ? kLazySmall : kLazyLarge,
+      launch(small ? kF64 : kLazyLarge,
              PolySelect{periods * lazy_count, period, lazy_count, 0, l},
              e - l);
       l = e;

@@ -16,12 +16,11 @@
 //   kExact      the reference's radix-2 formulas with Montgomery twiddles
 //               (src/operation/ntt.cpp:46-134, :177-272), so every lazy
 //               representative in [0, 2q) matches the reference;
-//   kLazySmall  for q < 2^42: Shoup products with standard-form twiddles and
-//               no reductions inside the transform.  Forward values grow by
-//               less than 2q per stage; inverse sums double per stage and the
-//               difference of global stage t is offset by q << (1 + t) (a
-//               bound of every input of that stage when the transform's input
-//               is below 2q).  Sixteen stages stay below 2^60.
+//   kF64        for q < 2^42: integers in doubles (f64mod.h), standard-form
+//               twiddles, no reductions inside a pass.  Between the two
+//               passes of a transform the values stay doubles (in the int64
+//               buffers); the first pass reads integers and the last one
+//               writes integers.
 //   kLazyLarge  Harvey's lazy forms for any q < 2^61: forward values in
 //               [0, 4q) with one conditional subtraction per butterfly,
 //               inverse values in [0, 2q).
@@ -30,13 +29,18 @@
 // dependent reads them.
 #pragma once
 
+#include <type_traits>
+
 #include "device.h"
+#include "f64mod.h"
 
 namespace fhe {
 
 // Low (contiguous) and high (strided) index bits of the two radix-16 passes
 // of N = 2^log_n, and the sizes they serve.
-inline bool r16_supported(int log_n) { return log_n >= 13 && log_n <= 16; }
+__host__ __device__ constexpr bool r16_supported(int log_n) {
+  return log_n >= 13 && log_n <= 16;
+}
 __host__ __device__ constexpr int r16_low_bits(int log_n) {
   return (log_n + 1) / 2;
 }
@@ -44,14 +48,18 @@ __host__ __device__ constexpr int r16_high_bits(int log_n) {
   return log_n - r16_low_bits(log_n);
 }
 
-enum NttArith : int { kExact = 0, kLazySmall = 1, kLazyLarge = 2 };
+enum NttArith : int { kExact = 0, kF64 = 1, kLazyLarge = 2 };
 
-// Primes below this bound take the kLazySmall forms.
-constexpr uint64_t kLazySmallBound = uint64_t(1) << 42;
+// Values of a transform in arithmetic A.
+template <int A>
+using R16Value = std::conditional_t<A == kF64, double, int64_t>;
 
-// Host side: whether prime p takes the kLazySmall forms.
+// Primes below this bound take the kF64 forms.
+constexpr uint64_t kF64Bound = uint64_t(1) << 42;
+
+// Host side: whether prime p takes the kF64 forms.
 inline bool t_host_q_small(const DeviceTables &t, int p) {
-  return t.host_q[p] < kLazySmallBound;
+  return t.host_q[p] < kF64Bound;
 }
 
 // Exact butterflies with the reference's signed arithmetic.  Operands are
@@ -110,7 +118,8 @@ __device__ __forceinline__ int64_t load_product(int64_t v, int64_t c,
 // sub-transform's index bits above b+L and r the thread's row.
 struct R16Pass {
   const int64_t *tw;   // Montgomery twiddles of this prime (kExact)
-  const uint64_t *ts;  // {w, w'} pairs of this prime (lazy forms)
+  const uint64_t *ts;  // {w, w'} pairs of this prime (kLazyLarge)
+  const double *tf;    // twiddles of this prime (kF64)
   int64_t n;
   int64_t hi;
   int log_n;
@@ -119,50 +128,72 @@ struct R16Pass {
   int64_t q2;
   int64_t nq2;  // -q2 through opaque_neg, for the exact arithmetic
   uint64_t q, k;
-  uint64_t nq;  // 2^64 - q through opaque_neg, for the lazy forms
+  uint64_t nq;  // 2^64 - q through opaque_neg, for kLazyLarge
+  F64Mod f;     // kF64
 };
+
+// The fields of a pass that depend on the prime p.
+template <int A, bool INV>
+__device__ __forceinline__ void r16_prime(R16Pass &s, const DeviceTables &t,
+                                          int p) {
+  const int64_t at = int64_t(p) << t.log_n;
+  s.n = int64_t(1) << t.log_n;
+  s.log_n = t.log_n;
+  s.q = t.q[p];
+  s.k = t.k[p];
+  s.q2 = int64_t(t.q2[p]);
+  if (A == kExact) {
+    s.tw = (INV ? t.root_inverse : t.root) + at;
+    s.nq2 = opaque_neg(s.q2);
+  } else if (A == kLazyLarge) {
+    s.ts = (INV ? t.root_inverse_shoup : t.root_shoup) + at * 2;
+    s.nq = uint64_t(opaque_neg(int64_t(s.q)));
+  } else {
+    s.tf = (INV ? t.root_inverse_f64 : t.root_f64) + at;
+    s.f = {t.q_f64[p], t.q_inverse_f64[p]};
+  }
+}
 
 // One forward butterfly on (x, y) with twiddle entry idx.
 template <int A>
-__device__ __forceinline__ void fwd_bfly(int64_t &x, int64_t &y,
+__device__ __forceinline__ void fwd_bfly(R16Value<A> &x, R16Value<A> &y,
                                          const R16Pass &s, int64_t idx) {
-  if (A == kExact) {
+  if constexpr (A == kExact) {
     ct_butterfly(x, y, s.tw[idx], s.q2, s.nq2, s.q, s.k);
-    return;
+  } else if constexpr (A == kF64) {
+    const double p = f64_mul(y, s.tf[idx], s.f);
+    y = x - p;
+    x = x + p;
+  } else {
+    const uint64_t w = s.ts[2 * idx], wq = s.ts[2 * idx + 1];
+    const int64_t x0 = guard_u(x, s.q2);
+    const int64_t p = int64_t(shoup_mult_neg(uint64_t(y), w, wq, s.nq));
+    x = add64(x0, p);
+    y = sub64(add64(x0, s.q2), p);
   }
-  const uint64_t w = s.ts[2 * idx], wq = s.ts[2 * idx + 1];
-  int64_t x0 = x;
-  if (A == kLazyLarge)
-    x0 = guard_u(x0, s.q2);
-  const int64_t t = int64_t(shoup_mult_neg(uint64_t(y), w, wq, s.nq));
-  x = add64(x0, t);
-  y = sub64(add64(x0, s.q2), t);
 }
 
-// One inverse butterfly at global stage t.
+// One inverse butterfly.
 template <int A>
-__device__ __forceinline__ void inv_bfly(int64_t &x, int64_t &y,
-                                         const R16Pass &s, int64_t idx,
-                                         int t) {
-  if (A == kExact) {
+__device__ __forceinline__ void inv_bfly(R16Value<A> &x, R16Value<A> &y,
+                                         const R16Pass &s, int64_t idx) {
+  if constexpr (A == kExact) {
     gs_butterfly(x, y, s.tw[idx], s.q2, s.nq2, s.q, s.k);
-    return;
+  } else if constexpr (A == kF64) {
+    const double d = x - y;
+    x = x + y;
+    y = f64_mul(d, s.tf[idx], s.f);
+  } else {
+    const uint64_t w = s.ts[2 * idx], wq = s.ts[2 * idx + 1];
+    const int64_t d = sub64(add64(x, s.q2), y);
+    x = guard_u(add64(x, y), s.q2);
+    y = int64_t(shoup_mult_neg(uint64_t(d), w, wq, s.nq));
   }
-  const uint64_t w = s.ts[2 * idx], wq = s.ts[2 * idx + 1];
-  int64_t sum = add64(x, y);
-  int64_t off = s.q2;
-  if (A == kLazyLarge)
-    sum = guard_u(sum, s.q2);
-  else
-    off = int64_t(s.q << (1 + t));
-  const int64_t d = sub64(add64(x, off), y);
-  x = sum;
-  y = int64_t(shoup_mult_neg(uint64_t(d), w, wq, s.nq));
 }
 
 // forward local bits L-1..L-4, ROWS ownership
-template <int L, int A = kExact>
-__device__ __forceinline__ void r16_forward_high(int64_t (&v)[16],
+template <int L, int A>
+__device__ __forceinline__ void r16_forward_high(R16Value<A> (&v)[16],
                                                  const R16Pass &s) {
 #pragma unroll
   for (int x = 3; x >= 0; x--) {
@@ -179,8 +210,8 @@ __device__ __forceinline__ void r16_forward_high(int64_t (&v)[16],
 }
 
 // forward local bits L-5..0, COLS ownership
-template <int L, int A = kExact>
-__device__ __forceinline__ void r16_forward_low(int64_t (&v)[16],
+template <int L, int A>
+__device__ __forceinline__ void r16_forward_low(R16Value<A> (&v)[16],
                                                 const R16Pass &s) {
 #pragma unroll
   for (int u = L - 5; u >= 0; u--) {
@@ -197,8 +228,8 @@ __device__ __forceinline__ void r16_forward_low(int64_t (&v)[16],
 }
 
 // inverse local bits 0..L-5, COLS ownership
-template <int L, int A = kExact>
-__device__ __forceinline__ void r16_inverse_low(int64_t (&v)[16],
+template <int L, int A>
+__device__ __forceinline__ void r16_inverse_low(R16Value<A> (&v)[16],
                                                 const R16Pass &s) {
 #pragma unroll
   for (int u = 0; u <= L - 5; u++) {
@@ -208,14 +239,14 @@ __device__ __forceinline__ void r16_inverse_low(int64_t (&v)[16],
     for (int m = 0; m < 16; m++) {
       if (m & (1 << u))
         continue;
-      inv_bfly<A>(v[m], v[m + (1 << u)], s, tb + (m >> (u + 1)), s.b + u);
+      inv_bfly<A>(v[m], v[m + (1 << u)], s, tb + (m >> (u + 1)));
     }
   }
 }
 
 // inverse local bits L-4..L-1, ROWS ownership
-template <int L, int A = kExact>
-__device__ __forceinline__ void r16_inverse_high(int64_t (&v)[16],
+template <int L, int A>
+__device__ __forceinline__ void r16_inverse_high(R16Value<A> (&v)[16],
                                                  const R16Pass &s) {
 #pragma unroll
   for (int x = 0; x <= 3; x++) {
@@ -225,21 +256,20 @@ __device__ __forceinline__ void r16_inverse_high(int64_t (&v)[16],
     for (int m = 0; m < 16; m++) {
       if (m & (1 << x))
         continue;
-      inv_bfly<A>(v[m], v[m + (1 << x)], s, tb + (m >> (x + 1)), s.b + u);
+      inv_bfly<A>(v[m], v[m + (1 << x)], s, tb + (m >> (x + 1)));
     }
   }
 }
 
-// Bring lazy forward outputs to [0, 2q) (kLazyLarge values are below 4q;
-// kLazySmall values are left as they are: their consumers accept them).
+// Bring kLazyLarge forward outputs (below 4q) to [0, 2q).
 template <int A>
-__device__ __forceinline__ void r16_forward_settle(int64_t (&v)[16],
+__device__ __forceinline__ void r16_forward_settle(R16Value<A> (&v)[16],
                                                    const R16Pass &s) {
-  if (A != kLazyLarge)
-    return;
+  if constexpr (A == kLazyLarge) {
 #pragma unroll
-  for (int m = 0; m < 16; m++)
-    v[m] = guard_u(v[m], s.q2);
+    for (int m = 0; m < 16; m++)
+      v[m] = guard_u(v[m], s.q2);
+  }
 }
 
 // LDS exchange buffer: a tile's sub-transforms in rows of 2^L points, padded
@@ -270,9 +300,10 @@ __device__ __forceinline__ void wave_lds_sync() {
 // Starts with a barrier so the previous use of the buffer has finished.
 // WAVE: the threads sharing c are consecutive (c = tid / T, T <= 16), hence
 // in one wavefront, and a wavefront barrier replaces the block's.
-template <int L, bool TO_COLS, bool WAVE = false>
-__device__ __forceinline__ void r16_exchange(int64_t (&v)[16], int64_t *lds,
+template <int L, bool TO_COLS, bool WAVE = false, class V>
+__device__ __forceinline__ void r16_exchange(V (&v)[16], int64_t *buffer,
                                              int c, int r) {
+  V *lds = reinterpret_cast<V *>(buffer);
   if (WAVE)
     wave_lds_sync();
   else
@@ -292,11 +323,14 @@ __device__ __forceinline__ void r16_exchange(int64_t (&v)[16], int64_t *lds,
 // r16_exchange through a buffer of 32-bit words, half the LDS of the 64-bit
 // exchange (so that twice as many blocks fit on a CU): the low words go
 // through first, then the high words, each between two barriers.
-template <int L, bool TO_COLS>
-__device__ __forceinline__ void r16_exchange_words(int64_t (&v)[16],
-                                                   uint32_t *lds, int c,
-                                                   int r) {
+template <int L, bool TO_COLS, class V>
+__device__ __forceinline__ void r16_exchange_words(V (&x)[16], uint32_t *lds,
+                                                   int c, int r) {
+  int64_t v[16];
   uint32_t lo[16];
+#pragma unroll
+  for (int m = 0; m < 16; m++)
+    v[m] = __builtin_bit_cast(int64_t, x[m]);
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < 16; m++)
@@ -313,9 +347,9 @@ __device__ __forceinline__ void r16_exchange_words(int64_t (&v)[16],
   __syncthreads();
 #pragma unroll
   for (int m = 0; m < 16; m++)
-    v[m] = int64_t(
-        (uint64_t(lds[r16_lds<L>(c, r16_point<L, TO_COLS>(r, m))]) << 32) |
-        lo[m]);
+    x[m] = __builtin_bit_cast(
+        V, (uint64_t(lds[r16_lds<L>(c, r16_point<L, TO_COLS>(r, m))]) << 32) |
+               lo[m]);
 }
 
 // One register-resident L-bit pass over one 4096-point tile of one limb:
@@ -335,8 +369,6 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
                                               const int64_t *pre, int post,
                                               bool last, const DeviceTables &t,
                                               int64_t *lds) {
-  const int log_n = t.log_n;
-  const int64_t n = int64_t(1) << log_n;
   const int tid = OPAQUE ? opaque_tid() : int(threadIdx.x);
   constexpr int T = 1 << (L - 4), C = 4096 >> L;
   const int c = COLS ? (tid & (C - 1)) : (tid >> (L - 4));
@@ -349,31 +381,47 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
   int64_t *dst = dst_limb + base;
 
   R16Pass s;
-  s.tw = (INV ? t.root_inverse : t.root) + int64_t(p) * n;
-  s.ts = (INV ? t.root_inverse_shoup : t.root_shoup) + int64_t(p) * n * 2;
-  s.n = n;
+  r16_prime<A, INV>(s, t, p);
   s.hi = hi;
-  s.log_n = log_n;
   s.b = b;
   s.r = r;
-  s.q = t.q[p];
-  s.k = t.k[p];
-  s.q2 = int64_t(t.q2[p]);
-  s.nq2 = A == kExact ? opaque_neg(s.q2) : 0;  // exact guards only
-  s.nq = A == kExact ? 0 : uint64_t(opaque_neg(int64_t(s.q)));
 
-  int64_t v[16];
+  R16Value<A> v[16];
   // load in the ownership of the first round; the contiguous inverse pass
   // loads coalesced ROWS and re-owns through LDS
   constexpr bool cols_load = INV && COLS;
+  constexpr bool first_pass = INV != COLS; // of the two in this direction
+  int64_t w[16];
 #pragma unroll
   for (int m = 0; m < 16; m++)
-    v[m] = src[int64_t(r16_point<L, cols_load>(r, m)) << b];
-  if (pre) {
-    const int64_t cst = pre[p];
+    w[m] = src[int64_t(r16_point<L, cols_load>(r, m)) << b];
+  if constexpr (A == kF64) {
+    if (first_pass) {
+      f64_load(w, v, s.f);
+      if (pre) {
+        // the Montgomery product with pre is one with pre R^-1
+        const double c = double(mont_exit(pre[p], s.q, s.k));
+#pragma unroll
+        for (int m = 0; m < 16; m++)
+          v[m] = f64_mul(v[m], c, s.f);
+      } else if (INV) {
+        // lazy residues in [0, 2q), centred
+#pragma unroll
+        for (int m = 0; m < 16; m++)
+          v[m] -= s.f.q;
+      }
+    } else {
+#pragma unroll
+      for (int m = 0; m < 16; m++) {
+        v[m] = __longlong_as_double(w[m]);
+        if (INV)
+          v[m] = f64_center(v[m], s.f);
+      }
+    }
+  } else {
 #pragma unroll
     for (int m = 0; m < 16; m++)
-      v[m] = load_product<A>(v[m], cst, s.q, s.k);
+      v[m] = pre ? load_product<A>(w[m], pre[p], s.q, s.k) : w[m];
   }
   if (INV && !COLS)
     r16_exchange<L, true, !COLS>(v, lds, c, r);
@@ -390,26 +438,38 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
     r16_inverse_low<L, A>(v, s);
     r16_exchange<L, false, !COLS>(v, lds, c, r);
     r16_inverse_high<L, A>(v, s);
-    if (post != kInttRaw) {
+    if constexpr (A == kF64) {
+      if (post != kInttRaw) {
+        // N^-1 and the exit of the Montgomery form in one product; the key
+        // products of kInttKeyReduce carry one more R
+        int64_t c = mont_exit(mont_exit(t.ninv[p], s.q, s.k), s.q, s.k);
+        if (post == kInttKeyReduce)
+          c = mont_exit(c, s.q, s.k);
+        const double cd = double(c);
+#pragma unroll
+        for (int m = 0; m < 16; m++)
+          v[m] = f64_canonical(f64_mul(v[m], cd, s.f), s.f);
+      }
+    } else if (post != kInttRaw) {
       const int64_t ninv = t.ninv[p];
-      if (A == kExact) {
+      const bool reduce = post != kInttExit;
+      if constexpr (A == kExact) {
 #pragma unroll
         for (int m = 0; m < 16; m++) {
           // only the exact arithmetic carries negative values
           const int64_t y =
               mont_exit(mont_mult_cs(ninv, v[m], s.q, s.k), s.q, s.k);
-          v[m] = post == kInttExitReduce ? guard(y, int64_t(s.q)) : y;
+          v[m] = reduce ? guard(y, int64_t(s.q)) : y;
         }
       } else {
-        // the lazy forms need only the residue: one product with
-        // N^-1 R^-1 (the exit folded into the constant) gives it below
-        // v q / 2^62 + q < 2q (v < 2^60 for kLazySmall, v < 2q for
-        // kLazyLarge), which the reduce brings to the canonical value
+        // kLazyLarge needs only the residue: one product with N^-1 R^-1
+        // (the exit folded into the constant) gives it below v q / 2^62 + q
+        // < 2q (v < 2q), which the reduce brings to the canonical value
         const int64_t ninv_exit = mont_exit(ninv, s.q, s.k);
 #pragma unroll
         for (int m = 0; m < 16; m++) {
           const int64_t y = mont_mult_u(v[m], ninv_exit, s.q, s.k);
-          v[m] = post == kInttExitReduce ? guard_u(y, int64_t(s.q)) : y;
+          v[m] = reduce ? guard_u(y, int64_t(s.q)) : y;
         }
       }
     }
@@ -417,8 +477,17 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
   // store: ROWS ownership except the strided forward pass (COLS)
   constexpr bool cols_store = !INV && COLS;
 #pragma unroll
-  for (int m = 0; m < 16; m++)
-    dst[int64_t(r16_point<L, cols_store>(r, m)) << b] = v[m];
+  for (int m = 0; m < 16; m++) {
+    int64_t y;
+    if constexpr (A != kF64)
+      y = v[m];
+    else if (first_pass)
+      y = __double_as_longlong(v[m]);
+    else
+      y = f64_to_int(INV && post != kInttRaw ? v[m]
+                                             : f64_floor_mod(v[m], s.f));
+    dst[int64_t(r16_point<L, cols_store>(r, m)) << b] = y;
+  }
 }
 
 } // namespace fhe

@@ -63,8 +63,10 @@ struct UnevenSchedule {
   int xcd = 1;
 };
 
-// Stage launchers (uneven_kernels.hip).  Arithmetic variants: 0 exact,
-// 1 lazy small-prime, 2 lazy large-prime forms (ntt_r16.h).
+// Stage launchers (uneven_kernels.hip).  Arithmetic variants: NttArith
+// (ntt_r16.h), and for the extension the kF64 form after signed digits.
+constexpr int kUnevenSignedF64 = 3;
+
 //
 // One 8-bit NTT pass over the listed limbs: unit (ct, poly, limb, tile) is
 // limb `limb` of polynomial `poly` at src.p[ct] + (poly * stride + limb) N,
@@ -86,8 +88,8 @@ void launch_uneven_digits(const DeviceTables &t, const UnevenCt *cts,
                           hipStream_t stream);
 
 // Extended limbs (ct, partition, limb, tile) from the digits with the first
-// forward NTT pass fused: ext.p[ct] receives [parts][ext][N].  variant 0 is
-// the exact extension with signed digits.
+// forward NTT pass fused: ext.p[ct] receives [parts][ext][N].  variant 0 and
+// kUnevenSignedF64 are the exact extension with signed digits.
 void launch_uneven_extend(const DeviceTables &t, const UnevenCt *cts,
                           const UnitList &list, const UnevenPtrs &digits,
                           const UnevenPtrs &ext, int maxz, int variant,

@@ -85,8 +85,7 @@ void uneven_plan_free(UnevenPlan *plan) {
 namespace {
 
 int lazy_variant(const fhe::CkksParams &P, int prime) {
-  return P.q[prime] < fhe::kLazySmallBound ? fhe::kLazySmall
-                                           : fhe::kLazyLarge;
+  return P.q[prime] < fhe::kF64Bound ? fhe::kF64 : fhe::kLazyLarge;
 }
 
 // Build (or find) the plan of a batch shape.
@@ -157,8 +156,8 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     int64_t key;
     uint32_t unit;
   };
-  auto emit = [&](int stage, std::vector<Keyed> (&by_variant)[3]) {
-    for (int v = 0; v < 3; v++) {
+  auto emit = [&](int stage, std::vector<Keyed> (&by_variant)[4]) {
+    for (int v = 0; v < 4; v++) {
       auto &list = by_variant[v];
       if (list.empty())
         continue;
@@ -177,7 +176,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
   if (relin) {
     // the trio's d2 exact (it feeds ModUp), d0 / d1 lazy
     for (int stage : {int(kStTrioIntt1), int(kStTrioIntt2)}) {
-      std::vector<Keyed> lists[3];
+      std::vector<Keyed> lists[4];
       for (int c = 0; c < count; c++) {
         const UnevenCt &u = plan->host[c];
         for (int poly = 0; poly < 3; poly++)
@@ -193,7 +192,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     }
   }
   {
-    std::vector<Keyed> lists[3];
+    std::vector<Keyed> lists[4];
     for (int c = 0; c < count; c++)
       for (int p = 0; p < plan->host[c].parts; p++)
         for (int ch = 0; ch < chunks; ch++)
@@ -201,7 +200,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     emit(kStDigits, lists);
   }
   {
-    std::vector<Keyed> lists[3];
+    std::vector<Keyed> lists[4];
     for (int c = 0; c < count; c++) {
       const UnevenCt &u = plan->host[c];
       for (int p = 0; p < u.parts; p++)
@@ -211,8 +210,11 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
           if (relin && i >= u.start[p] && i < u.start[p] + u.size[p])
             continue;
           const int prime = u.moduli_id + i;
-          const int v = ((u.signed_mask >> p) & 1) ? fhe::kExact
-                                                   : lazy_variant(P, prime);
+          // signed digits: the exact extension, before the arithmetic that
+          // the key product reads
+          int v = lazy_variant(P, prime);
+          if ((u.signed_mask >> p) & 1)
+            v = v == fhe::kF64 ? fhe::kUnevenSignedF64 : int(fhe::kExact);
           for (int t = 0; t < tiles; t++)
             lists[v].push_back({tile_key(prime, t),
                                 fhe::unit_pack(c, p, i, t)});
@@ -221,7 +223,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     emit(kStExtend, lists);
   }
   {
-    std::vector<Keyed> lists[3];
+    std::vector<Keyed> lists[4];
     for (int c = 0; c < count; c++) {
       const UnevenCt &u = plan->host[c];
       for (int i = 0; i < u.ext; i++) {
@@ -234,7 +236,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     emit(kStKs, lists);
   }
   {
-    std::vector<Keyed> lists[3];
+    std::vector<Keyed> lists[4];
     for (int c = 0; c < count; c++) {
       const UnevenCt &u = plan->host[c];
       for (int h = 0; h < 2; h++)
@@ -248,7 +250,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     emit(kStAccIntt2, lists);
   }
   {
-    std::vector<Keyed> lists[3];
+    std::vector<Keyed> lists[4];
     for (int c = 0; c < count; c++)
       for (int h = 0; h < 2; h++)
         for (int ch = 0; ch < chunks; ch++)
@@ -256,7 +258,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     emit(kStModDown, lists);
   }
   if (!relin) {
-    std::vector<Keyed> lists[3];
+    std::vector<Keyed> lists[4];
     const int aut_chunks = int(P.n / (4 * fhe::kBlock));
     for (int c = 0; c < count; c++)
       for (int poly = 0; poly < 2; poly++)
@@ -343,7 +345,7 @@ void uneven_run(fhe_context *ctx, UnevenPlan *plan, const int64_t *const *src,
         break;
       case kStAccIntt2:
         fhe::launch_uneven_ntt(t, plan->dev, list, acc, acc, 1, true, 8,
-                               nullptr, fhe::kInttExitReduce, true, L.variant,
+                               nullptr, fhe::kInttKeyReduce, true, L.variant,
                                s.cap, ctx->stream);
         break;
       case kStModDown:

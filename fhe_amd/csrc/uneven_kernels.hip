@@ -116,7 +116,7 @@ struct UnevenExtArgs {
 template <int A, int MAXZ, bool SIGNED>
 __global__ __launch_bounds__(kBlock) void uneven_extend_kernel(
     UnevenExtArgs a, DeviceTables t) {
-  __shared__ uint32_t lds[kR16Lds<8>];
+  __shared__ __align__(8) uint32_t lds[kExtendLds<16, A>];
   for (UnitWalk u(a.list); u.w < u.end; u.w += u.step) {
     const uint32_t unit = a.list.units[u.w];
     const int c = unit_ct(unit), part = unit_a(unit);
@@ -126,6 +126,7 @@ __global__ __launch_bounds__(kBlock) void uneven_extend_kernel(
     it.cst = ct.cst + int64_t(part) * ct.cst_stride;
     it.ext = const_cast<int64_t *>(a.ext.p[c]) +
              (int64_t(part) * ct.ext << t.log_n);
+    it.start = ct.start[part];
     it.size = ct.size[part];
     it.ext_limbs = ct.ext;
     it.moduli_id = ct.moduli_id;
@@ -289,8 +290,8 @@ void launch_uneven_ntt(const DeviceTables &t, const UnevenCt *cts,
   do {                                                                         \
     if (variant == kExact)                                                     \
       FHE_UNTT(I, C, kExact);                                                  \
-    else if (variant == kLazySmall)                                            \
-      FHE_UNTT(I, C, kLazySmall);                                              \
+    else if (variant == kF64)                                            \
+      FHE_UNTT(I, C, kF64);                                              \
     else                                                                       \
       FHE_UNTT(I, C, kLazyLarge);                                              \
   } while (0)
@@ -348,8 +349,10 @@ void launch_uneven_extend(const DeviceTables &t, const UnevenCt *cts,
   do {                                                                         \
     if (variant == kExact)                                                     \
       FHE_UEXT(kExact, W, true);                                               \
-    else if (variant == kLazySmall)                                            \
-      FHE_UEXT(kLazySmall, W, false);                                          \
+    else if (variant == kF64)                                            \
+      FHE_UEXT(kF64, W, false);                                          \
+    else if (variant == kUnevenSignedF64)                                      \
+      FHE_UEXT(kF64, W, true);                                                 \
     else                                                                       \
       FHE_UEXT(kLazyLarge, W, false);                                          \
   } while (0)
@@ -382,8 +385,8 @@ void launch_uneven_ks(const DeviceTables &t, const UnevenCt *cts,
   if (variant == kExact)
     hipLaunchKernelGGL(uneven_ks_kernel<kExact>, grid, dim3(kBlock), 0,
                        stream, a, t);
-  else if (variant == kLazySmall)
-    hipLaunchKernelGGL(uneven_ks_kernel<kLazySmall>, grid, dim3(kBlock), 0,
+  else if (variant == kF64)
+    hipLaunchKernelGGL(uneven_ks_kernel<kF64>, grid, dim3(kBlock), 0,
                        stream, a, t);
   else
     hipLaunchKernelGGL(uneven_ks_kernel<kLazyLarge>, grid, dim3(kBlock), 0,

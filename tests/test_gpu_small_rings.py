@@ -79,3 +79,31 @@ def test_noalloc_splits_batches(gpu_lib):
         assert np.array_equal(want.download(), got.download())
         for arr in (da, dk, want, got):
             arr.free()
+
+
+@pytest.mark.parametrize("log_n,alpha,limbs", [(13, 1, 3), (16, 4, 6)])
+def test_wild_representatives(gpu_lib, log_n, alpha, limbs):
+    """Inputs that are other representatives of their residues, up to 2^61 in
+    magnitude (the load of the double-held transforms and of the first
+    digits): polynomial 0 of the factors of a product, and a rotation."""
+    primes = fhe_amd.resolve_primes(log_n, alpha)
+    rng = np.random.Generator(np.random.PCG64(9))
+    orc = Oracle(log_n, primes, alpha)
+    with fhe_amd.Context(log_n, alpha) as ctx:
+        n, mid, key_mid = ctx.n, ctx.chain_count - limbs, ctx.key_moduli_id()
+        a = uniform(rng, primes, mid, (1, 2, limbs, n))
+        b = uniform(rng, primes, mid, (1, 2, limbs, n))
+        key = uniform(rng, primes, key_mid, ctx.key_shape(key_mid), 2)
+        wild = a.copy()
+        for l in range(limbs):
+            q = int(primes[mid + l])
+            if q < 1 << 42:
+                most = (1 << 61) // q
+                wild[0, 0, l] += q * rng.integers(-most, most, n)
+        da, db, dk = (ctx.to_device(x) for x in (wild, b, key))
+        out = ctx.array((1, 2, limbs - 1, n))
+        ctx.hmult_relin_rescale(da, db, dk, key_mid, out, mid)
+        got = out.download()
+        for arr in (da, db, dk, out):
+            arr.free()
+    assert np.array_equal(got[0], orc.hmult(a[0], b[0], key, mid, key_mid))
