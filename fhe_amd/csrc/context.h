@@ -125,15 +125,7 @@ struct fhe_context {
   bool staged_modup = true;
   // each partition's own extended limbs from the NTT-form d2 when at hand
   bool own_limbs = true;
-  // the coefficient forms of d0 and d1 on a second stream, concurrent with
-  // the key switching of d2 (a second stream and two events, default
-  // priority)
-  // (1: forked once the trio is written; 2: once d2's INTT is done, so
-  // that the side stream runs beside the key inner product)
-  int overlap_trio = 1;
-  hipStream_t side = nullptr;
-  hipEvent_t fork_event = nullptr, join_event = nullptr;
-  // small-prime key products accumulated without guards, reduced once
+  // large-prime key products kept below 2q with one guard
   bool ks_lazy_accumulate = true;
   // second growable device buffer (Garner digits of the staged ModUp)
   void *aux = nullptr;
@@ -200,12 +192,6 @@ struct fhe_context {
     hip_check(hipGetDevice(&device), "hipGetDevice");
     hip_check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking),
               "stream creation");
-    hip_check(hipStreamCreateWithFlags(&side, hipStreamNonBlocking),
-              "stream creation");
-    hip_check(hipEventCreateWithFlags(&fork_event, hipEventDisableTiming),
-              "event creation");
-    hip_check(hipEventCreateWithFlags(&join_event, hipEventDisableTiming),
-              "event creation");
     auto &t = tables;
     t.q = upload(params.q, owned);
     t.k = upload(params.k, owned);
@@ -240,7 +226,6 @@ struct fhe_context {
     t.q_top = upload(params.q_top, owned);
     t.rescale = upload(params.rescale_scale, owned);
     t.host_q = params.q.data();
-    t.split_variants = 1;
     t.prime_count = params.prime_count;
     t.log_n = params.log_n;
     t.alpha = params.alpha;
@@ -250,8 +235,6 @@ struct fhe_context {
   ~fhe_context() {
     if (stream)
       (void)hipStreamSynchronize(stream);
-    if (side)
-      (void)hipStreamSynchronize(side);
     for (auto &st : pending) {
       (void)hipEventDestroy(st.start);
       (void)hipEventDestroy(st.stop);
@@ -272,12 +255,6 @@ struct fhe_context {
       (void)hipFree(aux);
     if (stash_buf)
       (void)hipFree(stash_buf);
-    if (side)
-      (void)hipStreamDestroy(side);
-    if (fork_event)
-      (void)hipEventDestroy(fork_event);
-    if (join_event)
-      (void)hipEventDestroy(join_event);
     if (stream)
       (void)hipStreamDestroy(stream);
   }
@@ -335,6 +312,10 @@ struct fhe_context {
     return fused_key_switch && params.partition_count(moduli_id) *
                                        (params.limbs_at(moduli_id) +
                                         params.alpha) <= kMaxExtLimbs;
+  }
+  // lazy arithmetic of whole transforms: the radix-16 sizes
+  bool lazy_transforms() const {
+    return lazy_key_switch && fhe::ks_fused_supported(tables);
   }
   // extended polynomials held at once by key switching: every partition on
   // the fused path, one at a time otherwise
@@ -638,11 +619,19 @@ struct fhe_context {
     const int64_t acc_l = int64_t(count) * 2 * ext_limbs;
     int64_t *ws = scratch(size_t(trio_l + ext_l + acc_l) * N * 8);
     int64_t *trio = ws, *ext = trio + trio_l * N, *acc = ext + ext_l * N;
-    const fhe::LazySpec d01 =
-        lazy_key_switch ? fhe::LazySpec{3, 2} : fhe::LazySpec();
+    const int64_t poly = int64_t(limbs) * N;
+    // d0 and d1 are canonicalized by the relinearization add; d2 feeds the
+    // representative-sensitive ModUp (the flags are in the accumulators,
+    // written after them)
+    fhe::LazySpec lazy{lazy_transforms(), reinterpret_cast<uint32_t *>(acc),
+                       3};
     stage("intt(trio)", [&] {
       fhe::ntt_inverse(tables, trios, trio, trio_l, limbs, moduli_id,
-                       fhe::kInttExit, stream, d01);
+                       fhe::kInttExit, stream, lazy);
+      if (lazy.on)
+        fhe::launch_repair_intt(tables, lazy.zero, trios + 2 * poly, 3 * poly,
+                                trio + 2 * poly, 3 * poly, count, limbs,
+                                moduli_id, stream);
     });
     // the caller's NTT-form d2 provides the partitions' own extended limbs
     key_switch(count, moduli_id, key, key_moduli_id, trio + 2 * limbs * N,
@@ -773,8 +762,7 @@ struct fhe_context {
     const int64_t *cst = modup_constants(moduli_id, key_moduli_id);
     const int stride = params.ks_stride(moduli_id);
     const int np = int(parts.size());
-    const fhe::LazySpec lazy = lazy_key_switch ? fhe::kAllLazy
-                                               : fhe::LazySpec();
+    const fhe::LazySpec lazy{lazy_key_switch};
     int max_size = 0;
     bool is_signed[fhe::kMaxFusedParts] = {};
     std::vector<int> starts(np), sizes(np);
@@ -831,8 +819,7 @@ struct fhe_context {
     const int key_offset = params.limbs_at(key_moduli_id) - limbs;
     const auto parts = params.partitions(moduli_id, key_moduli_id);
     const int np = int(parts.size());
-    const fhe::LazySpec lazy = lazy_key_switch ? fhe::kAllLazy
-                                               : fhe::LazySpec();
+    const fhe::LazySpec lazy{lazy_key_switch};
     std::vector<int> starts(np), sizes(np);
     for (int p = 0; p < np; p++) {
       starts[p] = parts[p].start;

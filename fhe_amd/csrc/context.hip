@@ -168,17 +168,14 @@ int fhe_context_set_option(fhe_context *ctx, const char *name, int value) {
       ctx->staged_modup = value != 0;
     else if (n == "own_limbs")
       ctx->own_limbs = value != 0;
-    else if (n == "overlap_trio")
-      ctx->overlap_trio = value < 0 ? 0 : value > 2 ? 2 : value;
     else if (n == "ks_lazy_accumulate")
       ctx->ks_lazy_accumulate = value != 0;
-    else if (n == "split_variants")
-      ctx->tables.split_variants = value != 0 ? 1 : 0;
     else
       // names of pipelines that the defaults have replaced: no effect
       require(n == "fuse_modup" || n == "fuse_tensor" ||
                   n == "ks_occupancy" || n == "ks_prefetch" ||
-                  n == "ks_wide_accumulate",
+                  n == "ks_wide_accumulate" || n == "overlap_trio" ||
+                  n == "split_variants",
               "unknown option " + n);
   });
 }
@@ -357,78 +354,38 @@ void hmult_relin_rescale_into(fhe_context *ctx, int count, int moduli_id,
     int64_t *an = ws, *bn = an + duo_l * N, *trio = bn + duo_l * N;
     int64_t *trio_c = trio + trio_l * N;
     int64_t *ext = trio_c + trio_l * N, *acc = ext + ext_l * N;
-    // prepare_for_multiply: to NTT form (src/ckks/engine_multiply.cpp:13-27)
-    // Only a1 * b1 reaches the representative-sensitive ModUp (through the
-    // exact INTT of d2), so the transforms of a0 and b0 may be lazy.
-    const fhe::LazySpec first_poly =
-        ctx->lazy_key_switch ? fhe::LazySpec{2, 1} : fhe::LazySpec();
-    // relinearize: to_intt of all three, key switch of the third; d0 and d1
-    // are canonicalized by the relinearization add, d2 feeds ModUp exactly
-    const fhe::LazySpec d01 =
-        ctx->lazy_key_switch ? fhe::LazySpec{3, 2} : fhe::LazySpec();
-    const bool overlap =
-        ctx->overlap_trio && ctx->lazy_key_switch &&
-        fhe::ntt_parts_supported(ctx->tables);
-    // once the side stream has forked, every exit (an exception included)
-    // makes the main stream wait for it, so later work on the workspace is
-    // ordered after the side-stream INTT
-    bool joined = true;
-    struct Join {
-      fhe_context *ctx;
-      bool &joined;
-      ~Join() {
-        if (!joined)
-          (void)hipStreamWaitEvent(ctx->stream, ctx->join_event, 0);
-      }
-    } join_guard{ctx, joined};
+    // prepare_for_multiply: to NTT form (src/ckks/engine_multiply.cpp:13-27).
+    // Lazy throughout: d0 and d1 are canonicalized by the relinearization
+    // add, and d2's inverse feeds the representative-sensitive ModUp
+    // canonical, but for limbs with a zero residue, which are recomputed
+    // (the flags are in the accumulators, written after them)
+    const int64_t poly = int64_t(limbs) * N;
+    const fhe::LazySpec lazy{ctx->lazy_transforms()};
+    fhe::LazySpec flagged = lazy;
+    flagged.zero = reinterpret_cast<uint32_t *>(acc);
+    flagged.zero_period = 3;
     ctx->stage("ntt(inputs)", [&] {
       fhe::ntt_forward(ctx->tables, a, an, duo_l, limbs, moduli_id,
-                       ctx->tables.r2, ctx->stream, first_poly);
+                       ctx->tables.r2, ctx->stream, lazy);
       fhe::ntt_forward(ctx->tables, b, bn, duo_l, limbs, moduli_id,
-                       ctx->tables.r2, ctx->stream, first_poly);
+                       ctx->tables.r2, ctx->stream, lazy);
     });
     ctx->stage("tensor", [&] {
       fhe::launch_tensor(ctx->tables, an, bn, trio, count, limbs, moduli_id,
                          ctx->stream);
     });
-    if (overlap) {
-      // d0, d1 (lazy) on the side stream, forked once the trio is written
-      // (overlap_trio 1) or once d2's INTT is done (2, alongside the key
-      // switching of d2); d2 (exact, feeds ModUp) here
-      fhe::LazySpec lazy_part = d01, exact_part = d01;
-      lazy_part.part = 2;
-      exact_part.part = 1;
-      auto fork = [&] {
-        hip_check(hipEventRecord(ctx->fork_event, ctx->stream), "event");
-        hip_check(hipStreamWaitEvent(ctx->side, ctx->fork_event, 0),
-                  "event");
-        fhe::ntt_inverse(ctx->tables, trio, trio_c, trio_l, limbs,
-                         moduli_id, fhe::kInttExit, ctx->side, lazy_part);
-        hip_check(hipEventRecord(ctx->join_event, ctx->side), "event");
-        joined = false;
-      };
-      if (ctx->overlap_trio == 1)
-        fork();
-      ctx->stage("intt(trio)", [&] {
-        fhe::ntt_inverse(ctx->tables, trio, trio_c, trio_l, limbs,
-                         moduli_id, fhe::kInttExit, ctx->stream,
-                         exact_part);
-      });
-      if (ctx->overlap_trio != 1)
-        fork();
-    } else {
-      ctx->stage("intt(trio)", [&] {
-        fhe::ntt_inverse(ctx->tables, trio, trio_c, trio_l, limbs,
-                         moduli_id, fhe::kInttExit, ctx->stream, d01);
-      });
-    }
+    // relinearize: to_intt of all three, key switch of the third
+    ctx->stage("intt(trio)", [&] {
+      fhe::ntt_inverse(ctx->tables, trio, trio_c, trio_l, limbs, moduli_id,
+                       fhe::kInttExit, ctx->stream, flagged);
+      if (flagged.on)
+        fhe::launch_repair_product(ctx->tables, flagged.zero, a, false, b,
+                                   false, an, trio_c + 2 * poly, 3 * poly,
+                                   count, limbs, moduli_id, ctx->stream);
+    });
     ctx->key_switch(count, moduli_id, key, key_moduli_id,
                     trio_c + 2 * limbs * N, 3 * limbs * N, ext, acc,
                     trio + 2 * limbs * N, 3 * limbs * N, false, digits);
-    if (overlap) {
-      joined = true;
-      hip_check(hipStreamWaitEvent(ctx->stream, ctx->join_event, 0), "event");
-    }
     ctx->stage("moddown_relin_rescale", [&] {
       fhe::launch_moddown_relin_rescale(ctx->tables, acc, trio_c, out, count,
                                         limbs, moduli_id, ctx->stream);

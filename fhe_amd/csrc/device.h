@@ -37,9 +37,6 @@ struct DeviceTables {
   // HOST copy of the primes (for launch decisions on the host; kernels
   // never read it)
   const uint64_t *host_q;
-  // launch choice (host): one launch per arithmetic variant instead of a
-  // per-block choice inside one kernel
-  int split_variants;
   int prime_count;
   int log_n;
   int alpha;

@@ -7,24 +7,38 @@
 
 namespace fhe {
 
-// Which polynomials of a batched transform may use the lazy arithmetic
-// (ntt_r16.h): those whose index modulo `period` is below `count`.  Lazy
-// outputs are other representatives of the same residues: forward outputs
-// below 2q, or below 2^48 for primes under 2^42; inverse outputs with the
-// exit below 2q (canonical with kInttExitReduce).  The default is exact
-// everywhere.
+// Whether a batched transform may use the lazy arithmetic (ntt_r16.h; the
+// radix-16 sizes): its outputs are other representatives of the same
+// residues, forward outputs below 2q, inverse outputs with the exit
+// canonical.
+//
+// The exact inverse with the exit (kInttExit) is canonical too but for zero
+// residues, whose representative, 0 or q, depends on the exact values before:
+// y = mont(N^-1 R, v) lies in (-q, 2q) and the exit returns the
+// representative in [y / 2^62, y / 2^62 + q), canonical for y != 0 mod q.
+// Where the representative matters, `zero` names a flag word per
+// (polynomial, limb) of the polynomials whose index modulo zero_period is
+// zero_period - 1; the transform clears them and sets those of limbs with a
+// zero residue, which launch_repair_* then recompute exactly.
 struct LazySpec {
-  int period = 0;
-  int count = 0;
-  // 0: every polynomial; 1: only the exact ones; 2: only the lazy ones
-  // (split per-variant launches of the radix-16 passes only)
-  int part = 0;
+  bool on = false;
+  uint32_t *zero = nullptr;
+  int zero_period = 1;
 };
-constexpr LazySpec kAllLazy{1, 1};
 
-// Whether LazySpec::part may select a subset of the polynomials: the
-// radix-16 passes with per-variant launches.
-bool ntt_parts_supported(const DeviceTables &t);
+// Exact recomputation of the flagged limbs [count][limbs]: out = the exact
+// inverse with the exit of the NTT-form polynomial z, or of the product of
+// polynomials 1 of the duos x and y [count][2][limbs][N] (INTT form, or NTT
+// form with x_ntt / y_ntt; scratch: [2][count][limbs][N]).
+void launch_repair_intt(const DeviceTables &t, const uint32_t *zero,
+                        const int64_t *z, int64_t z_stride, int64_t *out,
+                        int64_t out_stride, int count, int limbs,
+                        int moduli_id, hipStream_t stream);
+void launch_repair_product(const DeviceTables &t, const uint32_t *zero,
+                           const int64_t *x, bool x_ntt, const int64_t *y,
+                           bool y_ntt, int64_t *scratch, int64_t *out,
+                           int64_t out_stride, int count, int limbs,
+                           int moduli_id, hipStream_t stream);
 
 // In-place capable forward NTT of total_limbs limbs.  pre (device, indexed by
 // absolute prime) multiplies each input value in Montgomery form first, e.g.

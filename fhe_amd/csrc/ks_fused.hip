@@ -249,23 +249,6 @@ __global__ __launch_bounds__(kBlock) void extend_ntt_mixed_kernel(
   });
 }
 
-// Calls f with log2 N as a compile-time constant.
-template <class F> void with_log_n(int log_n, F &&f) {
-  switch (log_n) {
-  case 13:
-    f(std::integral_constant<int, 13>());
-    break;
-  case 14:
-    f(std::integral_constant<int, 14>());
-    break;
-  case 15:
-    f(std::integral_constant<int, 15>());
-    break;
-  default:
-    f(std::integral_constant<int, 16>());
-  }
-}
-
 // Calls f(first limb, limbs, small) for each run of extended limbs of one
 // prime class.
 template <class F>

@@ -37,9 +37,9 @@ struct PassArgs {
   const int64_t *pre; // forward first pass: multiply by pre[prime] on load
   int post;           // inverse last pass: InttPost
   int last;           // the pass completes the transform
-  int lazy_period;    // lazy arithmetic for polynomial index % period <
-  int lazy_count;     //   count (radix-16 passes only; 0: all exact)
-  int lazy_part = 0;  // LazySpec::part
+  bool lazy;          // lazy arithmetic (radix-16 passes only)
+  uint32_t *zero;     // LazySpec::zero
+  int zero_period;
 };
 
 template <bool INV>
@@ -142,56 +142,17 @@ __global__ __launch_bounds__(kBlock) void ntt_pass_kernel(PassArgs a,
   }
 }
 
-// Register-resident L-bit pass (r16_limb_pass, ntt_r16.h) on limb l of
-// polynomial `poly` of the batch.
-template <int L, bool INV, bool COLS, int A>
-__device__ __forceinline__ void r16_pass(const PassArgs &a,
-                                         const DeviceTables &t, int64_t *lds,
-                                         int64_t poly, int tile, int l) {
-  const int64_t limb = (poly * a.limbs + l) << t.log_n;
-  r16_limb_pass<L, INV, COLS, A>(a.src + limb, a.dst + limb, a.moduli_id + l,
-                              tile, a.low_bit, a.pre, a.post, a.last != 0, t,
-                              lds);
-}
-
-// Register-resident pass kernel with one arithmetic A per launch (a single
-// code path per kernel keeps the instruction footprint and the register
-// allocation to that path).  The launch covers the polynomials
-// poly = (j / sel_count) * sel_period + sel_offset + j % sel_count,
-// j < sel_polys, and the limbs l0 .. l0 + limbs_in_launch - 1.
-struct PolySelect {
-  int polys;   // selected polynomials
-  int period, count, offset;
-  int l0;      // first limb of the launch
-};
-
-template <int L, bool INV, bool COLS, int A>
+// A register-resident L-bit pass (r16_limb_pass, ntt_r16.h) over every limb
+// of the batch, exact or lazy with the arithmetic of each limb's prime class
+// chosen per block: one launch for the batch (the two lazy forms take about
+// the same registers, and a launch for the few large primes of a chain alone
+// would run its chain of butterflies on a nearly empty chip).
+//
+// Block -> (limb l, tile, polynomial), polynomial fastest so blocks sharing
+// a prime's twiddles run together; with swizzle each of the 8 XCDs (blocks
+// are dealt round-robin to XCDs) gets one contiguous range of that order.
+template <int L, bool INV, bool COLS, bool LAZY>
 __global__ __launch_bounds__(kBlock) void ntt_radix16_kernel(
-    PassArgs a, DeviceTables t, PolySelect sel, int tiles_per_limb,
-    int swizzle) {
-  __shared__ int64_t lds[kR16Lds<L>];
-  // block -> (limb l, tile, polynomial), polynomial fastest so blocks sharing
-  // a prime's twiddles run together; with swizzle each of the 8 XCDs (blocks
-  // are dealt round-robin to XCDs) gets one contiguous range of that order.
-  int64_t w = blockIdx.x;
-  if (swizzle) {
-    const int64_t per = int64_t(gridDim.x) >> 3;
-    w = int64_t(blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  }
-  const int64_t j = w % sel.polys;
-  const int64_t rest = w / sel.polys;
-  const int tile = int(rest % tiles_per_limb);
-  const int l = sel.l0 + int(rest / tiles_per_limb);
-  const int64_t poly =
-      (j / sel.count) * sel.period + sel.offset + (j % sel.count);
-  r16_pass<L, INV, COLS, A>(a, t, lds, poly, tile, l);
-}
-
-// The same pass with the arithmetic chosen per block: polynomials whose index
-// modulo a.lazy_period is below a.lazy_count take the lazy arithmetic of
-// their prime's size class, the others the exact one (one launch for all).
-template <int L, bool INV, bool COLS>
-__global__ __launch_bounds__(kBlock) void ntt_radix16_mixed_kernel(
     PassArgs a, DeviceTables t, int polys, int tiles_per_limb, int swizzle) {
   __shared__ int64_t lds[kR16Lds<L>];
   int64_t w = blockIdx.x;
@@ -203,13 +164,27 @@ __global__ __launch_bounds__(kBlock) void ntt_radix16_mixed_kernel(
   const int64_t rest = w / polys;
   const int tile = int(rest % tiles_per_limb);
   const int l = int(rest / tiles_per_limb);
-  const bool lazy = a.lazy_period > 0 && (poly % a.lazy_period) < a.lazy_count;
-  if (!lazy)
-    r16_pass<L, INV, COLS, kExact>(a, t, lds, poly, tile, l);
-  else if (r16_supported(t.log_n) && t.q[a.moduli_id + l] < kF64Bound)
-    r16_pass<L, INV, COLS, kF64>(a, t, lds, poly, tile, l);
-  else
-    r16_pass<L, INV, COLS, kLazyLarge>(a, t, lds, poly, tile, l);
+  const int64_t limb = (poly * a.limbs + l) << t.log_n;
+  const int64_t *src = a.src + limb;
+  int64_t *dst = a.dst + limb;
+  const int p = a.moduli_id + l;
+  if constexpr (!LAZY) {
+    r16_limb_pass<L, INV, COLS, kExact>(src, dst, p, tile, a.low_bit, a.pre,
+                                        a.post, a.last != 0, t, lds);
+  } else {
+    uint32_t *zero =
+        a.zero && poly % a.zero_period == a.zero_period - 1
+            ? a.zero + (poly / a.zero_period) * a.limbs + l
+            : nullptr;
+    // (the generic second pass of N = 2^17 takes no doubles)
+    if (r16_supported(t.log_n) && t.q[p] < kF64Bound)
+      r16_limb_pass<L, INV, COLS, kF64>(src, dst, p, tile, a.low_bit, a.pre,
+                                        a.post, a.last != 0, t, lds, zero);
+    else
+      r16_limb_pass<L, INV, COLS, kLazyLarge>(src, dst, p, tile, a.low_bit,
+                                              a.pre, a.post, a.last != 0, t,
+                                              lds, zero);
+  }
 }
 
 // Split log_n into the bit ranges of at most two passes (each <= 12 bits),
@@ -237,60 +212,16 @@ void launch_r16_pass(const PassArgs &a, const DeviceTables &t,
   const int64_t total_limbs = a.total_subs >> (t.log_n - L);
   const int polys = int(total_limbs / a.limbs);
   const int tiles = int(int64_t(1) << (t.log_n - 12));
-  if (!t.split_variants) {
-    const int64_t blocks = total_limbs * tiles;
-    hipLaunchKernelGGL((ntt_radix16_mixed_kernel<L, INV, COLS>),
+  const int64_t blocks = total_limbs * tiles;
+  const int swizzle = blocks % 8 == 0 ? 1 : 0;
+  if (a.lazy)
+    hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, true>),
                        dim3(unsigned(blocks)), dim3(kBlock), 0, stream, a, t,
-                       polys, tiles, blocks % 8 == 0 ? 1 : 0);
-    return;
-  }
-  auto launch = [&](int arith, PolySelect sel, int limbs_in_launch) {
-    const int64_t blocks = int64_t(sel.polys) * tiles * limbs_in_launch;
-    if (blocks == 0)
-      return;
-    const dim3 grid{unsigned(blocks), 1, 1};
-    const int swizzle = blocks % 8 == 0 ? 1 : 0;
-    if (arith == kExact)
-      hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, kExact>), grid,
-                         dim3(kBlock), 0, stream, a, t, sel, tiles, swizzle);
-    else if (arith == kF64)
-      hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, kF64>), grid,
-                         dim3(kBlock), 0, stream, a, t, sel, tiles, swizzle);
-    else
-      hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, kLazyLarge>), grid,
-                         dim3(kBlock), 0, stream, a, t, sel, tiles, swizzle);
-  };
-  const int period = a.lazy_period > 0 ? a.lazy_period : 1;
-  const int lazy_count = a.lazy_period > 0 ? a.lazy_count : 0;
-  // polynomials in whole periods (every caller passes whole periods)
-  if (polys % period != 0)
-    throw std::invalid_argument(
-        "NTT: the polynomial count is not a whole number of lazy periods");
-  const int periods = polys / period;
-  // exact polynomials: all limbs in one launch
-  if (lazy_count < period && a.lazy_part != 2)
-    launch(kExact,
-           PolySelect{periods * (period - lazy_count), period,
-                      period - lazy_count, lazy_count, 0},
-           a.limbs);
-  // lazy polynomials: one launch per run of limbs of one prime class
-  if (lazy_count > 0 && a.lazy_part != 1) {
-    int l = 0;
-    while (l < a.limbs) {
-      // (the generic second pass of N = 2^17 takes no doubles)
-      auto is_small = [&](int limb) {
-        return r16_supported(t.log_n) && t_host_q_small(t, a.moduli_id + limb);
-      };
-      const bool small = is_small(l);
-      int e = l + 1;
-      while (e < a.limbs && is_small(e) == small)
-        e++;
-      launch(small ? kF64 : kLazyLarge,
-             PolySelect{periods * lazy_count, period, lazy_count, 0, l},
-             e - l);
-      l = e;
-    }
-  }
+                       polys, tiles, swizzle);
+  else
+    hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, false>),
+                       dim3(unsigned(blocks)), dim3(kBlock), 0, stream, a, t,
+                       polys, tiles, swizzle);
 }
 
 template <bool INV>
@@ -323,10 +254,6 @@ void launch_pass(const PassArgs &a, const DeviceTables &t,
 
 } // namespace
 
-bool ntt_parts_supported(const DeviceTables &t) {
-  return t.split_variants && r16_supported(t.log_n);
-}
-
 void ntt_forward(const DeviceTables &t, const int64_t *src, int64_t *dst,
                  int64_t total_limbs, int limbs, int moduli_id,
                  const int64_t *pre, hipStream_t stream, LazySpec lazy) {
@@ -336,13 +263,13 @@ void ntt_forward(const DeviceTables &t, const int64_t *src, int64_t *dst,
   PassArgs a{src,     dst,      total_limbs << (t.log_n - l1),
              limbs,   moduli_id, t.log_n - l1,
              l1,      pre,       kInttRaw,
-             l2 == 0, lazy.period, lazy.count, lazy.part};
+             l2 == 0, lazy.on, lazy.zero, lazy.zero_period};
   launch_pass<false>(a, t, stream);
   if (l2 > 0) {
     PassArgs b2{dst,   dst,      total_limbs << (t.log_n - l2),
                 limbs, moduli_id, 0,
                 l2,    nullptr,   kInttRaw,
-                1,     lazy.period, lazy.count, lazy.part};
+                1,     lazy.on, lazy.zero, lazy.zero_period};
     launch_pass<false>(b2, t, stream);
   }
 }
@@ -356,13 +283,13 @@ void ntt_inverse(const DeviceTables &t, const int64_t *src, int64_t *dst,
   PassArgs a{src,     dst,      total_limbs << (t.log_n - l1),
              limbs,   moduli_id, 0,
              l1,      nullptr,   l2 > 0 ? int(kInttRaw) : post,
-             l2 == 0, lazy.period, lazy.count, lazy.part};
+             l2 == 0, lazy.on, lazy.zero, lazy.zero_period};
   launch_pass<true>(a, t, stream);
   if (l2 > 0) {
     PassArgs b2{dst,   dst,      total_limbs << (t.log_n - l2),
                 limbs, moduli_id, l1,
                 l2,    nullptr,   post,
-                1,     lazy.period, lazy.count, lazy.part};
+                1,     lazy.on, lazy.zero, lazy.zero_period};
     launch_pass<true>(b2, t, stream);
   }
 }
@@ -376,7 +303,7 @@ void ntt_forward_first(const DeviceTables &t, const int64_t *src, int64_t *dst,
   PassArgs a{src,     dst,      total_limbs << (t.log_n - l1),
              limbs,   moduli_id, t.log_n - l1,
              l1,      pre,       kInttRaw,
-             l2 == 0, lazy.period, lazy.count, lazy.part};
+             l2 == 0, lazy.on, lazy.zero, lazy.zero_period};
   launch_pass<false>(a, t, stream);
 }
 
@@ -395,7 +322,7 @@ void ntt_forward_second(const DeviceTables &t, const int64_t *src,
   PassArgs b2{src,   dst,      total_limbs << (t.log_n - l2),
               limbs, moduli_id, 0,
               l2,    nullptr,   kInttRaw,
-              1,     lazy.period, lazy.count, lazy.part};
+              1,     lazy.on, lazy.zero, lazy.zero_period};
   launch_pass<false>(b2, t, stream);
 }
 
@@ -408,8 +335,146 @@ void ntt_inverse_second(const DeviceTables &t, const int64_t *src,
   PassArgs a{src,   dst,      total_limbs << (t.log_n - l2),
              limbs, moduli_id, l1,
              l2,    nullptr,   post,
-             1,     lazy.period, lazy.count, lazy.part};
+             1,     lazy.on, lazy.zero, lazy.zero_period};
   launch_pass<true>(a, t, stream);
+}
+
+namespace {
+
+// Recomputation of flagged limbs with the reference's exact arithmetic: one
+// block per (ciphertext, limb), which leaves at once where the flag is clear
+// (the rule: a zero residue comes up once in 2^40 coefficients).  The block
+// walks the limb's tiles pass by pass; its own stores of one pass are what
+// it reads in the next, behind a block barrier.  bound: latency of the
+// launch, 3 us; a flagged limb takes about 0.2 ms.
+struct RepairArgs {
+  const uint32_t *zero; // [count][limbs]
+  // the NTT-form source polynomial of ciphertext c at z + c * z_stride, or,
+  // where a is set, the product of the transforms of a and b (polynomial 1
+  // of INTT-form duos, or NTT-form ones), formed in the scratch limbs
+  const int64_t *z;
+  int64_t z_stride;
+  const int64_t *a, *b;
+  int a_ntt, b_ntt;
+  int64_t *scratch;     // [2][count][limbs][N]
+  int64_t *out;         // [limbs][N] of ciphertext c at out + c * out_stride
+  int64_t out_stride;
+  int count, limbs, moduli_id;
+};
+
+template <int LOGN>
+__device__ __forceinline__ bool all_zero(const int64_t *x) {
+  int any = 0;
+  for (int j = threadIdx.x; j < (1 << LOGN); j += kBlock)
+    any |= x[j] != 0;
+  return !__syncthreads_or(any);
+}
+
+template <int LOGN>
+__global__ __launch_bounds__(kBlock) void repair_zero_kernel(RepairArgs a,
+                                                             DeviceTables t) {
+  constexpr int LO = r16_low_bits(LOGN), HI = r16_high_bits(LOGN);
+  constexpr int tiles = 1 << (LOGN - 12);
+  constexpr int64_t n = int64_t(1) << LOGN;
+  __shared__ int64_t
+      lds[kR16Lds<LO> > kR16Lds<HI> ? kR16Lds<LO> : kR16Lds<HI>];
+  if (a.zero[blockIdx.x] == 0)
+    return;
+  const int c = int(blockIdx.x) / a.limbs, l = int(blockIdx.x) % a.limbs;
+  const int p = a.moduli_id + l;
+  int64_t *out = a.out + c * a.out_stride + int64_t(l) * n;
+  const int64_t *z;
+  if (a.a) {
+    const int64_t *x[2];
+    bool zero = false;
+    int64_t *mine = nullptr;
+    for (int k = 0; k < 2; k++) {
+      const int64_t *in = (k ? a.b : a.a) +
+                          ((int64_t(2) * c + 1) * a.limbs + l) * n;
+      zero = zero || all_zero<LOGN>(in);
+      x[k] = in;
+      mine = a.scratch +
+             ((int64_t(k) * a.count + c) * a.limbs + l) * n;
+      if (k ? a.b_ntt : a.a_ntt)
+        continue;
+      x[k] = mine;
+      for (int tile = 0; tile < tiles; tile++)
+        r16_limb_pass<HI, false, true, kExact>(in, mine, p, tile, LO, t.r2,
+                                               kInttRaw, false, t, lds);
+      __syncthreads();
+      for (int tile = 0; tile < tiles; tile++)
+        r16_limb_pass<LO, false, false, kExact>(mine, mine, p, tile, 0,
+                                                nullptr, kInttRaw, true, t,
+                                                lds);
+      __syncthreads();
+    }
+    // an all-zero factor gives an all-zero product and inverse
+    if (zero) {
+      for (int j = threadIdx.x; j < n; j += kBlock)
+        out[j] = 0;
+      return;
+    }
+    for (int j = threadIdx.x; j < n; j += kBlock)
+      mine[j] = mont_mult_u(x[0][j], x[1][j], t.q[p], t.k[p]);
+    __syncthreads();
+    z = mine;
+  } else {
+    z = a.z + c * a.z_stride + int64_t(l) * n;
+  }
+  for (int tile = 0; tile < tiles; tile++)
+    r16_limb_pass<LO, true, false, kExact>(z, out, p, tile, 0, nullptr,
+                                           kInttRaw, false, t, lds);
+  __syncthreads();
+  for (int tile = 0; tile < tiles; tile++)
+    r16_limb_pass<HI, true, true, kExact>(out, out, p, tile, LO, nullptr,
+                                          kInttExit, true, t, lds);
+}
+
+void launch_repair(const DeviceTables &t, const RepairArgs &a,
+                   hipStream_t stream) {
+  with_log_n(t.log_n, [&](auto logn) {
+    hipLaunchKernelGGL(repair_zero_kernel<decltype(logn)::value>,
+                       dim3(unsigned(a.count * a.limbs)), dim3(kBlock), 0,
+                       stream, a, t);
+  });
+}
+
+} // namespace
+
+void launch_repair_intt(const DeviceTables &t, const uint32_t *zero,
+                        const int64_t *z, int64_t z_stride, int64_t *out,
+                        int64_t out_stride, int count, int limbs,
+                        int moduli_id, hipStream_t stream) {
+  RepairArgs a{};
+  a.zero = zero;
+  a.z = z;
+  a.z_stride = z_stride;
+  a.out = out;
+  a.out_stride = out_stride;
+  a.count = count;
+  a.limbs = limbs;
+  a.moduli_id = moduli_id;
+  launch_repair(t, a, stream);
+}
+
+void launch_repair_product(const DeviceTables &t, const uint32_t *zero,
+                           const int64_t *x, bool x_ntt, const int64_t *y,
+                           bool y_ntt, int64_t *scratch, int64_t *out,
+                           int64_t out_stride, int count, int limbs,
+                           int moduli_id, hipStream_t stream) {
+  RepairArgs a{};
+  a.zero = zero;
+  a.a = x;
+  a.b = y;
+  a.a_ntt = x_ntt;
+  a.b_ntt = y_ntt;
+  a.scratch = scratch;
+  a.out = out;
+  a.out_stride = out_stride;
+  a.count = count;
+  a.limbs = limbs;
+  a.moduli_id = moduli_id;
+  launch_repair(t, a, stream);
 }
 
 } // namespace fhe

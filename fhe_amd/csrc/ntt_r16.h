@@ -48,6 +48,23 @@ __host__ __device__ constexpr int r16_high_bits(int log_n) {
   return log_n - r16_low_bits(log_n);
 }
 
+// Calls f with log2 N (13 .. 16) as a compile-time constant.
+template <class F> void with_log_n(int log_n, F &&f) {
+  switch (log_n) {
+  case 13:
+    f(std::integral_constant<int, 13>());
+    break;
+  case 14:
+    f(std::integral_constant<int, 14>());
+    break;
+  case 15:
+    f(std::integral_constant<int, 15>());
+    break;
+  default:
+    f(std::integral_constant<int, 16>());
+  }
+}
+
 enum NttArith : int { kExact = 0, kF64 = 1, kLazyLarge = 2 };
 
 // Values of a transform in arithmetic A.
@@ -361,6 +378,8 @@ __device__ __forceinline__ void r16_exchange_words(V (&x)[16], uint32_t *lds,
 // (prime p); the pass covers index bits [b, b + L); COLS is b > 0.  pre
 // (forward, per prime) multiplies every loaded value first; post (inverse)
 // is the InttPost epilogue; last = the pass completes a forward transform.
+// zero (lazy inverse): a flag word of the limb, cleared by the first pass and
+// set by the last one where a canonical result is zero (repair_zero_limb).
 // OPAQUE: the pass runs inside a persistent loop (opaque_tid).
 template <int L, bool INV, bool COLS, int A, bool OPAQUE = false>
 __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
@@ -368,7 +387,8 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
                                               int tile, int b,
                                               const int64_t *pre, int post,
                                               bool last, const DeviceTables &t,
-                                              int64_t *lds) {
+                                              int64_t *lds,
+                                              uint32_t *zero = nullptr) {
   const int tid = OPAQUE ? opaque_tid() : int(threadIdx.x);
   constexpr int T = 1 << (L - 4), C = 4096 >> L;
   const int c = COLS ? (tid & (C - 1)) : (tid >> (L - 4));
@@ -452,8 +472,8 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
       }
     } else if (post != kInttRaw) {
       const int64_t ninv = t.ninv[p];
-      const bool reduce = post != kInttExit;
       if constexpr (A == kExact) {
+        const bool reduce = post != kInttExit;
 #pragma unroll
         for (int m = 0; m < 16; m++) {
           // only the exact arithmetic carries negative values
@@ -464,18 +484,18 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
       } else {
         // kLazyLarge needs only the residue: one product with N^-1 R^-1
         // (the exit folded into the constant) gives it below v q / 2^62 + q
-        // < 2q (v < 2q), which the reduce brings to the canonical value
+        // < 2q (v < 2q), which the guard brings to the canonical value
         const int64_t ninv_exit = mont_exit(ninv, s.q, s.k);
 #pragma unroll
-        for (int m = 0; m < 16; m++) {
-          const int64_t y = mont_mult_u(v[m], ninv_exit, s.q, s.k);
-          v[m] = reduce ? guard_u(y, int64_t(s.q)) : y;
-        }
+        for (int m = 0; m < 16; m++)
+          v[m] = guard_u(mont_mult_u(v[m], ninv_exit, s.q, s.k),
+                         int64_t(s.q));
       }
     }
   }
   // store: ROWS ownership except the strided forward pass (COLS)
   constexpr bool cols_store = !INV && COLS;
+  bool any_zero = false;
 #pragma unroll
   for (int m = 0; m < 16; m++) {
     int64_t y;
@@ -486,7 +506,13 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
     else
       y = f64_to_int(INV && post != kInttRaw ? v[m]
                                              : f64_floor_mod(v[m], s.f));
+    if (INV && A != kExact && !first_pass)
+      any_zero = any_zero || y == 0;
     dst[int64_t(r16_point<L, cols_store>(r, m)) << b] = y;
+  }
+  if (INV && A != kExact && zero) {
+    if (first_pass ? (tile == 0 && tid == 0) : any_zero)
+      *zero = first_pass ? 0 : 1;
   }
 }
 

@@ -72,12 +72,21 @@ constexpr int kUnevenSignedF64 = 3;
 // limb `limb` of polynomial `poly` at src.p[ct] + (poly * stride + limb) N,
 // stride = the ciphertext's limbs (ext_stride = 0) or extended limbs (1);
 // prime moduli_id + limb.  inverse / b / pre / post / last as
-// r16_limb_pass.
+// r16_limb_pass.  zero (optional): polynomial 2's zero-residue flag of limb l
+// is word l of zero->p[ct] (uint32_t).
 void launch_uneven_ntt(const DeviceTables &t, const UnevenCt *cts,
                        const UnitList &list, const UnevenPtrs &src,
                        const UnevenPtrs &dst, int ext_stride, bool inverse,
                        int b, const int64_t *pre, int post, bool last,
-                       int variant, int cap, hipStream_t stream);
+                       int variant, int cap, hipStream_t stream,
+                       const UnevenPtrs *zero = nullptr);
+
+// Exact recomputation of the flagged limbs of polynomial 2 (launch_repair_intt)
+// from its NTT form z.p[ct] into out.p[ct], both [limbs][N].
+void launch_uneven_repair(const DeviceTables &t, const UnevenCt *cts,
+                          int count, int max_limbs, const UnevenPtrs &zero,
+                          const UnevenPtrs &z, const UnevenPtrs &out,
+                          hipStream_t stream);
 
 // Garner digits of every listed (ct, partition, coefficient chunk of 256):
 // x.p[ct] is the INTT-form source polynomial, digits.p[ct] receives

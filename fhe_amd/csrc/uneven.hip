@@ -60,6 +60,7 @@ struct UnevenPlan {
   int key_moduli_id = 0;
   int count = 0;
   int maxz = 1;
+  int max_limbs = 1;
   std::vector<UnevenCt> host;
   UnevenCt *dev = nullptr;
   uint32_t *units = nullptr;
@@ -114,6 +115,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     u.moduli_id = m;
     u.limbs = P.limbs_at(m);
     u.ext = u.limbs + P.alpha;
+    plan->max_limbs = std::max(plan->max_limbs, u.limbs);
     const auto parts = P.partitions(m, key_moduli_id);
     require(int(parts.size()) <= fhe::kUnevenMaxParts,
             "Uneven batch: too many key-switching partitions");
@@ -174,7 +176,6 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
     return int64_t(prime) * 256 + tile;
   };
   if (relin) {
-    // the trio's d2 exact (it feeds ModUp), d0 / d1 lazy
     for (int stage : {int(kStTrioIntt1), int(kStTrioIntt2)}) {
       std::vector<Keyed> lists[4];
       for (int c = 0; c < count; c++) {
@@ -183,7 +184,7 @@ UnevenPlan *uneven_plan(fhe_context *ctx, bool relin,
           for (int l = 0; l < u.limbs; l++)
             for (int t = 0; t < tiles; t++) {
               const int prime = u.moduli_id + l;
-              const int v = poly == 2 ? fhe::kExact : lazy_variant(P, prime);
+              const int v = lazy_variant(P, prime);
               lists[v].push_back({tile_key(prime, t),
                                   fhe::unit_pack(c, poly, l, t)});
             }
@@ -322,14 +323,20 @@ void uneven_run(fhe_context *ctx, UnevenPlan *plan, const int64_t *const *src,
       case kStTrioIntt1:
         fhe::launch_uneven_ntt(t, plan->dev, list, in, tmp, 0, true, 0,
                                nullptr, fhe::kInttRaw, false, L.variant,
-                               s.cap, ctx->stream);
+                               s.cap, ctx->stream, &acc);
         break;
       case kStTrioIntt2:
         fhe::launch_uneven_ntt(t, plan->dev, list, tmp, tmp, 0, true, 8,
                                nullptr, fhe::kInttExit, true, L.variant,
-                               s.cap, ctx->stream);
+                               s.cap, ctx->stream, &acc);
         break;
       case kStDigits:
+        // d2's limbs with a zero residue again, exactly (the flags are in
+        // the accumulators, written later)
+        if (plan->relin)
+          fhe::launch_uneven_repair(t, plan->dev, plan->count,
+                                    plan->max_limbs, acc, own, x,
+                                    ctx->stream);
         fhe::launch_uneven_digits(t, plan->dev, list, x, digits, plan->maxz,
                                   s.cap, ctx->stream);
         break;

@@ -43,7 +43,7 @@ unsigned grid_of(int count, int cap) {
 struct UnevenNttArgs {
   UnitList list;
   const UnevenCt *cts;
-  UnevenPtrs src, dst;
+  UnevenPtrs src, dst, zero;
   const int64_t *pre;
   int ext_stride, b, post, last;
 };
@@ -58,11 +58,43 @@ __global__ __launch_bounds__(kBlock) void uneven_ntt_kernel(UnevenNttArgs a,
     const UnevenCt &ct = a.cts[c];
     const int stride = a.ext_stride ? ct.ext : ct.limbs;
     const int64_t off = (int64_t(unit_a(unit)) * stride + l) << t.log_n;
+    uint32_t *zero = nullptr;
+    if (A != kExact && a.zero.p[c] && unit_a(unit) == 2)
+      zero = reinterpret_cast<uint32_t *>(const_cast<int64_t *>(a.zero.p[c])) +
+             l;
     r16_limb_pass<8, INV, COLS, A, true>(a.src.p[c] + off,
                                 const_cast<int64_t *>(a.dst.p[c]) + off,
                                 ct.moduli_id + l, unit_tile(unit), a.b, a.pre,
-                                a.post, a.last != 0, t, lds);
+                                a.post, a.last != 0, t, lds, zero);
   }
+}
+
+struct UnevenRepairArgs {
+  const UnevenCt *cts;
+  UnevenPtrs zero, z, out;
+  int max_limbs;
+};
+
+// As repair_zero_kernel (ntt.hip) for an NTT-form source.
+__global__ __launch_bounds__(kBlock) void uneven_repair_kernel(
+    UnevenRepairArgs a, DeviceTables t) {
+  __shared__ int64_t lds[kR16Lds<8>];
+  const int c = int(blockIdx.x) / a.max_limbs;
+  const int l = int(blockIdx.x) % a.max_limbs;
+  const UnevenCt &ct = a.cts[c];
+  if (l >= ct.limbs ||
+      reinterpret_cast<const uint32_t *>(a.zero.p[c])[l] == 0)
+    return;
+  const int64_t at = int64_t(l) << t.log_n;
+  const int64_t *z = a.z.p[c] + at;
+  int64_t *out = const_cast<int64_t *>(a.out.p[c]) + at;
+  for (int tile = 0; tile < 16; tile++)
+    r16_limb_pass<8, true, false, kExact>(z, out, ct.moduli_id + l, tile, 0,
+                                          nullptr, kInttRaw, false, t, lds);
+  __syncthreads();
+  for (int tile = 0; tile < 16; tile++)
+    r16_limb_pass<8, true, true, kExact>(out, out, ct.moduli_id + l, tile, 8,
+                                         nullptr, kInttExit, true, t, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -277,10 +309,12 @@ void launch_uneven_ntt(const DeviceTables &t, const UnevenCt *cts,
                        const UnitList &list, const UnevenPtrs &src,
                        const UnevenPtrs &dst, int ext_stride, bool inverse,
                        int b, const int64_t *pre, int post, bool last,
-                       int variant, int cap, hipStream_t stream) {
+                       int variant, int cap, hipStream_t stream,
+                       const UnevenPtrs *zero) {
   if (list.count == 0)
     return;
-  UnevenNttArgs a{list, cts, src, dst, pre, ext_stride, b, post, last ? 1 : 0};
+  UnevenNttArgs a{list, cts, src, dst, zero ? *zero : UnevenPtrs{}, pre,
+                  ext_stride, b, post, last ? 1 : 0};
   const dim3 grid(grid_of(list.count, cap));
   const bool cols = b > 0;
 #define FHE_UNTT(I, C, A)                                                      \
@@ -308,6 +342,15 @@ void launch_uneven_ntt(const DeviceTables &t, const UnevenCt *cts,
   }
 #undef FHE_UNTT_A
 #undef FHE_UNTT
+}
+
+void launch_uneven_repair(const DeviceTables &t, const UnevenCt *cts,
+                          int count, int max_limbs, const UnevenPtrs &zero,
+                          const UnevenPtrs &z, const UnevenPtrs &out,
+                          hipStream_t stream) {
+  UnevenRepairArgs a{cts, zero, z, out, max_limbs};
+  hipLaunchKernelGGL(uneven_repair_kernel, dim3(unsigned(count * max_limbs)),
+                     dim3(kBlock), 0, stream, a, t);
 }
 
 void launch_uneven_digits(const DeviceTables &t, const UnevenCt *cts,

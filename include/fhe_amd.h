@@ -752,21 +752,11 @@ int fhe_mod_raise(fhe_context *ctx, int count, const int64_t *in,
  *   "staged_modup" 1       ModUp through the Garner digits;
  *   "own_limbs" 1          partitions' own extended limbs from the NTT-form
  *                          input;
- *   "split_variants" 1     one NTT launch per arithmetic variant;
- *   "ks_lazy_accumulate" 1 small-prime key products summed without
- *                          intermediate reductions, large-prime sums kept
- *                          below 2q with one conditional subtraction;
- *   "overlap_trio" 1       N >= 2^13 with split_variants: the INTT of d0 and
- *                          d1 in fhe_hmult_relin_rescale runs on a second
- *                          non-blocking stream of the context (default
- *                          priority), joined by an event before ModDown;
- *                          forked once the trio is written (1), or once
- *                          d2's INTT is done (2: beside the key inner
- *                          product, about 1% more throughput, that kernel's
- *                          launches then sharing the device); 0: one stream.
- * "fuse_modup", "fuse_tensor", "ks_wide_accumulate", "ks_occupancy" and
- * "ks_prefetch" name pipelines that the defaults have replaced; they are
- * accepted and have no effect.
+ *   "ks_lazy_accumulate" 1 large-prime key-product sums kept below 2q with
+ *                          one conditional subtraction.
+ * "fuse_modup", "fuse_tensor", "ks_wide_accumulate", "ks_occupancy",
+ * "ks_prefetch", "overlap_trio" and "split_variants" name pipelines that the
+ * defaults have replaced; they are accepted and have no effect.
  * Synchronizes the context's stream. */
 int fhe_context_set_option(fhe_context *ctx, const char *name, int value);
 
