@@ -216,6 +216,8 @@ Text apply_butterfly_bk(TextEngine &e, const fhe_bootstrap_key &bk,
   const int64_t N = ctx->n(), ext = int64_t(E) * N;
   const int parts = int(P.partitions(m, m).size());
 
+  // only residues matter in the extended basis (bk_kernels.hip)
+  const fhe::LazySpec lazy{ctx->lazy_transforms()};
   // attach_special_prime_chains_ (src/ckks/core.cpp:1127-1155): x P in the
   // chain limbs, zero special limbs, NTT
   auto attached_h = e.take(size_t(B) * 2 * ext * 8);
@@ -224,7 +226,7 @@ Text apply_butterfly_bk(TextEngine &e, const fhe_bootstrap_key &bk,
     fhe::launch_bk_attach(T, r.data, attached, int64_t(B) * 2, limbs, E,
                           stream);
     fhe::ntt_forward(T, attached, attached, int64_t(B) * 2 * E, E, m,
-                     bk.p_r2, stream);
+                     bk.p_r2, stream, lazy);
   });
   auto dec_h = e.take(size_t(B) * parts * ext * 8);
   int64_t *dec = static_cast<int64_t *>(dec_h.get());
@@ -301,7 +303,7 @@ Text apply_butterfly_bk(TextEngine &e, const fhe_bootstrap_key &bk,
     int64_t *reduced = static_cast<int64_t *>(reduced_h.get());
     ctx->stage("bk_giant_moddown", [&] {
       fhe::ntt_inverse(T, c1s, c1s, int64_t(rotating) * B * E, E, m,
-                       fhe::kInttExitReduce, stream);
+                       fhe::kInttExitReduce, stream, lazy);
       fhe::launch_moddown_polys(T, c1s, reduced, int64_t(rotating) * B, limbs,
                                 m, stream);
     });
@@ -345,7 +347,7 @@ Text apply_butterfly_bk(TextEngine &e, const fhe_bootstrap_key &bk,
   Text out = e.alloc(2, out_level, 0, B);
   ctx->stage("bk_remove_special", [&] {
     fhe::ntt_inverse(T, outer, outer, int64_t(B) * 2 * E, E, m,
-                     fhe::kInttExitReduce, stream);
+                     fhe::kInttExitReduce, stream, lazy);
     fhe::launch_moddown_add(T, outer, nullptr, 0, 0, out.data, B, limbs, m,
                             stream);
   });

@@ -850,15 +850,17 @@ void encode_texts(fhe_context *ctx, const double *values, bool complex_input,
 // skips the NTT tables (host-only queries).
 fhe::CkksParams resolve_params(const fhe_params *p, bool twiddles = true);
 
-// The batched HMult + relinearize + rescale pipeline (context.hip) on a
+// The batched product, relinearization and, with rescale, rescale pipeline
+// (context.hip) of duos in INTT form, or NTT form with a_ntt / b_ntt, on a
 // caller-given workspace of hmult_workspace_words words and, when given, a
 // digits buffer of ks_digits_words words.
 int64_t hmult_workspace_words(const fhe_context *ctx, int count,
                               int moduli_id);
-void hmult_relin_rescale_into(fhe_context *ctx, int count, int moduli_id,
-                              const int64_t *a, const int64_t *b,
-                              const int64_t *key, int key_moduli_id,
-                              int64_t *out, int64_t *ws, int64_t *digits);
+void hmult_relin_into(fhe_context *ctx, int count, int moduli_id,
+                      const int64_t *a, bool a_ntt, const int64_t *b,
+                      bool b_ntt, const int64_t *key, int key_moduli_id,
+                      bool rescale, int64_t *out, int64_t *ws,
+                      int64_t *digits);
 // Set-up of the allocation-free entry point on the current device `device`
 // (noalloc.hip).
 void noalloc_scratch_setup(int device);

@@ -333,14 +333,15 @@ int64_t hmult_workspace_words(const fhe_context *ctx, int count,
   return (2 * duo_l + 2 * trio_l + ext_l + acc_l) * int64_t(P.n);
 }
 
-// The batched HMult + relinearize + rescale pipeline on the workspace ws
+// The batched HMult + relinearize (+ rescale) pipeline on the workspace ws
 // (hmult_workspace_words) and, when given, the digits buffer (the staged
 // ModUp's Garner digits; else the context's second buffer).  Arguments are
 // checked by the caller.
-void hmult_relin_rescale_into(fhe_context *ctx, int count, int moduli_id,
-                              const int64_t *a, const int64_t *b,
-                              const int64_t *key, int key_moduli_id,
-                              int64_t *out, int64_t *ws, int64_t *digits) {
+void hmult_relin_into(fhe_context *ctx, int count, int moduli_id,
+                      const int64_t *a, bool a_ntt, const int64_t *b,
+                      bool b_ntt, const int64_t *key, int key_moduli_id,
+                      bool rescale, int64_t *out, int64_t *ws,
+                      int64_t *digits) {
     const auto &P = ctx->params;
     const int limbs = P.limbs_at(moduli_id);
     const int ext_limbs = limbs + P.alpha;
@@ -364,14 +365,25 @@ void hmult_relin_rescale_into(fhe_context *ctx, int count, int moduli_id,
     fhe::LazySpec flagged = lazy;
     flagged.zero = reinterpret_cast<uint32_t *>(acc);
     flagged.zero_period = 3;
+    const int64_t *x = a_ntt ? a : an, *y = b_ntt ? b : bn;
+    const bool square = a == b && a_ntt == b_ntt;
+    if (square)
+      y = x;
     ctx->stage("ntt(inputs)", [&] {
-      fhe::ntt_forward(ctx->tables, a, an, duo_l, limbs, moduli_id,
-                       ctx->tables.r2, ctx->stream, lazy);
-      fhe::ntt_forward(ctx->tables, b, bn, duo_l, limbs, moduli_id,
-                       ctx->tables.r2, ctx->stream, lazy);
+      if (!a_ntt && !b_ntt && !square) {
+        fhe::ntt_forward_pair(ctx->tables, a, b, an, duo_l, limbs, moduli_id,
+                              ctx->tables.r2, ctx->stream, lazy);
+        return;
+      }
+      if (!a_ntt)
+        fhe::ntt_forward(ctx->tables, a, an, duo_l, limbs, moduli_id,
+                         ctx->tables.r2, ctx->stream, lazy);
+      if (!b_ntt && !square)
+        fhe::ntt_forward(ctx->tables, b, bn, duo_l, limbs, moduli_id,
+                         ctx->tables.r2, ctx->stream, lazy);
     });
     ctx->stage("tensor", [&] {
-      fhe::launch_tensor(ctx->tables, an, bn, trio, count, limbs, moduli_id,
+      fhe::launch_tensor(ctx->tables, x, y, trio, count, limbs, moduli_id,
                          ctx->stream);
     });
     // relinearize: to_intt of all three, key switch of the third
@@ -379,13 +391,20 @@ void hmult_relin_rescale_into(fhe_context *ctx, int count, int moduli_id,
       fhe::ntt_inverse(ctx->tables, trio, trio_c, trio_l, limbs, moduli_id,
                        fhe::kInttExit, ctx->stream, flagged);
       if (flagged.on)
-        fhe::launch_repair_product(ctx->tables, flagged.zero, a, false, b,
-                                   false, an, trio_c + 2 * poly, 3 * poly,
+        fhe::launch_repair_product(ctx->tables, flagged.zero, a, a_ntt, b,
+                                   b_ntt, an, trio_c + 2 * poly, 3 * poly,
                                    count, limbs, moduli_id, ctx->stream);
     });
     ctx->key_switch(count, moduli_id, key, key_moduli_id,
                     trio_c + 2 * limbs * N, 3 * limbs * N, ext, acc,
                     trio + 2 * limbs * N, 3 * limbs * N, false, digits);
+    if (!rescale) {
+      ctx->stage("moddown_relin", [&] {
+        fhe::launch_moddown_relin(ctx->tables, acc, trio_c, out, count, limbs,
+                                  moduli_id, ctx->stream);
+      });
+      return;
+    }
     ctx->stage("moddown_relin_rescale", [&] {
       fhe::launch_moddown_relin_rescale(ctx->tables, acc, trio_c, out, count,
                                         limbs, moduli_id, ctx->stream);
@@ -405,8 +424,8 @@ int fhe_hmult_relin_rescale(fhe_context *ctx, int count, int moduli_id,
     ctx->check_key(moduli_id, key_moduli_id, "Multiply");
     int64_t *ws = ctx->scratch(
         size_t(hmult_workspace_words(ctx, count, moduli_id)) * 8);
-    hmult_relin_rescale_into(ctx, count, moduli_id, a, b, key, key_moduli_id,
-                             out, ws, nullptr);
+    hmult_relin_into(ctx, count, moduli_id, a, false, b, false, key,
+                     key_moduli_id, true, out, ws, nullptr);
     ctx->check_launch("Multiply");
   });
 }
@@ -439,14 +458,13 @@ static void multiply_texts(fhe_context *ctx, int count, const int64_t *a,
   const int prod_polys = b_polys == 2 ? 3 : a_polys;
   if (key)
     ctx->check_key(mid, key_moduli_id, op);
-  // prepared inputs and the product in the stash; the preparation's
-  // temporaries in the scratch workspace, which relinearization reuses
+  // prepared inputs in the stash; the preparation's temporaries in the
+  // scratch workspace, which the product reuses
   const int64_t an_l = int64_t(count) * a_polys * poly;
   const int64_t bn_l = int64_t(count) * b_polys * poly;
-  const int64_t prod_l = int64_t(count) * prod_polys * poly;
-  int64_t *an = ctx->stash(size_t(an_l + bn_l + (key ? prod_l : 0)) * 8);
+  int64_t *an = ctx->stash(size_t(an_l + bn_l) * 8);
   int64_t *bn = an + an_l;
-  int64_t *prod = key ? bn + bn_l : out;
+  int64_t *prod = out;
   auto limbs_of = [&](int l, int f) {
     return int64_t(P.limbs_at(ctx->moduli_id_of(l, f & FHE_FLAG_RESCALED)));
   };
@@ -454,7 +472,31 @@ static void multiply_texts(fhe_context *ctx, int count, const int64_t *a,
       std::max(int64_t(count) * a_polys * limbs_of(a_level, a_flags),
                int64_t(count) * b_polys * limbs_of(b_level, b_flags)) *
       N;
-  int64_t *t0 = ctx->scratch(size_t(2 * t_l) * 8), *t1 = t0 + t_l;
+  const int64_t ws_l = key ? hmult_workspace_words(ctx, count, mid) : 0;
+  int64_t *t0 = ctx->scratch(size_t(std::max(2 * t_l, ws_l)) * 8);
+  int64_t *t1 = t0 + t_l;
+  if (key) {
+    // rescaled at the lower level, in the coefficient domain unless the text
+    // is there in NTT form already; the product's pipeline transforms it
+    auto prepared = [&](const int64_t *in, int level_in, int flags,
+                        int64_t *dst, bool &ntt) {
+      ntt = (flags & FHE_FLAG_NTT_FORM) && (flags & FHE_FLAG_RESCALED) &&
+            level_in == level;
+      return ntt ? in
+                 : ctx->transform_into(in, int64_t(count) * 2, level_in, flags,
+                                       true, level, true, false, dst, t0, t1);
+    };
+    bool a_ntt = false, b_ntt = false;
+    const int64_t *ap = prepared(a, a_level, a_flags, an, a_ntt);
+    const bool same = a == b && a_level == b_level && a_flags == b_flags;
+    if (same)
+      b_ntt = a_ntt;
+    const int64_t *bp =
+        same ? ap : prepared(b, b_level, b_flags, bn, b_ntt);
+    hmult_relin_into(ctx, count, mid, ap, a_ntt, bp, b_ntt, key, key_moduli_id,
+                     false, out, t0, nullptr);
+    return;
+  }
   const int64_t *ap = ctx->prepare_for_multiply_into(
       a, int64_t(count) * a_polys, a_level, a_flags, level, an, t0, t1);
   const int64_t *bp = ctx->prepare_for_multiply_into(
@@ -476,8 +518,6 @@ static void multiply_texts(fhe_context *ctx, int count, const int64_t *a,
                                 limbs, mid, ctx->stream);
     });
   }
-  if (key)
-    ctx->relinearize_into(count, mid, prod, key, key_moduli_id, out);
 }
 
 int fhe_multiply(fhe_context *ctx, int count, const int64_t *a, int a_level,

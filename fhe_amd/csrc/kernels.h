@@ -48,6 +48,13 @@ void ntt_forward(const DeviceTables &t, const int64_t *src, int64_t *dst,
                  const int64_t *pre, hipStream_t stream,
                  LazySpec lazy = LazySpec());
 
+// ntt_forward of two batches of total_limbs limbs each, x then y, into one
+// buffer dst (one launch per pass at the radix-16 sizes).
+void ntt_forward_pair(const DeviceTables &t, const int64_t *x,
+                      const int64_t *y, int64_t *dst, int64_t total_limbs,
+                      int limbs, int moduli_id, const int64_t *pre,
+                      hipStream_t stream, LazySpec lazy = LazySpec());
+
 // In-place capable inverse NTT with the InttPost epilogue.
 void ntt_inverse(const DeviceTables &t, const int64_t *src, int64_t *dst,
                  int64_t total_limbs, int limbs, int moduli_id, int post,

@@ -98,9 +98,9 @@ extern "C" int fhe_hmult_relin_rescale_noalloc(fhe_context *ctx, int count,
     const int64_t res = in - 2 * ctx->n();
     for (int c = 0; c < count; c += part) {
       const int n = std::min(part, count - c);
-      hmult_relin_rescale_into(
-          ctx, n, moduli_id, a + c * in, b + c * in, key, key_moduli_id,
-          out + c * res, base, base + hmult_workspace_words(ctx, n, moduli_id));
+      hmult_relin_into(ctx, n, moduli_id, a + c * in, false, b + c * in, false,
+                       key, key_moduli_id, true, out + c * res, base,
+                       base + hmult_workspace_words(ctx, n, moduli_id));
     }
     ctx->check_launch("Multiply");
   });

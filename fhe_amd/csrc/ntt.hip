@@ -40,6 +40,9 @@ struct PassArgs {
   bool lazy;          // lazy arithmetic (radix-16 passes only)
   uint32_t *zero;     // LazySpec::zero
   int zero_period;
+  // radix-16 passes: polynomials from `split` on are read from src2
+  const int64_t *src2 = nullptr;
+  int64_t split = 0;
 };
 
 template <bool INV>
@@ -165,7 +168,10 @@ __global__ __launch_bounds__(kBlock) void ntt_radix16_kernel(
   const int tile = int(rest % tiles_per_limb);
   const int l = int(rest / tiles_per_limb);
   const int64_t limb = (poly * a.limbs + l) << t.log_n;
-  const int64_t *src = a.src + limb;
+  const int64_t *src =
+      a.src2 && poly >= a.split
+          ? a.src2 + (((poly - a.split) * a.limbs + l) << t.log_n)
+          : a.src + limb;
   int64_t *dst = a.dst + limb;
   const int p = a.moduli_id + l;
   if constexpr (!LAZY) {
@@ -272,6 +278,33 @@ void ntt_forward(const DeviceTables &t, const int64_t *src, int64_t *dst,
                 1,     lazy.on, lazy.zero, lazy.zero_period};
     launch_pass<false>(b2, t, stream);
   }
+}
+
+void ntt_forward_pair(const DeviceTables &t, const int64_t *x,
+                      const int64_t *y, int64_t *dst, int64_t total_limbs,
+                      int limbs, int moduli_id, const int64_t *pre,
+                      hipStream_t stream, LazySpec lazy) {
+  if (!r16_supported(t.log_n)) {
+    ntt_forward(t, x, dst, total_limbs, limbs, moduli_id, pre, stream, lazy);
+    ntt_forward(t, y, dst + (total_limbs << t.log_n), total_limbs, limbs,
+                moduli_id, pre, stream, lazy);
+    return;
+  }
+  int l1, l2;
+  split_bits(t.log_n, false, l1, l2);
+  PassArgs a{x,       dst,       (2 * total_limbs) << (t.log_n - l1),
+             limbs,   moduli_id, t.log_n - l1,
+             l1,      pre,       kInttRaw,
+             0,       lazy.on,   lazy.zero,
+             lazy.zero_period,   y,
+             total_limbs / limbs};
+  launch_pass<false>(a, t, stream);
+  PassArgs b{dst,   dst,       (2 * total_limbs) << (t.log_n - l2),
+             limbs, moduli_id, 0,
+             l2,    nullptr,   kInttRaw,
+             1,     lazy.on,   lazy.zero,
+             lazy.zero_period};
+  launch_pass<false>(b, t, stream);
 }
 
 void ntt_inverse(const DeviceTables &t, const int64_t *src, int64_t *dst,
