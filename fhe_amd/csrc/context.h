@@ -134,6 +134,8 @@ struct fhe_context {
   // use the other two
   void *stash_buf = nullptr;
   size_t stash_bytes = 0;
+  void *partial_buf = nullptr;
+  size_t partial_bytes = 0;
   // encoding tables, uploaded on the first encode
   fhe::EncodeDevice encode{};
   bool encode_ready = false;
@@ -255,6 +257,8 @@ struct fhe_context {
       (void)hipFree(aux);
     if (stash_buf)
       (void)hipFree(stash_buf);
+    if (partial_buf)
+      (void)hipFree(partial_buf);
     if (stream)
       (void)hipStreamDestroy(stream);
   }
@@ -351,6 +355,23 @@ struct fhe_context {
       aux_bytes = bytes;
     }
     return static_cast<int64_t *>(aux);
+  }
+
+  // partial sums of the split key inner product; null where the buffer would
+  // have to grow while a graph holds it (the caller then does not split)
+  int64_t *partial_sums(size_t bytes) {
+    if (bytes > partial_bytes) {
+      if (capturing || live_graphs != 0)
+        return nullptr;
+      hip_check(hipStreamSynchronize(stream), "workspace sync");
+      if (partial_buf)
+        hip_check(hipFree(partial_buf), "workspace free");
+      partial_buf = nullptr;
+      partial_bytes = 0;
+      hip_check(hipMalloc(&partial_buf, bytes), "workspace allocation");
+      partial_bytes = bytes;
+    }
+    return static_cast<int64_t *>(partial_buf);
   }
 
   int64_t *stash(size_t bytes) {
@@ -701,7 +722,7 @@ struct fhe_context {
       ks_decompose(count, moduli_id, key_moduli_id, src, src_stride, ext,
                    own != nullptr, signed_input, digits);
       ks_apply(count, moduli_id, key, key_moduli_id, ext, acc, own,
-               own_stride);
+               own_stride, digits == nullptr);
       return;
     }
     const int limbs = params.limbs_at(moduli_id);
@@ -812,7 +833,8 @@ struct fhe_context {
   // into acc [count][2][ext][N].
   void ks_apply(int count, int moduli_id, const int64_t *key,
                 int key_moduli_id, const int64_t *ext, int64_t *acc,
-                const int64_t *own = nullptr, int64_t own_stride = 0) {
+                const int64_t *own = nullptr, int64_t own_stride = 0,
+                bool may_allocate = true) {
     const int limbs = params.limbs_at(moduli_id);
     const int ext_limbs = limbs + params.alpha;
     const int key_chain = params.limbs_at(key_moduli_id) + params.alpha;
@@ -827,16 +849,33 @@ struct fhe_context {
     }
     if (np > fhe::kMaxFusedParts)
       own = nullptr;
+    fhe::KsSplit split;
+    fhe::PartialSums more;
+    int64_t *partials = nullptr;
+    if (may_allocate) {
+      split = fhe::ks_split(tables, np, count, ext_limbs, lazy_key_switch);
+      more.stride = int64_t(count) * 2 * ext_limbs * n();
+      more.count = split.groups - 1;
+      if (more.count > 0) {
+        partials = partial_sums(size_t(more.stride) * more.count * 8);
+        if (!partials) {
+          split = fhe::KsSplit();
+          more.count = 0;
+        }
+      }
+      more.data = partials;
+    }
     stage("ks_inner_product_r16", [&] {
       fhe::launch_ks_inner_product_fused(
           tables, ext, key, key_chain, key_offset, parts[0].key_index, np, acc,
           count, ext_limbs, moduli_id, lazy_key_switch, own, own_stride,
-          starts.data(), sizes.data(), ks_lazy_accumulate, stream);
+          starts.data(), sizes.data(), ks_lazy_accumulate, split, partials,
+          stream);
     });
     stage("intt_pass_high(acc)", [&] {
       fhe::ntt_inverse_second(tables, acc, acc, int64_t(count) * 2 * ext_limbs,
                               ext_limbs, moduli_id, fhe::kInttKeyReduce,
-                              stream, lazy);
+                              stream, lazy, more);
     });
   }
 };

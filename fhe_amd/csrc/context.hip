@@ -510,6 +510,12 @@ static void multiply_texts(fhe_context *ctx, int count, const int64_t *a,
   } else {
     // CKKSCore::multiply(ct, pt) (src/ckks/core.cpp:257-282)
     ctx->stage("mont_mult", [&] {
+      const fhe::TextOpArgs products{ap,   bp,   prod, a_polys * poly,
+                                     poly, poly, 0,    prod_polys * poly,
+                                     poly, a_polys, limbs, mid};
+      if (fhe::launch_text_op(ctx->tables, false, products, count,
+                              ctx->stream))
+        return;
       for (int c = 0; c < count; c++)
         for (int p = 0; p < a_polys; p++)
           fhe::launch_mont_mult(ctx->tables, ap + (c * a_polys + p) * poly,
@@ -923,13 +929,20 @@ int fhe_encrypt_pk(fhe_context *ctx, int count, int moduli_id,
                                 ctx->stream);
       fhe::ntt_forward(ctx->tables, un, un, int64_t(count) * limbs, limbs,
                        moduli_id, ctx->tables.r2, ctx->stream);
-      for (int c = 0; c < count; c++)
-        for (int h = 0; h < 2; h++)
-          fhe::launch_mont_mult(
-              ctx->tables, un + c * poly,
-              pk + (int64_t(h) * pk_limbs + (moduli_id - pk_moduli_id)) * N,
-              out + (2 * int64_t(c) + h) * poly, limbs, limbs, moduli_id,
-              ctx->stream);
+      const int64_t *pk0 = pk + int64_t(moduli_id - pk_moduli_id) * N;
+      const fhe::TextOpArgs products{un,   pk0,  out,
+                                     poly, 0,    0,
+                                     int64_t(pk_limbs) * N,
+                                     2 * poly, poly,
+                                     2,    limbs, moduli_id};
+      if (!fhe::launch_text_op(ctx->tables, false, products, count,
+                               ctx->stream))
+        for (int c = 0; c < count; c++)
+          for (int h = 0; h < 2; h++)
+            fhe::launch_mont_mult(ctx->tables, un + c * poly,
+                                  pk0 + int64_t(h) * pk_limbs * N,
+                                  out + (2 * int64_t(c) + h) * poly, limbs,
+                                  limbs, moduli_id, ctx->stream);
       fhe::ntt_inverse(ctx->tables, out, out, int64_t(count) * 2 * limbs,
                        limbs, moduli_id, fhe::kInttExit, ctx->stream);
       fhe::launch_encrypt_finish(ctx->tables, pt, e0, e1, out, count, limbs,
@@ -956,20 +969,26 @@ int fhe_decrypt(fhe_context *ctx, int count, int moduli_id, const int64_t *ct,
     const int64_t *s = sk + int64_t(moduli_id - sk_moduli_id) * N;
     ctx->stage("decrypt", [&] {
       // out_c = to_intt(to_ntt(c1) * s) (src/ckks/core.cpp:171-194)
-      for (int c = 0; c < count; c++) {
-        fhe::ntt_forward(ctx->tables, ct + (2 * int64_t(c) + 1) * poly,
-                         out + c * poly, limbs, limbs, moduli_id,
-                         ctx->tables.r2, ctx->stream);
-        fhe::launch_mont_mult(ctx->tables, out + c * poly, s, out + c * poly,
-                              limbs, limbs, moduli_id, ctx->stream);
-      }
+      if (!fhe::ntt_forward_strided(ctx->tables, ct + poly, 2 * poly, out,
+                                    count, limbs, moduli_id, ctx->tables.r2,
+                                    ctx->stream))
+        for (int c = 0; c < count; c++)
+          fhe::ntt_forward(ctx->tables, ct + (2 * int64_t(c) + 1) * poly,
+                           out + c * poly, limbs, limbs, moduli_id,
+                           ctx->tables.r2, ctx->stream);
+      fhe::launch_mont_mult_broadcast(ctx->tables, out, s, out,
+                                      int64_t(count) * limbs, limbs,
+                                      moduli_id, ctx->stream);
       fhe::ntt_inverse(ctx->tables, out, out, int64_t(count) * limbs, limbs,
                        moduli_id, fhe::kInttExit, ctx->stream);
-      for (int c = 0; c < count; c++)
-        fhe::launch_elementwise(ctx->tables, fhe::kEwAddReduce,
-                                ct + 2 * int64_t(c) * poly, out + c * poly,
-                                out + c * poly, limbs, limbs, moduli_id,
-                                nullptr, ctx->stream);
+      const fhe::TextOpArgs sums{ct, out, out,  2 * poly, 0,     poly,
+                                 0,  poly, 0, 1,        limbs, moduli_id};
+      if (!fhe::launch_text_op(ctx->tables, true, sums, count, ctx->stream))
+        for (int c = 0; c < count; c++)
+          fhe::launch_elementwise(ctx->tables, fhe::kEwAddReduce,
+                                  ct + 2 * int64_t(c) * poly, out + c * poly,
+                                  out + c * poly, limbs, limbs, moduli_id,
+                                  nullptr, ctx->stream);
     });
     ctx->check_launch("Decrypt");
   });

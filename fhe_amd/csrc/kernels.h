@@ -48,6 +48,13 @@ void ntt_forward(const DeviceTables &t, const int64_t *src, int64_t *dst,
                  const int64_t *pre, hipStream_t stream,
                  LazySpec lazy = LazySpec());
 
+// ntt_forward of `polys` polynomials at src + i * src_stride into dst
+// [polys][limbs][N] (the radix-16 sizes; false for others, nothing done).
+bool ntt_forward_strided(const DeviceTables &t, const int64_t *src,
+                         int64_t src_stride, int64_t *dst, int64_t polys,
+                         int limbs, int moduli_id, const int64_t *pre,
+                         hipStream_t stream);
+
 // ntt_forward of two batches of total_limbs limbs each, x then y, into one
 // buffer dst (one launch per pass at the radix-16 sizes).
 void ntt_forward_pair(const DeviceTables &t, const int64_t *x,
@@ -60,6 +67,14 @@ void ntt_inverse(const DeviceTables &t, const int64_t *src, int64_t *dst,
                  int64_t total_limbs, int limbs, int moduli_id, int post,
                  hipStream_t stream, LazySpec lazy = LazySpec());
 
+// Buffers like the source of the (lazy) second inverse pass, `count` of them
+// `stride` words apart, added to it as it is read.
+struct PartialSums {
+  const int64_t *data = nullptr;
+  int64_t stride = 0;
+  int count = 0;
+};
+
 // Single passes of the two-pass transform (N >= 2^13): the forward pass over
 // the high index bits, and the inverse pass over the high index bits with
 // the InttPost epilogue.  The remaining passes run inside fused kernels.
@@ -70,7 +85,8 @@ void ntt_forward_first(const DeviceTables &t, const int64_t *src, int64_t *dst,
 void ntt_inverse_second(const DeviceTables &t, const int64_t *src,
                         int64_t *dst, int64_t total_limbs, int limbs,
                         int moduli_id, int post, hipStream_t stream,
-                        LazySpec lazy = LazySpec());
+                        LazySpec lazy = LazySpec(),
+                        PartialSums more = PartialSums());
 // The forward pass over the low index bits, after ntt_forward_first: the two
 // together are ntt_forward.
 void ntt_forward_second(const DeviceTables &t, const int64_t *src,
@@ -85,6 +101,15 @@ void ntt_forward_second(const DeviceTables &t, const int64_t *src,
 // both accumulators.  ext: [count][parts][ext_limbs][N] after
 // ntt_forward_first; acc: [count][2][ext_limbs][N] before ntt_inverse_second.
 bool ks_fused_supported(const DeviceTables &t);
+// How the items of a small batch are split over blocks.  Group g > 0 of the
+// partitions writes its own sums, to partials + (g - 1) * [count][2]
+// [ext_limbs][N], which the second inverse pass adds (PartialSums).
+struct KsSplit {
+  int groups = 1, halves = 1;
+};
+constexpr int kKsMaxGroups = 8;
+KsSplit ks_split(const DeviceTables &t, int parts, int count, int ext_limbs,
+                 bool lazy);
 void launch_ks_inner_product_fused(const DeviceTables &t, const int64_t *ext,
                                    const int64_t *key, int key_chain,
                                    int key_offset, int key_partition0,
@@ -92,7 +117,8 @@ void launch_ks_inner_product_fused(const DeviceTables &t, const int64_t *ext,
                                    int ext_limbs, int moduli_id, bool lazy,
                                    const int64_t *own, int64_t own_stride,
                                    const int *starts, const int *sizes,
-                                   bool lazy_accumulate, hipStream_t stream);
+                                   bool lazy_accumulate, const KsSplit &split,
+                                   int64_t *partials, hipStream_t stream);
 
 // out = mont_mult(a, b) elementwise (src/montgomery/unit.cpp:5-10).
 void launch_mont_mult(const DeviceTables &t, const int64_t *a,
@@ -105,6 +131,20 @@ void launch_mont_mult_broadcast(const DeviceTables &t, const int64_t *a,
                                 const int64_t *b, int64_t *out,
                                 int64_t total_limbs, int limbs, int moduli_id,
                                 hipStream_t stream);
+
+// out = mont(a, b), or with add guard(guard(a + b, 2q), q) (kEwAddReduce),
+// over the polynomials (c, h), h < polys, of `count` texts: polynomial (c, h)
+// of an operand at base + c * text + h * poly words, strides in whole limbs.
+// False when the addresses do not allow it (16-byte alignment, N >= 1024):
+// the caller then works text by text.
+struct TextOpArgs {
+  const int64_t *a, *b;
+  int64_t *out;
+  int64_t a_text, a_poly, b_text, b_poly, o_text, o_poly;
+  int polys, limbs, moduli_id;
+};
+bool launch_text_op(const DeviceTables &t, bool add, const TextOpArgs &a,
+                    int count, hipStream_t stream);
 
 // NTT-form tensor of `count` duo pairs -> trios (src/ckks/core.cpp:284-314).
 void launch_tensor(const DeviceTables &t, const int64_t *a, const int64_t *b,

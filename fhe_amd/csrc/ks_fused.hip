@@ -10,6 +10,8 @@
 // the first (low-bit) pass of the inverse NTT on both accumulators before a
 // single write.  Each coefficient sees the reference's exact sequence of
 // butterflies, products and guards.
+#include <algorithm>
+
 #include "kernels.h"
 #include "ks_tile.h"
 
@@ -33,8 +35,15 @@ __device__ __forceinline__ void ks_block(const KsArgs &a, F &&item) {
     w = int64_t(blockIdx.x & 7) * per + (blockIdx.x >> 3);
   }
   const int ct = int(w % a.count);
-  const int64_t rest = w / a.count;
-  item(ct, int(rest % tiles), a.limb0 + int(rest / tiles));
+  int64_t rest = w / a.count;
+  const int sub = int(rest % (a.groups * a.halves));
+  rest /= a.groups * a.halves;
+  const int group = sub / a.halves;
+  // partitions [p0, p1) of the group
+  const int p0 = group * a.parts / a.groups;
+  const int p1 = (group + 1) * a.parts / a.groups;
+  item(KsBatchAddr<LOGN>(a, ct, group), int(rest % tiles),
+       a.limb0 + int(rest / tiles), p0, p1, sub % a.halves);
 }
 
 // One arithmetic per launch, over a run of extended limbs of its class.
@@ -42,24 +51,24 @@ template <int LOGN, int A>
 __global__ __launch_bounds__(kBlock, A == kF64 ? kKsF64Waves : 2)
 void ks_inner_product_r16_kernel(KsArgs a, DeviceTables t) {
   __shared__ int64_t lds[kR16Lds<r16_low_bits(LOGN)>];
-  ks_block<LOGN>(a, [&](int ct, int tile, int i) {
-    const KsBatchAddr<LOGN> ad(a, ct);
-    ks_item_tile<LOGN, A>(ad, t, lds, tile, i);
+  ks_block<LOGN>(a, [&](const auto &ad, int tile, int i, int p0, int p1,
+                        int half) {
+    ks_item_tile<LOGN, A, true>(ad, t, lds, tile, i, p0, p1, half);
   });
 }
 
 // The lazy arithmetic of each limb's class chosen per block: one launch for
-// all limbs.
-template <int LOGN>
+// all limbs.  BOTH: both key halves per block.
+template <int LOGN, bool BOTH>
 __global__ __launch_bounds__(kBlock, 2) void ks_inner_product_mixed_kernel(
     KsArgs a, DeviceTables t) {
   __shared__ int64_t lds[kR16Lds<r16_low_bits(LOGN)>];
-  ks_block<LOGN>(a, [&](int ct, int tile, int i) {
-    const KsBatchAddr<LOGN> ad(a, ct);
+  ks_block<LOGN>(a, [&](const auto &ad, int tile, int i, int p0, int p1,
+                        int half) {
     if (t.q[a.moduli_id + i] < kF64Bound)
-      ks_item_tile<LOGN, kF64>(ad, t, lds, tile, i);
+      ks_item_tile<LOGN, kF64, BOTH>(ad, t, lds, tile, i, p0, p1, half);
     else
-      ks_item_tile<LOGN, kLazyLarge>(ad, t, lds, tile, i);
+      ks_item_tile<LOGN, kLazyLarge, BOTH>(ad, t, lds, tile, i, p0, p1, half);
   });
 }
 
@@ -378,6 +387,26 @@ void launch_staged_modup(const DeviceTables &t, const int64_t *x,
   });
 }
 
+// A batch whose items fill fewer blocks than there are CUs is split further:
+// the partitions into groups until they do, and, where even that leaves most
+// of the chip idle, one block per key half.  The line is at one block per CU
+// (measured per launch sequence: N = 2^14, 36 blocks, 142 -> 109 us; N = 2^16,
+// 464 blocks, 423 -> 468 us with three groups, whose sums then cost more than
+// the idle slots did).
+constexpr int64_t kSplitTarget = 256;
+
+KsSplit ks_split(const DeviceTables &t, int parts, int count, int ext_limbs,
+                 bool lazy) {
+  const int64_t blocks = (int64_t(ext_limbs) * count) << (t.log_n - 12);
+  KsSplit s;
+  if (!lazy || blocks >= kSplitTarget)
+    return s;
+  s.groups = int(std::min<int64_t>(std::min(parts, kKsMaxGroups),
+                                   (kSplitTarget + blocks - 1) / blocks));
+  s.halves = blocks * s.groups <= kSplitTarget ? 2 : 1;
+  return s;
+}
+
 void launch_ks_inner_product_fused(const DeviceTables &t, const int64_t *ext,
                                    const int64_t *key, int key_chain,
                                    int key_offset, int key_partition0,
@@ -385,7 +414,8 @@ void launch_ks_inner_product_fused(const DeviceTables &t, const int64_t *ext,
                                    int ext_limbs, int moduli_id, bool lazy,
                                    const int64_t *own, int64_t own_stride,
                                    const int *starts, const int *sizes,
-                                   bool lazy_accumulate, hipStream_t stream) {
+                                   bool lazy_accumulate, const KsSplit &split,
+                                   int64_t *partials, hipStream_t stream) {
   const int tiles = int((int64_t(1) << t.log_n) >> 12);
   const int64_t blocks = int64_t(ext_limbs) * tiles * count;
   KsArgs a{};
@@ -402,6 +432,9 @@ void launch_ks_inner_product_fused(const DeviceTables &t, const int64_t *ext,
   a.own = own;
   a.own_stride = own_stride;
   a.lazy_acc = lazy_accumulate ? 1 : 0;
+  a.groups = split.groups;
+  a.halves = split.halves;
+  a.partials = partials;
   for (int p = 0; p < parts && p < kMaxFusedParts; p++) {
     a.start[p] = own ? starts[p] : 0;
     a.size[p] = own ? sizes[p] : 0;
@@ -410,15 +443,17 @@ void launch_ks_inner_product_fused(const DeviceTables &t, const int64_t *ext,
     constexpr int LOGN = decltype(logn)::value;
     auto launch = [&](auto *kernel, int l, int n) {
       a.limb0 = l;
-      const int64_t b = blocks / ext_limbs * n;
+      const int64_t b = blocks / ext_limbs * n * a.groups * a.halves;
       a.swizzle = b % 8 == 0 ? 1 : 0;
       hipLaunchKernelGGL(kernel, dim3(unsigned(b)), dim3(kBlock), 0, stream, a,
                          t);
     };
     if (!lazy)
       launch(ks_inner_product_r16_kernel<LOGN, kExact>, 0, ext_limbs);
+    else if (blocks < kSplitBlocks && split.halves == 2)
+      launch(ks_inner_product_mixed_kernel<LOGN, false>, 0, ext_limbs);
     else if (blocks < kSplitBlocks)
-      launch(ks_inner_product_mixed_kernel<LOGN>, 0, ext_limbs);
+      launch(ks_inner_product_mixed_kernel<LOGN, true>, 0, ext_limbs);
     else
       for_class_runs(t, moduli_id, ext_limbs, [&](int l, int n, bool small) {
         if (small)

@@ -35,6 +35,11 @@ struct KsArgs {
   int key_partition0;  // key partition index of the ciphertext's partition 0
   int limb0;           // first extended limb of the launch
   int swizzle;
+  // splits of an item over blocks: `groups` ranges of partitions, group g > 0
+  // writing its sums to partials + (g - 1) * [count][2][ext_limbs][N], and
+  // with halves = 2 one block per key half
+  int groups, halves;
+  int64_t *partials;
   // NTT form of the key-switched polynomial, when the caller has it: limb i
   // of ciphertext c at own + c * own_stride + i * N.  The extended limbs of a
   // partition's own primes are that polynomial's limbs, so their transforms
@@ -71,10 +76,12 @@ struct KsArgs {
 // accumulators are canonicalized after the inverse transform.
 // LOGN: log2 N.
 // OPAQUE: the tile runs inside a persistent loop (opaque_tid).
-template <int LOGN, int A, class Addr, bool OPAQUE = false>
+// p0, p1: the partitions to sum.  BOTH: both key halves, else half `half`.
+template <int LOGN, int A, bool BOTH, class Addr, bool OPAQUE = false>
 __device__ __forceinline__ void ks_item_tile(const Addr &a,
                                              const DeviceTables &t,
-                                             int64_t *lds, int tile, int i) {
+                                             int64_t *lds, int tile, int i,
+                                             int p0, int p1, int half) {
   constexpr int L = r16_low_bits(LOGN);
   const int64_t n = int64_t(1) << t.log_n;
   const int p = a.moduli_id + i;
@@ -92,7 +99,7 @@ __device__ __forceinline__ void ks_item_tile(const Addr &a,
   const int64_t qq = int64_t(f.q);
 
   R16Value<A> acc0[16], acc1[16], v[16];
-  for (int pp = 0; pp < a.parts; pp++) {
+  for (int pp = p0; pp < p1; pp++) {
     int64_t w[16];
     // block-uniform: every thread of the block has the same (i, pp)
     if (a.is_own(pp, i)) {
@@ -119,7 +126,8 @@ __device__ __forceinline__ void ks_item_tile(const Addr &a,
       r16_forward_settle<A>(v, f);
     }
     // v[m] is now the NTT value at coefficient off + 16 r + m
-    const int64_t *k0 = a.key_tile(pp, i, off) + 16 * r;
+    const int64_t *k0 = a.key_tile(pp, i, off) + 16 * r +
+                        (BOTH ? 0 : int64_t(half) * a.key_chain * n);
     const int64_t *k1 = k0 + int64_t(a.key_chain) * n;
     if constexpr (A == kF64) {
       // plain products: the sums carry the key's Montgomery factor R, which
@@ -127,15 +135,18 @@ __device__ __forceinline__ void ks_item_tile(const Addr &a,
 #pragma unroll
       for (int m = 0; m < 16; m++) {
         const double x0 = f64_mul(v[m], f64_from_int(k0[m]), f.f);
-        const double x1 = f64_mul(v[m], f64_from_int(k1[m]), f.f);
-        acc0[m] = pp == 0 ? x0 : acc0[m] + x0;
-        acc1[m] = pp == 0 ? x1 : acc1[m] + x1;
+        acc0[m] = pp == p0 ? x0 : acc0[m] + x0;
+        if (BOTH) {
+          const double x1 = f64_mul(v[m], f64_from_int(k1[m]), f.f);
+          acc1[m] = pp == p0 ? x1 : acc1[m] + x1;
+        }
       }
-    } else if (pp == 0) {
+    } else if (pp == p0) {
 #pragma unroll
       for (int m = 0; m < 16; m++) {
         acc0[m] = mont_mult_u(v[m], k0[m], f.q, f.k);
-        acc1[m] = mont_mult_u(v[m], k1[m], f.q, f.k);
+        if (BOTH)
+          acc1[m] = mont_mult_u(v[m], k1[m], f.q, f.k);
       }
     } else if (A == kLazyLarge && a.lazy_acc) {
       // sums kept below 2q (one conditional subtraction of 2q): the lazy
@@ -144,8 +155,9 @@ __device__ __forceinline__ void ks_item_tile(const Addr &a,
       for (int m = 0; m < 16; m++) {
         acc0[m] = guard_u(add64(mont_mult_u(v[m], k0[m], f.q, f.k), acc0[m]),
                           f.q2);
-        acc1[m] = guard_u(add64(mont_mult_u(v[m], k1[m], f.q, f.k), acc1[m]),
-                          f.q2);
+        if (BOTH)
+          acc1[m] = guard_u(
+              add64(mont_mult_u(v[m], k1[m], f.q, f.k), acc1[m]), f.q2);
       }
     } else {
 #pragma unroll
@@ -153,9 +165,11 @@ __device__ __forceinline__ void ks_item_tile(const Addr &a,
         acc0[m] = guard_u(
             guard_u(add64(mont_mult_u(v[m], k0[m], f.q, f.k), acc0[m]), f.q2),
             qq);
-        acc1[m] = guard_u(
-            guard_u(add64(mont_mult_u(v[m], k1[m], f.q, f.k), acc1[m]), f.q2),
-            qq);
+        if (BOTH)
+          acc1[m] = guard_u(
+              guard_u(add64(mont_mult_u(v[m], k1[m], f.q, f.k), acc1[m]),
+                      f.q2),
+              qq);
       }
     }
   }
@@ -164,6 +178,8 @@ __device__ __forceinline__ void ks_item_tile(const Addr &a,
   r16_prime<A, true>(g, t, p);
   int64_t *d0 = a.acc(i, off);
   int64_t *d1 = d0 + int64_t(a.ext_limbs) * n;
+  if (!BOTH && half)
+    d0 = d1;
   auto inverse = [&](R16Value<A> (&x)[16], int64_t *d) {
     if constexpr (A == kF64) {
 #pragma unroll
@@ -178,16 +194,23 @@ __device__ __forceinline__ void ks_item_tile(const Addr &a,
       d[r16_point<L, false>(r, m)] = __builtin_bit_cast(int64_t, x[m]);
   };
   inverse(acc0, d0);
-  inverse(acc1, d1);
+  if (BOTH)
+    inverse(acc1, d1);
 }
 
 // Addressing of ciphertext ct of a batch at one moduli_id (KsArgs).
 template <int LOGN> struct KsBatchAddr {
   const KsArgs &a;
   int ct;
+  int64_t *sums;
   int parts, ext_limbs, moduli_id, key_chain, lazy_acc;
-  __device__ KsBatchAddr(const KsArgs &args, int c)
-      : a(args), ct(c), parts(args.parts),
+  __device__ KsBatchAddr(const KsArgs &args, int c, int group)
+      : a(args), ct(c),
+        sums(group == 0
+                 ? args.acc
+                 : args.partials + ((int64_t(group - 1) * args.count * 2 *
+                                     args.ext_limbs)
+                                    << LOGN)), parts(args.parts),
         ext_limbs(args.ext_limbs), moduli_id(args.moduli_id),
         key_chain(args.key_chain), lazy_acc(args.lazy_acc) {}
   __device__ bool is_own(int pp, int i) const {
@@ -206,7 +229,7 @@ template <int LOGN> struct KsBatchAddr {
            ((int64_t(2 * kp) * a.key_chain + a.key_offset + i) << LOGN) + off;
   }
   __device__ int64_t *acc(int i, int64_t off) const {
-    return a.acc + ((int64_t(ct) * 2 * a.ext_limbs + i) << LOGN) + off;
+    return sums + ((int64_t(ct) * 2 * a.ext_limbs + i) << LOGN) + off;
   }
 };
 

@@ -43,6 +43,9 @@ struct PassArgs {
   // radix-16 passes: polynomials from `split` on are read from src2
   const int64_t *src2 = nullptr;
   int64_t split = 0;
+  // radix-16 passes: words between the source's polynomials (0: dense)
+  int64_t src_stride = 0;
+  PartialSums more = {};
 };
 
 template <bool INV>
@@ -171,7 +174,8 @@ __global__ __launch_bounds__(kBlock) void ntt_radix16_kernel(
   const int64_t *src =
       a.src2 && poly >= a.split
           ? a.src2 + (((poly - a.split) * a.limbs + l) << t.log_n)
-          : a.src + limb;
+      : a.src_stride ? a.src + poly * a.src_stride + (int64_t(l) << t.log_n)
+                     : a.src + limb;
   int64_t *dst = a.dst + limb;
   const int p = a.moduli_id + l;
   if constexpr (!LAZY) {
@@ -182,14 +186,17 @@ __global__ __launch_bounds__(kBlock) void ntt_radix16_kernel(
         a.zero && poly % a.zero_period == a.zero_period - 1
             ? a.zero + (poly / a.zero_period) * a.limbs + l
             : nullptr;
+    const int64_t *more = a.more.data + limb;
     // (the generic second pass of N = 2^17 takes no doubles)
     if (r16_supported(t.log_n) && t.q[p] < kF64Bound)
       r16_limb_pass<L, INV, COLS, kF64>(src, dst, p, tile, a.low_bit, a.pre,
-                                        a.post, a.last != 0, t, lds, zero);
+                                        a.post, a.last != 0, t, lds, zero,
+                                        more, a.more.stride, a.more.count);
     else
       r16_limb_pass<L, INV, COLS, kLazyLarge>(src, dst, p, tile, a.low_bit,
                                               a.pre, a.post, a.last != 0, t,
-                                              lds, zero);
+                                              lds, zero, more, a.more.stride,
+                                              a.more.count);
   }
 }
 
@@ -280,6 +287,25 @@ void ntt_forward(const DeviceTables &t, const int64_t *src, int64_t *dst,
   }
 }
 
+bool ntt_forward_strided(const DeviceTables &t, const int64_t *src,
+                         int64_t src_stride, int64_t *dst, int64_t polys,
+                         int limbs, int moduli_id, const int64_t *pre,
+                         hipStream_t stream) {
+  if (!r16_supported(t.log_n))
+    return false;
+  int l1, l2;
+  split_bits(t.log_n, false, l1, l2);
+  PassArgs a{src,     dst,       (polys * limbs) << (t.log_n - l1),
+             limbs,   moduli_id, t.log_n - l1,
+             l1,      pre,       kInttRaw,
+             0,       false,     nullptr,
+             1};
+  a.src_stride = src_stride;
+  launch_pass<false>(a, t, stream);
+  ntt_forward_second(t, dst, dst, polys * limbs, limbs, moduli_id, stream);
+  return true;
+}
+
 void ntt_forward_pair(const DeviceTables &t, const int64_t *x,
                       const int64_t *y, int64_t *dst, int64_t total_limbs,
                       int limbs, int moduli_id, const int64_t *pre,
@@ -362,13 +388,14 @@ void ntt_forward_second(const DeviceTables &t, const int64_t *src,
 void ntt_inverse_second(const DeviceTables &t, const int64_t *src,
                         int64_t *dst, int64_t total_limbs, int limbs,
                         int moduli_id, int post, hipStream_t stream,
-                        LazySpec lazy) {
+                        LazySpec lazy, PartialSums more) {
   int l1, l2;
   split_bits(t.log_n, true, l1, l2);
   PassArgs a{src,   dst,      total_limbs << (t.log_n - l2),
              limbs, moduli_id, l1,
              l2,    nullptr,   post,
              1,     lazy.on, lazy.zero, lazy.zero_period};
+  a.more = more;
   launch_pass<true>(a, t, stream);
 }
 

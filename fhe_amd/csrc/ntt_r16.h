@@ -380,6 +380,8 @@ __device__ __forceinline__ void r16_exchange_words(V (&x)[16], uint32_t *lds,
 // is the InttPost epilogue; last = the pass completes a forward transform.
 // zero (lazy inverse): a flag word of the limb, cleared by the first pass and
 // set by the last one where a canonical result is zero (repair_zero_limb).
+// more (lazy second inverse pass): this limb of the first of more_count
+// buffers, more_stride words apart, that are added to the source.
 // OPAQUE: the pass runs inside a persistent loop (opaque_tid).
 template <int L, bool INV, bool COLS, int A, bool OPAQUE = false>
 __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
@@ -388,7 +390,10 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
                                               const int64_t *pre, int post,
                                               bool last, const DeviceTables &t,
                                               int64_t *lds,
-                                              uint32_t *zero = nullptr) {
+                                              uint32_t *zero = nullptr,
+                                              const int64_t *more = nullptr,
+                                              int64_t more_stride = 0,
+                                              int more_count = 0) {
   const int tid = OPAQUE ? opaque_tid() : int(threadIdx.x);
   constexpr int T = 1 << (L - 4), C = 4096 >> L;
   const int c = COLS ? (tid & (C - 1)) : (tid >> (L - 4));
@@ -434,7 +439,16 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
 #pragma unroll
       for (int m = 0; m < 16; m++) {
         v[m] = __longlong_as_double(w[m]);
-        if (INV)
+      }
+      if (INV) {
+        for (int g = 0; g < more_count; g++)
+#pragma unroll
+          for (int m = 0; m < 16; m++)
+            v[m] += __longlong_as_double(
+                more[g * more_stride + base +
+                     (int64_t(r16_point<L, cols_load>(r, m)) << b)]);
+#pragma unroll
+        for (int m = 0; m < 16; m++)
           v[m] = f64_center(v[m], s.f);
       }
     }
@@ -442,6 +456,15 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
 #pragma unroll
     for (int m = 0; m < 16; m++)
       v[m] = pre ? load_product<A>(w[m], pre[p], s.q, s.k) : w[m];
+    if (A == kLazyLarge && INV && !first_pass)
+      for (int g = 0; g < more_count; g++)
+#pragma unroll
+        for (int m = 0; m < 16; m++)
+          v[m] = guard_u(
+              add64(v[m], more[g * more_stride + base +
+                               (int64_t(r16_point<L, cols_load>(r, m))
+                                << b)]),
+              s.q2);
   }
   if (INV && !COLS)
     r16_exchange<L, true, !COLS>(v, lds, c, r);

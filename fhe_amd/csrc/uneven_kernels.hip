@@ -220,8 +220,8 @@ __global__ __launch_bounds__(kBlock, 2) void uneven_ks_kernel(UnevenKsArgs a,
   for (UnitWalk u(a.list); u.w < u.end; u.w += u.step) {
     const uint32_t unit = a.list.units[u.w];
     const UnevenKsAddr ad(a, unit_ct(unit), t.log_n);
-    ks_item_tile<16, A, UnevenKsAddr, true>(
-        ad, t, lds, unit_tile(unit), unit_limb(unit));
+    ks_item_tile<16, A, true, UnevenKsAddr, true>(
+        ad, t, lds, unit_tile(unit), unit_limb(unit), 0, ad.parts, 0);
   }
 }
 

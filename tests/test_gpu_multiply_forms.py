@@ -50,3 +50,57 @@ def test_forms(gpu_lib, log_n, alpha):
                 arr.free()
         for arr in [key] + list(texts.values()):
             arr.free()
+
+
+@pytest.mark.parametrize("log_n,alpha,shift", [(13, 1, 0), (14, 1, 1),
+                                               (15, 2, 0)])
+def test_batches_equal_single_texts(gpu_lib, log_n, alpha, shift):
+    """Plaintext products, encryption and decryption of a batch against each
+    text alone; shift: operands 8 bytes past a 16-byte boundary."""
+    count, level = 3, 2
+    with fhe_amd.Context(log_n, alpha) as ctx:
+        n, full = ctx.n, ctx.info["full_level"]
+        rng = np.random.Generator(np.random.PCG64(6))
+        mid = full - level
+        limbs = ctx.limbs_at(mid)
+        made = []
+
+        class At:
+            """A device array of `shape` starting `shift` words in."""
+
+            def __init__(self, shape, host=None):
+                whole = ctx.array((int(np.prod(shape)) + 2,))
+                made.append(whole)
+                self.whole, self.shape = whole, shape
+                self.ptr = type(whole.ptr)(whole.ptr.value + 8 * shift)
+                if host is not None:
+                    whole.upload_at(np.ascontiguousarray(host), shift)
+
+            def download(self):
+                flat = self.whole.download()
+                return flat[shift:shift + int(np.prod(self.shape))].reshape(
+                    self.shape)
+
+        ct = uniform(rng, ctx.primes, mid, (count, 2, limbs, n))
+        pt = uniform(rng, ctx.primes, mid, (count, limbs, n))
+        keys = uniform(rng, ctx.primes, 0, (2, ctx.chain_count, n))
+        small = rng.integers(-4, 5, (3, count, n))
+
+        def run(sel):
+            k = len(sel)
+            c, p = At((k, 2, limbs, n), ct[sel]), At((k, limbs, n), pt[sel])
+            pk, sk = At(keys.shape, keys), At(keys.shape[1:], keys[0])
+            u, e0, e1 = (At((k, n), x[sel]) for x in small)
+            prod = At((k, 2, limbs - 1, n))
+            enc, dec = At((k, 2, limbs, n)), At((k, limbs, n))
+            ctx.multiply_plain(c, level, 0, p, level, 0, prod)
+            ctx.encrypt_pk(p, pk, 0, u, e0, e1, enc, mid)
+            ctx.decrypt(c, sk, 0, dec, mid)
+            return [x.download() for x in (prod, enc, dec)]
+
+        whole = run(list(range(count)))
+        for i in range(count):
+            for w, one in zip(whole, run([i])):
+                assert np.array_equal(w[i], one[0])
+        for arr in made:
+            arr.free()
