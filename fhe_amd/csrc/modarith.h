@@ -210,6 +210,20 @@ FHE_HD uint64_t shoup_mult_neg(uint64_t y, uint64_t w, uint64_t wq,
   return w * y + mulhi64(wq, y) * nq;
 }
 
+// shoup_mult_neg with the quotient's low partial products dropped: the high
+// word of wq y without the low-by-low product and the carries of the low
+// words of the cross products (three terms below 2^32 each) misses at most
+// two, so the product lies in [0, 4q) (any y < 2^64, q < 2^62).  Two
+// mul_hi and one multiply-add in place of a mul_hi and three multiply-adds.
+FHE_HD uint64_t shoup_short_neg(uint64_t y, uint64_t w, uint64_t wq,
+                                uint64_t nq) {
+  const uint32_t y0 = uint32_t(y), y1 = uint32_t(y >> 32);
+  const uint32_t v0 = uint32_t(wq), v1 = uint32_t(wq >> 32);
+  const uint32_t c0 = uint32_t((uint64_t(v0) * y1) >> 32);
+  const uint32_t c1 = uint32_t((uint64_t(v1) * y0) >> 32);
+  const uint64_t h = uint64_t(v1) * y1 + c0 + c1;
+  return w * y + h * nq;
+}
 
 // Montgomery exit x * R^-1 (src/montgomery/unit.h:25-31): the single-word
 // operand is sign-extended to 128 bits.

@@ -21,9 +21,10 @@
 //               passes of a transform the values stay doubles (in the int64
 //               buffers); the first pass reads integers and the last one
 //               writes integers.
-//   kLazyLarge  Harvey's lazy forms for any q < 2^61: forward values in
-//               [0, 4q) with one conditional subtraction per butterfly,
-//               inverse values in [0, 2q).
+//   kLazyLarge  lazy forms after Harvey for any q < 2^61 on short Shoup
+//               products (shoup_short_neg, in [0, 4q)): forward values in
+//               [0, 8q), inverse values in [0, 4q), one conditional
+//               subtraction of 4q per butterfly.
 // The lazy forms give other representatives of the same residues; they serve
 // stages whose results are canonicalized before anything representative-
 // dependent reads them.
@@ -183,10 +184,10 @@ __device__ __forceinline__ void fwd_bfly(R16Value<A> &x, R16Value<A> &y,
     x = x + p;
   } else {
     const uint64_t w = s.ts[2 * idx], wq = s.ts[2 * idx + 1];
-    const int64_t x0 = guard_u(x, s.q2);
-    const int64_t p = int64_t(shoup_mult_neg(uint64_t(y), w, wq, s.nq));
+    const int64_t x0 = guard_u(x, 2 * s.q2);
+    const int64_t p = int64_t(shoup_short_neg(uint64_t(y), w, wq, s.nq));
     x = add64(x0, p);
-    y = sub64(add64(x0, s.q2), p);
+    y = sub64(add64(x0, 2 * s.q2), p);
   }
 }
 
@@ -202,9 +203,9 @@ __device__ __forceinline__ void inv_bfly(R16Value<A> &x, R16Value<A> &y,
     y = f64_mul(d, s.tf[idx], s.f);
   } else {
     const uint64_t w = s.ts[2 * idx], wq = s.ts[2 * idx + 1];
-    const int64_t d = sub64(add64(x, s.q2), y);
-    x = guard_u(add64(x, y), s.q2);
-    y = int64_t(shoup_mult_neg(uint64_t(d), w, wq, s.nq));
+    const int64_t d = sub64(add64(x, 2 * s.q2), y);
+    x = guard_u(add64(x, y), 2 * s.q2);
+    y = int64_t(shoup_short_neg(uint64_t(d), w, wq, s.nq));
   }
 }
 
@@ -278,14 +279,14 @@ __device__ __forceinline__ void r16_inverse_high(R16Value<A> (&v)[16],
   }
 }
 
-// Bring kLazyLarge forward outputs (below 4q) to [0, 2q).
+// Bring kLazyLarge forward outputs (below 8q) to [0, 2q).
 template <int A>
 __device__ __forceinline__ void r16_forward_settle(R16Value<A> (&v)[16],
                                                    const R16Pass &s) {
   if constexpr (A == kLazyLarge) {
 #pragma unroll
     for (int m = 0; m < 16; m++)
-      v[m] = guard_u(v[m], s.q2);
+      v[m] = guard_u(guard_u(v[m], 2 * s.q2), s.q2);
   }
 }
 
@@ -464,7 +465,7 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
               add64(v[m], more[g * more_stride + base +
                                (int64_t(r16_point<L, cols_load>(r, m))
                                 << b)]),
-              s.q2);
+              2 * s.q2);
   }
   if (INV && !COLS)
     r16_exchange<L, true, !COLS>(v, lds, c, r);
@@ -506,13 +507,14 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
         }
       } else {
         // kLazyLarge needs only the residue: one product with N^-1 R^-1
-        // (the exit folded into the constant) gives it below v q / 2^62 + q
-        // < 2q (v < 2q), which the guard brings to the canonical value
+        // (the exit folded into the constant) of v brought below 2q gives it
+        // below v q / 2^62 + q < 2q, which the guard makes canonical
         const int64_t ninv_exit = mont_exit(ninv, s.q, s.k);
 #pragma unroll
         for (int m = 0; m < 16; m++)
-          v[m] = guard_u(mont_mult_u(v[m], ninv_exit, s.q, s.k),
-                         int64_t(s.q));
+          v[m] = guard_u(
+              mont_mult_u(guard_u(v[m], s.q2), ninv_exit, s.q, s.k),
+              int64_t(s.q));
       }
     }
   }
