@@ -22,13 +22,13 @@ namespace {
 // Waves per SIMD of the kF64 key inner product.
 constexpr int kKsF64Waves = 3;
 
-// Block -> (limb i, tile, ciphertext), ciphertext fastest: the blocks of a
+// Block -> (tile, limb i, ciphertext), ciphertext fastest: the blocks of a
 // key tile run together and share its reads through L2; with swizzle each of
 // the 8 XCDs (blocks are dealt round-robin to XCDs) gets one contiguous
-// range of that order.
+// range of that order.  The tile runs slowest, so that every XCD has its
+// share of the 60-bit limbs, whose items take about three times as long.
 template <int LOGN, class F>
 __device__ __forceinline__ void ks_block(const KsArgs &a, F &&item) {
-  constexpr int tiles = 1 << (LOGN - 12);
   int64_t w = blockIdx.x;
   if (a.swizzle) {
     const int64_t per = int64_t(gridDim.x) >> 3;
@@ -42,8 +42,8 @@ __device__ __forceinline__ void ks_block(const KsArgs &a, F &&item) {
   // partitions [p0, p1) of the group
   const int p0 = group * a.parts / a.groups;
   const int p1 = (group + 1) * a.parts / a.groups;
-  item(KsBatchAddr<LOGN>(a, ct, group), int(rest % tiles),
-       a.limb0 + int(rest / tiles), p0, p1, sub % a.halves);
+  item(KsBatchAddr<LOGN>(a, ct, group), int(rest / a.limbs_here),
+       a.limb0 + int(rest % a.limbs_here), p0, p1, sub % a.halves);
 }
 
 // One arithmetic per launch, over a run of extended limbs of its class.
@@ -443,6 +443,7 @@ void launch_ks_inner_product_fused(const DeviceTables &t, const int64_t *ext,
     constexpr int LOGN = decltype(logn)::value;
     auto launch = [&](auto *kernel, int l, int n) {
       a.limb0 = l;
+      a.limbs_here = n;
       const int64_t b = blocks / ext_limbs * n * a.groups * a.halves;
       a.swizzle = b % 8 == 0 ? 1 : 0;
       hipLaunchKernelGGL(kernel, dim3(unsigned(b)), dim3(kBlock), 0, stream, a,

@@ -33,7 +33,7 @@ struct KsArgs {
   int key_chain;
   int key_offset;      // first key limb aligned with the ciphertext's limb 0
   int key_partition0;  // key partition index of the ciphertext's partition 0
-  int limb0;           // first extended limb of the launch
+  int limb0, limbs_here; // extended limbs of the launch
   int swizzle;
   // splits of an item over blocks: `groups` ranges of partitions, group g > 0
   // writing its sums to partials + (g - 1) * [count][2][ext_limbs][N], and

@@ -154,12 +154,14 @@ __global__ __launch_bounds__(kBlock) void ntt_pass_kernel(PassArgs a,
 // the same registers, and a launch for the few large primes of a chain alone
 // would run its chain of butterflies on a nearly empty chip).
 //
-// Block -> (limb l, tile, polynomial), polynomial fastest so blocks sharing
-// a prime's twiddles run together; with swizzle each of the 8 XCDs (blocks
+// Block -> (tile, limb l, polynomial), polynomial fastest so blocks sharing
+// a tile's twiddles run together; with swizzle each of the 8 XCDs (blocks
 // are dealt round-robin to XCDs) gets one contiguous range of that order.
+// The tile runs slowest, so that every XCD has its share of the 60-bit
+// limbs.
 template <int L, bool INV, bool COLS, bool LAZY>
 __global__ __launch_bounds__(kBlock) void ntt_radix16_kernel(
-    PassArgs a, DeviceTables t, int polys, int tiles_per_limb, int swizzle) {
+    PassArgs a, DeviceTables t, int polys, int swizzle) {
   __shared__ int64_t lds[kR16Lds<L>];
   int64_t w = blockIdx.x;
   if (swizzle) {
@@ -168,8 +170,8 @@ __global__ __launch_bounds__(kBlock) void ntt_radix16_kernel(
   }
   const int64_t poly = w % polys;
   const int64_t rest = w / polys;
-  const int tile = int(rest % tiles_per_limb);
-  const int l = int(rest / tiles_per_limb);
+  const int l = int(rest % a.limbs);
+  const int tile = int(rest / a.limbs);
   const int64_t limb = (poly * a.limbs + l) << t.log_n;
   const int64_t *src =
       a.src2 && poly >= a.split
@@ -230,11 +232,11 @@ void launch_r16_pass(const PassArgs &a, const DeviceTables &t,
   if (a.lazy)
     hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, true>),
                        dim3(unsigned(blocks)), dim3(kBlock), 0, stream, a, t,
-                       polys, tiles, swizzle);
+                       polys, swizzle);
   else
     hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, false>),
                        dim3(unsigned(blocks)), dim3(kBlock), 0, stream, a, t,
-                       polys, tiles, swizzle);
+                       polys, swizzle);
 }
 
 template <bool INV>
