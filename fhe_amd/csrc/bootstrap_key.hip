@@ -188,7 +188,7 @@ void decompose_full(fhe_context *ctx, int count, int m, const int64_t *src,
   const int ext_limbs = P.limbs_at(m) + P.alpha;
   const int parts = int(P.partitions(m, m).size());
   ctx->ks_decompose(count, m, m, src, src_stride, dec);
-  const fhe::LazySpec lazy{ctx->lazy_key_switch};
+  const fhe::LazySpec lazy{ctx->lazy_transforms()};
   ctx->stage("bk_ntt_pass_low(ext)", [&] {
     fhe::ntt_forward_second(ctx->tables, dec, dec,
                             int64_t(count) * parts * ext_limbs, ext_limbs, m,

@@ -783,7 +783,9 @@ struct fhe_context {
     const int64_t *cst = modup_constants(moduli_id, key_moduli_id);
     const int stride = params.ks_stride(moduli_id);
     const int np = int(parts.size());
-    const fhe::LazySpec lazy{lazy_key_switch};
+    // exact throughout where the second pass is (N > 2^16): its butterflies
+    // take values below 2q, the lazy first pass gives up to 8q
+    const fhe::LazySpec lazy{lazy_transforms()};
     int max_size = 0;
     bool is_signed[fhe::kMaxFusedParts] = {};
     std::vector<int> starts(np), sizes(np);
@@ -807,7 +809,7 @@ struct fhe_context {
                                  limbs, moduli_id, starts.data(), sizes.data(),
                                  is_signed, np, cst, stride,
                                  params.ks_ext_shoup_offset(moduli_id),
-                                 lazy_key_switch, skip_own, stream);
+                                 lazy.on, skip_own, stream);
       });
       return;
     }
@@ -820,7 +822,7 @@ struct fhe_context {
                           params.ks_ext_shoup_offset(moduli_id),
                           !signed_input &&
                               params.modup_non_negative(moduli_id, parts[p]),
-                          lazy_key_switch && !signed_input, stream);
+                          lazy.on && !signed_input, stream);
       });
     stage("ntt_pass_high(ext)", [&] {
       fhe::ntt_forward_first(tables, ext, ext, int64_t(count) * np * ext_limbs,

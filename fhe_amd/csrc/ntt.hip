@@ -189,8 +189,7 @@ __global__ __launch_bounds__(kBlock) void ntt_radix16_kernel(
             ? a.zero + (poly / a.zero_period) * a.limbs + l
             : nullptr;
     const int64_t *more = a.more.data + limb;
-    // (the generic second pass of N = 2^17 takes no doubles)
-    if (r16_supported(t.log_n) && t.q[p] < kF64Bound)
+    if (t.q[p] < kF64Bound)
       r16_limb_pass<L, INV, COLS, kF64>(src, dst, p, tile, a.low_bit, a.pre,
                                         a.post, a.last != 0, t, lds, zero,
                                         more, a.more.stride, a.more.count);
@@ -229,7 +228,10 @@ void launch_r16_pass(const PassArgs &a, const DeviceTables &t,
   const int tiles = int(int64_t(1) << (t.log_n - 12));
   const int64_t blocks = total_limbs * tiles;
   const int swizzle = blocks % 8 == 0 ? 1 : 0;
-  if (a.lazy)
+  // the lazy forms hand doubles or values up to 8q to the other pass, so both
+  // have to be lazy: the 8-bit pass of N = 2^17, whose other pass is the
+  // generic exact one, stays exact
+  if (a.lazy && r16_supported(t.log_n))
     hipLaunchKernelGGL((ntt_radix16_kernel<L, INV, COLS, true>),
                        dim3(unsigned(blocks)), dim3(kBlock), 0, stream, a, t,
                        polys, swizzle);
