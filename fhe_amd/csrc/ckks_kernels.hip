@@ -94,6 +94,10 @@ __global__ __launch_bounds__(kBlock) void text_op_kernel(TextOpArgs a,
   store4(a.out + c * a.o_text + h * a.o_poly + at, x);
 }
 
+// SIGNED: the operands may be negative (exact transforms of signed inputs,
+// texts given in NTT form); the products and guards are then the reference's
+// signed ones.
+template <bool SIGNED>
 __global__ __launch_bounds__(kBlock) void tensor_kernel(
     const int64_t *a, const int64_t *b, int64_t *trio, int64_t total,
     int limbs, int moduli_id, DeviceTables t) {
@@ -110,11 +114,14 @@ __global__ __launch_bounds__(kBlock) void tensor_kernel(
   const int64_t *bc = b + c * 2 * poly + r;
   int64_t *z = trio + c * 3 * poly + r;
   const int64_t a0 = ac[0], a1 = ac[poly], b0 = bc[0], b1 = bc[poly];
-  z[0] = mont_mult_u(a0, b0, q, k);
-  const int64_t z1 = mont_mult_u(a0, b1, q, k);
-  const int64_t z3 = mont_mult_u(a1, b0, q, k);
-  z[poly] = guard_u(guard_u(add64(z1, z3), q2), int64_t(q));
-  z[2 * poly] = mont_mult_u(a1, b1, q, k);
+  auto product = [&](int64_t x, int64_t y) {
+    return SIGNED ? mont_mult(x, y, q, k) : mont_mult_u(x, y, q, k);
+  };
+  z[0] = product(a0, b0);
+  const int64_t z13 = add64(product(a0, b1), product(a1, b0));
+  z[poly] = SIGNED ? guard(guard(z13, q2), int64_t(q))
+                   : guard_u(guard_u(z13, q2), int64_t(q));
+  z[2 * poly] = product(a1, b1);
 }
 
 // One thread per (ciphertext, coefficient): Garner digits of the partition
@@ -553,10 +560,12 @@ bool launch_text_op(const DeviceTables &t, bool add, const TextOpArgs &a,
 
 void launch_tensor(const DeviceTables &t, const int64_t *a, const int64_t *b,
                    int64_t *trio, int count, int limbs, int moduli_id,
-                   hipStream_t stream) {
+                   bool non_negative, hipStream_t stream) {
   const int64_t total = (int64_t(count) * limbs) << t.log_n;
-  hipLaunchKernelGGL(tensor_kernel, dim3(grid_for(total)), dim3(kBlock), 0,
-                     stream, a, b, trio, total, limbs, moduli_id, t);
+  hipLaunchKernelGGL(non_negative ? tensor_kernel<false>
+                                  : tensor_kernel<true>,
+                     dim3(grid_for(total)), dim3(kBlock), 0, stream, a, b,
+                     trio, total, limbs, moduli_id, t);
 }
 
 void launch_modup(const DeviceTables &t, const int64_t *x, int64_t x_stride,

@@ -383,8 +383,9 @@ void hmult_relin_into(fhe_context *ctx, int count, int moduli_id,
                          ctx->tables.r2, ctx->stream, lazy);
     });
     ctx->stage("tensor", [&] {
+      // only the lazy transforms' values are known to be non-negative
       fhe::launch_tensor(ctx->tables, x, y, trio, count, limbs, moduli_id,
-                         ctx->stream);
+                         lazy.on && !a_ntt && !b_ntt, ctx->stream);
     });
     // relinearize: to_intt of all three, key switch of the third
     ctx->stage("intt(trio)", [&] {
@@ -504,7 +505,7 @@ static void multiply_texts(fhe_context *ctx, int count, const int64_t *a,
   if (b_polys == 2) {
     // CKKSCore::multiply / square (src/ckks/core.cpp:284-343)
     ctx->stage("tensor", [&] {
-      fhe::launch_tensor(ctx->tables, ap, bp, prod, count, limbs, mid,
+      fhe::launch_tensor(ctx->tables, ap, bp, prod, count, limbs, mid, false,
                          ctx->stream);
     });
   } else {

@@ -149,7 +149,7 @@ bool launch_text_op(const DeviceTables &t, bool add, const TextOpArgs &a,
 // NTT-form tensor of `count` duo pairs -> trios (src/ckks/core.cpp:284-314).
 void launch_tensor(const DeviceTables &t, const int64_t *a, const int64_t *b,
                    int64_t *trio, int count, int limbs, int moduli_id,
-                   hipStream_t stream);
+                   bool non_negative, hipStream_t stream);
 
 // Garner digits of one partition and exact basis extension to all
 // limbs + alpha primes (src/ckks/core_key_switch.cpp:21-108).  x: INTT-form

@@ -478,8 +478,9 @@ __global__ __launch_bounds__(kBlock) void repair_zero_kernel(RepairArgs a,
         out[j] = 0;
       return;
     }
+    // the exact transforms of signed inputs may hold negative values
     for (int j = threadIdx.x; j < n; j += kBlock)
-      mine[j] = mont_mult_u(x[0][j], x[1][j], t.q[p], t.k[p]);
+      mine[j] = mont_mult(x[0][j], x[1][j], t.q[p], t.k[p]);
     __syncthreads();
     z = mine;
   } else {
