@@ -16,14 +16,43 @@
 // 2^40), so the fused multiply-add returns it exactly, and so does the last
 // sum.  For |y| <= 2^47 the quotient's error is below 0.55.
 //
-// Transforms (ntt_r16.h) need no reductions in between: forward values grow
-// by less than 0.55 q a stage; inverse sums double, 2^8 in a pass, and every
-// pass reduces or centres its inputs first, so that products see |y| <= 2^50.
+// Transforms (ntt_r16.h) need no reductions in between: forward values, loaded
+// below 2^47, grow by less than 0.55 q a stage; inverse sums double, 2^8 in a
+// pass, and every inverse pass starts from values centred to q + 2^32 or less
+// in magnitude (f64_load_centred, f64_center), so that products see
+// |y| <= 2^50 + 2^40.
 #pragma once
 
 #include "device.h"
 
 namespace fhe {
+
+// Whether one of 16 integers is negative or at least 2q + 2^32 (at most 4q,
+// for q >= 2^31; smaller primes answer yes always).  Decided on the high
+// words: half an instruction a value, and lazy residues, below 2q, never pass
+// for wider ones.
+__device__ __forceinline__ bool beyond_lazy(const int64_t (&v)[16],
+                                            uint64_t q) {
+  uint32_t top = 0;
+#pragma unroll
+  for (int i = 0; i < 16; i++)
+    top = max(top, uint32_t(uint64_t(v[i]) >> 32));
+  return top > uint32_t((2 * q - 1) >> 32) || q < (uint64_t(1) << 31);
+}
+
+// Replaces 16 representatives by residues in [0, 2q) where beyond_lazy.  One
+// at a time: the rare case takes no registers from the usual one.
+__device__ __forceinline__ void load_residues(int64_t (&v)[16], uint64_t q,
+                                              uint64_t k, int64_t r2) {
+  if (beyond_lazy(v, q)) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int64_t y = mont_exit(mont_mult(r2, v[i], q, k), q, k);
+      v[i] = y < 0 ? y + int64_t(q) : y;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
 
 struct F64Mod {
   double q, qi; // the prime and its rounded reciprocal
@@ -94,6 +123,27 @@ __device__ __forceinline__ void f64_load(const int64_t (&v)[16],
 #pragma unroll
     for (int i = 0; i < 16; i++)
       x[i] = f64_from_int(v[i]);
+  }
+}
+
+// Any int64's residue in about [-q/2, q/2].
+__device__ __forceinline__ double f64_center_any(int64_t v, const F64Mod &m) {
+  return f64_center(f64_from_any(v, m), m);
+}
+
+// Doubles of 16 representatives within q + 2^32 of zero: lazy residues less
+// q, others centred.
+__device__ __forceinline__ void f64_load_centred(const int64_t (&v)[16],
+                                                 double (&x)[16], uint64_t q,
+                                                 const F64Mod &m) {
+  if (beyond_lazy(v, q)) {
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+      x[i] = f64_center_any(v[i], m);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+      x[i] = f64_from_int(v[i]) - m.q;
   }
 }
 

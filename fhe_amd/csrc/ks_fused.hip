@@ -19,11 +19,6 @@ namespace fhe {
 
 namespace {
 
-// Waves per SIMD of the kF64 key inner product (168 registers; 1.90 ms at 32
-// Gold ciphertexts against 1.96 ms with two waves and 208 registers, both with
-// the 60-bit limbs' launch).
-constexpr int kKsF64Waves = 3;
-
 // Block -> (tile, limb i, ciphertext), ciphertext fastest: the blocks of a
 // key tile run together and share its reads through L2; with swizzle each of
 // the 8 XCDs (blocks are dealt round-robin to XCDs) gets one contiguous
@@ -48,10 +43,12 @@ __device__ __forceinline__ void ks_block(const KsArgs &a, F &&item) {
        a.limb0 + int(rest % a.limbs_here), p0, p1, sub % a.halves);
 }
 
-// One arithmetic per launch, over a run of extended limbs of its class.
+// One arithmetic per launch, over a run of extended limbs of its class.  Two
+// waves per SIMD: with three the kF64 form keeps part of its accumulators in
+// scratch memory (32 Gold HMults 8.04 against 7.60 ms).
 template <int LOGN, int A>
-__global__ __launch_bounds__(kBlock, A == kF64 ? kKsF64Waves : 2)
-void ks_inner_product_r16_kernel(KsArgs a, DeviceTables t) {
+__global__ __launch_bounds__(kBlock, 2) void ks_inner_product_r16_kernel(
+    KsArgs a, DeviceTables t) {
   __shared__ int64_t lds[kR16Lds<r16_low_bits(LOGN)>];
   ks_block<LOGN>(a, [&](const auto &ad, int tile, int i, int p0, int p1,
                         int half) {

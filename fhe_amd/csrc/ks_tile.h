@@ -110,6 +110,7 @@ __device__ __forceinline__ void ks_item_tile(const Addr &a,
       if constexpr (A == kF64) {
         f64_load(w, v, f.f);
       } else {
+        load_residues(w, f.q, f.k, t.r2[p]);
 #pragma unroll
         for (int m = 0; m < 16; m++)
           v[m] = w[m];
@@ -132,15 +133,21 @@ __device__ __forceinline__ void ks_item_tile(const Addr &a,
     if constexpr (A == kF64) {
       // plain products: the sums carry the key's Montgomery factor R, which
       // the epilogue of the second inverse pass takes out (kInttKeyReduce)
+      auto products = [&](const int64_t *key, double (&acc)[16]) {
+        int64_t kw[16];
 #pragma unroll
-      for (int m = 0; m < 16; m++) {
-        const double x0 = f64_mul(v[m], f64_from_int(k0[m]), f.f);
-        acc0[m] = pp == p0 ? x0 : acc0[m] + x0;
-        if (BOTH) {
-          const double x1 = f64_mul(v[m], f64_from_int(k1[m]), f.f);
-          acc1[m] = pp == p0 ? x1 : acc1[m] + x1;
+        for (int m = 0; m < 16; m++)
+          kw[m] = key[m];
+        load_residues(kw, f.q, f.k, t.r2[p]);
+#pragma unroll
+        for (int m = 0; m < 16; m++) {
+          const double x = f64_mul(v[m], f64_from_int(kw[m]), f.f);
+          acc[m] = pp == p0 ? x : acc[m] + x;
         }
-      }
+      };
+      products(k0, acc0);
+      if constexpr (BOTH)
+        products(k1, acc1);
     } else if (pp == p0) {
 #pragma unroll
       for (int m = 0; m < 16; m++) {

@@ -422,7 +422,9 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
   for (int m = 0; m < 16; m++)
     w[m] = src[int64_t(r16_point<L, cols_load>(r, m)) << b];
   if constexpr (A == kF64) {
-    if (first_pass) {
+    if (first_pass && INV) {
+      f64_load_centred(w, v, s.q, s.f);
+    } else if (first_pass) {
       f64_load(w, v, s.f);
       if (pre) {
         // the Montgomery product with pre is one with pre R^-1
@@ -430,11 +432,6 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
 #pragma unroll
         for (int m = 0; m < 16; m++)
           v[m] = f64_mul(v[m], c, s.f);
-      } else if (INV) {
-        // lazy residues in [0, 2q), centred
-#pragma unroll
-        for (int m = 0; m < 16; m++)
-          v[m] -= s.f.q;
       }
     } else {
 #pragma unroll
@@ -454,6 +451,8 @@ __device__ __forceinline__ void r16_limb_pass(const int64_t *src_limb,
       }
     }
   } else {
+    if (A == kLazyLarge && INV && first_pass)
+      load_residues(w, s.q, s.k, t.r2[p]);
 #pragma unroll
     for (int m = 0; m < 16; m++)
       v[m] = pre ? load_product<A>(w[m], pre[p], s.q, s.k) : w[m];
