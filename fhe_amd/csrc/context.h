@@ -302,30 +302,75 @@ struct fhe_context {
     pending.clear();
   }
 
-  // Whether key switching at moduli_id takes the fused path, which holds
-  // every partition's extended limbs at once.  Below N = 2^16 it is left for
-  // chains so long that these would take more than kMaxExtLimbs limbs per
-  // ciphertext, and by callers with a fixed workspace (fused_key_switch).
-  static constexpr int kMaxExtLimbs = 1024;
-  bool fused_key_switch = true;
-  bool ks_fused(int moduli_id) const {
-    if (!fhe::ks_fused_supported(tables))
-      return false;
-    if (tables.log_n == 16)
-      return true;
-    return fused_key_switch && params.partition_count(moduli_id) *
-                                       (params.limbs_at(moduli_id) +
-                                        params.alpha) <= kMaxExtLimbs;
-  }
   // lazy arithmetic of whole transforms: the radix-16 sizes
   bool lazy_transforms() const {
     return lazy_key_switch && fhe::ks_fused_supported(tables);
   }
-  // extended polynomials held at once by key switching: every partition on
-  // the fused path, one at a time otherwise
-  int ext_slots(int moduli_id) const {
-    return ks_fused(moduli_id) ? params.partition_count(moduli_id) : 1;
+
+  // How key switching of `count` ciphertexts at moduli_id runs: on the fused
+  // path with the extended limbs of every partition of `group` ciphertexts at
+  // once, group after group, or (group 0) one partition of the whole batch at
+  // a time.  ext_words: its extended-limb buffer.
+  struct KsPlan {
+    int group;
+    int64_t ext_words;
+  };
+  // Chains whose partitions together take more limbs per ciphertext run one
+  // partition at a time below N = 2^16.
+  static constexpr int kMaxExtLimbs = 1024;
+  bool ks_fused(int moduli_id) const {
+    return fhe::ks_fused_supported(tables) &&
+           (tables.log_n == 16 ||
+            params.partition_count(moduli_id) *
+                    (params.limbs_at(moduli_id) + params.alpha) <=
+                kMaxExtLimbs);
   }
+  // A group's extended limbs and digits below N = 2^16: 8 GiB, more than 80
+  // ciphertexts of the longest chains, so that larger batches need little
+  // more than one partition of each did (N = 2^16 holds the batch).
+  static constexpr int64_t kKsGroupWords = int64_t(1) << 30;
+  int64_t ext_poly_words(int moduli_id) const {
+    return int64_t(params.limbs_at(moduli_id) + params.alpha) * params.n;
+  }
+  KsPlan ks_one_partition(int count, int moduli_id) const {
+    return {0, count * ext_poly_words(moduli_id)};
+  }
+  KsPlan ks_groups_of(int group, int moduli_id) const {
+    return {group, group * int64_t(params.partition_count(moduli_id)) *
+                       ext_poly_words(moduli_id)};
+  }
+  // `others`: words that the caller's workspace holds beside the extended
+  // limbs.  Where the workspace may not grow (a graph holds it), the groups
+  // are as large as what is there allows.
+  KsPlan ks_plan(int count, int moduli_id, int64_t others) const {
+    const KsPlan least = ks_one_partition(count, moduli_id);
+    if (!ks_fused(moduli_id))
+      return least;
+    if (tables.log_n == 16)
+      return ks_groups_of(count, moduli_id);
+    const int64_t one = ks_groups_of(1, moduli_id).ext_words;
+    int64_t group = std::max(kKsGroupWords, least.ext_words) /
+                    (one + ks_digits_words(1, moduli_id));
+    if (!may_grow())
+      group = std::min(group,
+                       (int64_t(workspace_bytes / 8) - others) / one);
+    group = std::min<int64_t>(group, count);
+    return group > 0 ? ks_groups_of(int(group), moduli_id) : least;
+  }
+  // The scratch workspace with `others` words and the plan's extended limbs;
+  // below N = 2^16, where the device cannot hold them, smaller groups.
+  int64_t *ks_scratch(int count, int moduli_id, int64_t others, KsPlan &plan) {
+    plan = ks_plan(count, moduli_id, others);
+    while (tables.log_n != 16 && plan.group > 0 &&
+           !scratch_fits(size_t(others + plan.ext_words) * 8))
+      plan = plan.group > 1 ? ks_groups_of(plan.group / 2, moduli_id)
+                            : ks_one_partition(count, moduli_id);
+    return scratch(size_t(others + plan.ext_words) * 8);
+  }
+
+  // Whether workspaces may be reallocated: not under capture, nor while
+  // captured graphs hold their addresses.
+  bool may_grow() const { return !capturing && live_graphs == 0; }
 
   void require_not_capturing(const char *what) const {
     require(!capturing, std::string(what) +
@@ -343,49 +388,53 @@ struct fhe_context {
                                 "capturing)");
   }
 
-  int64_t *aux_scratch(size_t bytes) {
-    if (bytes > aux_bytes) {
-      require_workspace_fixed("workspace growth");
-      hip_check(hipStreamSynchronize(stream), "workspace sync");
-      if (aux)
-        hip_check(hipFree(aux), "workspace free");
-      aux = nullptr;
-      aux_bytes = 0;
-      hip_check(hipMalloc(&aux, bytes), "workspace allocation");
-      aux_bytes = bytes;
+  // Grows a buffer to `bytes` if it may and the device has the memory; the
+  // old contents are gone either way.
+  bool grow(void *&buffer, size_t &have, size_t bytes) {
+    if (bytes <= have)
+      return true;
+    if (!may_grow())
+      return false;
+    hip_check(hipStreamSynchronize(stream), "workspace sync");
+    if (buffer)
+      hip_check(hipFree(buffer), "workspace free");
+    buffer = nullptr;
+    have = 0;
+    const hipError_t error = hipMalloc(&buffer, bytes);
+    if (error == hipErrorOutOfMemory) {
+      (void)hipGetLastError(); // not the next launch check's
+      buffer = nullptr;
+      return false;
     }
-    return static_cast<int64_t *>(aux);
+    hip_check(error, "workspace allocation");
+    have = bytes;
+    return true;
+  }
+  int64_t *grown(void *&buffer, size_t &have, size_t bytes) {
+    if (bytes > have)
+      require_workspace_fixed("workspace growth");
+    if (!grow(buffer, have, bytes))
+      hip_check(hipErrorOutOfMemory, "workspace allocation");
+    return static_cast<int64_t *>(buffer);
   }
 
-  // partial sums of the split key inner product; null where the buffer would
-  // have to grow while a graph holds it (the caller then does not split)
+  int64_t *aux_scratch(size_t bytes) { return grown(aux, aux_bytes, bytes); }
+  // as aux_scratch, null where it cannot have that size
+  int64_t *aux_if_room(size_t bytes) {
+    return grow(aux, aux_bytes, bytes) ? static_cast<int64_t *>(aux)
+                                       : nullptr;
+  }
+
+  // partial sums of the split key inner product; null where the buffer cannot
+  // have that size (the caller then does not split)
   int64_t *partial_sums(size_t bytes) {
-    if (bytes > partial_bytes) {
-      if (capturing || live_graphs != 0)
-        return nullptr;
-      hip_check(hipStreamSynchronize(stream), "workspace sync");
-      if (partial_buf)
-        hip_check(hipFree(partial_buf), "workspace free");
-      partial_buf = nullptr;
-      partial_bytes = 0;
-      hip_check(hipMalloc(&partial_buf, bytes), "workspace allocation");
-      partial_bytes = bytes;
-    }
-    return static_cast<int64_t *>(partial_buf);
+    return grow(partial_buf, partial_bytes, bytes)
+               ? static_cast<int64_t *>(partial_buf)
+               : nullptr;
   }
 
   int64_t *stash(size_t bytes) {
-    if (bytes > stash_bytes) {
-      require_workspace_fixed("workspace growth");
-      hip_check(hipStreamSynchronize(stream), "workspace sync");
-      if (stash_buf)
-        hip_check(hipFree(stash_buf), "workspace free");
-      stash_buf = nullptr;
-      stash_bytes = 0;
-      hip_check(hipMalloc(&stash_buf, bytes), "workspace allocation");
-      stash_bytes = bytes;
-    }
-    return static_cast<int64_t *>(stash_buf);
+    return grown(stash_buf, stash_bytes, bytes);
   }
 
   // CKKSCore::switch_key (src/ckks/core.cpp:1058-1083) of `count` INTT-form
@@ -397,12 +446,12 @@ struct fhe_context {
     const int limbs = params.limbs_at(moduli_id);
     const int ext_limbs = limbs + params.alpha;
     const int64_t N = n();
-    const int64_t ext_l = int64_t(count) * ext_slots(moduli_id) * ext_limbs;
-    const int64_t acc_l = int64_t(count) * 2 * ext_limbs;
-    int64_t *ws = scratch(size_t(ext_l + acc_l) * N * 8);
-    int64_t *ext = ws, *acc = ext + ext_l * N;
+    KsPlan plan;
+    int64_t *ext = ks_scratch(count, moduli_id,
+                              int64_t(count) * 2 * ext_limbs * N, plan);
+    int64_t *acc = ext + plan.ext_words;
     key_switch(count, moduli_id, key, key_moduli_id, in + limbs * N,
-               2 * limbs * N, ext, acc, nullptr, 0, signed_input);
+               2 * limbs * N, ext, acc, plan, nullptr, 0, signed_input);
     stage("moddown_add", [&] {
       fhe::launch_moddown_add(tables, acc, in, 2 * limbs * N, 1, out, count,
                               limbs, moduli_id, stream);
@@ -410,17 +459,10 @@ struct fhe_context {
   }
 
   int64_t *scratch(size_t bytes) {
-    if (bytes > workspace_bytes) {
-      require_workspace_fixed("workspace growth");
-      hip_check(hipStreamSynchronize(stream), "workspace sync");
-      if (workspace)
-        hip_check(hipFree(workspace), "workspace free");
-      workspace = nullptr;
-      workspace_bytes = 0;
-      hip_check(hipMalloc(&workspace, bytes), "workspace allocation");
-      workspace_bytes = bytes;
-    }
-    return static_cast<int64_t *>(workspace);
+    return grown(workspace, workspace_bytes, bytes);
+  }
+  bool scratch_fits(size_t bytes) {
+    return grow(workspace, workspace_bytes, bytes);
   }
 
   const fhe::EncodeDevice &encode_tables() {
@@ -636,10 +678,10 @@ struct fhe_context {
     const int ext_limbs = limbs + params.alpha;
     const int64_t N = n();
     const int64_t trio_l = int64_t(count) * 3 * limbs;
-    const int64_t ext_l = int64_t(count) * ext_slots(moduli_id) * ext_limbs;
     const int64_t acc_l = int64_t(count) * 2 * ext_limbs;
-    int64_t *ws = scratch(size_t(trio_l + ext_l + acc_l) * N * 8);
-    int64_t *trio = ws, *ext = trio + trio_l * N, *acc = ext + ext_l * N;
+    KsPlan plan;
+    int64_t *trio = ks_scratch(count, moduli_id, (trio_l + acc_l) * N, plan);
+    int64_t *ext = trio + trio_l * N, *acc = ext + plan.ext_words;
     const int64_t poly = int64_t(limbs) * N;
     // d0 and d1 are canonicalized by the relinearization add; d2 feeds the
     // representative-sensitive ModUp (the flags are in the accumulators,
@@ -656,7 +698,8 @@ struct fhe_context {
     });
     // the caller's NTT-form d2 provides the partitions' own extended limbs
     key_switch(count, moduli_id, key, key_moduli_id, trio + 2 * limbs * N,
-               3 * limbs * N, ext, acc, trios + 2 * limbs * N, 3 * limbs * N);
+               3 * limbs * N, ext, acc, plan, trios + 2 * limbs * N,
+               3 * limbs * N);
     stage("moddown_relin", [&] {
       fhe::launch_moddown_relin(tables, acc, trio, out, count, limbs,
                                 moduli_id, stream);
@@ -708,21 +751,26 @@ struct fhe_context {
   // signed_input: the source limbs may be any int64 (the signed tile of
   // modulus raising), not residues in [0, 2q): every partition then takes
   // the signed Garner digits and the exact extension.
-  // digits (optional): room for the staged ModUp's Garner digits
+  // digits (optional): room for the staged ModUp's Garner digits of a group
   // (ks_digits_words) instead of the context's second growable buffer.
   void key_switch(int count, int moduli_id, const int64_t *key,
                   int key_moduli_id, const int64_t *src, int64_t src_stride,
-                  int64_t *ext, int64_t *acc, const int64_t *own = nullptr,
-                  int64_t own_stride = 0, bool signed_input = false,
-                  int64_t *digits = nullptr) {
-    if (ks_fused(moduli_id)) {
+                  int64_t *ext, int64_t *acc, const KsPlan &plan,
+                  const int64_t *own = nullptr, int64_t own_stride = 0,
+                  bool signed_input = false, int64_t *digits = nullptr) {
+    if (plan.group > 0) {
       if (!own_limbs || int(params.partitions(moduli_id, key_moduli_id)
                                 .size()) > fhe::kMaxFusedParts)
         own = nullptr;
-      ks_decompose(count, moduli_id, key_moduli_id, src, src_stride, ext,
-                   own != nullptr, signed_input, digits);
-      ks_apply(count, moduli_id, key, key_moduli_id, ext, acc, own,
-               own_stride, digits == nullptr);
+      for (int c = 0; c < count; c += plan.group) {
+        const int here = std::min(plan.group, count - c);
+        ks_decompose(here, moduli_id, key_moduli_id, src + c * src_stride,
+                     src_stride, ext, own != nullptr, signed_input, digits);
+        ks_apply(here, moduli_id, key, key_moduli_id, ext,
+                 acc + 2 * c * ext_poly_words(moduli_id),
+                 own ? own + c * own_stride : nullptr, own_stride,
+                 digits == nullptr);
+      }
       return;
     }
     const int limbs = params.limbs_at(moduli_id);
@@ -797,13 +845,17 @@ struct fhe_context {
                        !params.modup_non_negative(moduli_id, parts[p]);
       max_size = std::max(max_size, sizes[p]);
     }
+    int64_t *digits = nullptr;
     if (staged_modup && fhe::staged_modup_supported(tables, max_size, np)) {
       int maxz = 1;
       while (maxz < max_size)
         maxz <<= 1;
-      int64_t *digits =
-          digits_ws ? digits_ws
-                    : aux_scratch(size_t(count) * np * maxz * size_t(N) * 8);
+      // without room for the digits the extension recomputes them
+      digits = digits_ws
+                   ? digits_ws
+                   : aux_if_room(size_t(count) * np * maxz * size_t(N) * 8);
+    }
+    if (digits) {
       stage("modup_staged(ext)", [&] {
         fhe::launch_staged_modup(tables, src, src_stride, digits, ext, count,
                                  limbs, moduli_id, starts.data(), sizes.data(),
@@ -893,15 +945,25 @@ fhe::CkksParams resolve_params(const fhe_params *p, bool twiddles = true);
 
 // The batched product, relinearization and, with rescale, rescale pipeline
 // (context.hip) of duos in INTT form, or NTT form with a_ntt / b_ntt, on a
-// caller-given workspace of hmult_workspace_words words and, when given, a
-// digits buffer of ks_digits_words words.
-int64_t hmult_workspace_words(const fhe_context *ctx, int count,
-                              int moduli_id);
+// caller-given workspace (limbs of N words, per ciphertext).
+struct ProductSpace {
+  fhe_context::KsPlan plan;
+  int64_t *factors; // the factors' transforms: 4 x limbs
+  int64_t *trio;    // the trio in NTT form: 3 x limbs
+  int64_t *trio_c;  // and in coefficient form: 3 x limbs
+  int64_t *ext;     // plan.ext_words in all
+  int64_t *acc;     // 2 x (limbs + alpha)
+  int64_t *digits;  // ks_digits_words of a group, or null
+  // all but the extended limbs and digits of a batch, one after the other
+  static int64_t others(const fhe_context *ctx, int count, int moduli_id);
+  static ProductSpace at(const fhe_context *ctx, int count, int moduli_id,
+                         const fhe_context::KsPlan &plan, int64_t *ws,
+                         int64_t *digits);
+};
 void hmult_relin_into(fhe_context *ctx, int count, int moduli_id,
                       const int64_t *a, bool a_ntt, const int64_t *b,
                       bool b_ntt, const int64_t *key, int key_moduli_id,
-                      bool rescale, int64_t *out, int64_t *ws,
-                      int64_t *digits);
+                      bool rescale, int64_t *out, const ProductSpace &space);
 // Set-up of the allocation-free entry point on the current device `device`
 // (noalloc.hip).
 void noalloc_scratch_setup(int device);

@@ -321,40 +321,37 @@ int fhe_relinearize(fhe_context *ctx, int count, int moduli_id,
 
 } // extern "C"
 
-int64_t hmult_workspace_words(const fhe_context *ctx, int count,
-                              int moduli_id) {
-  const auto &P = ctx->params;
-  const int limbs = P.limbs_at(moduli_id);
-  const int ext_limbs = limbs + P.alpha;
-  const int64_t duo_l = int64_t(count) * 2 * limbs;
-  const int64_t trio_l = int64_t(count) * 3 * limbs;
-  const int64_t ext_l = int64_t(count) * ctx->ext_slots(moduli_id) * ext_limbs;
-  const int64_t acc_l = int64_t(count) * 2 * ext_limbs;
-  return (2 * duo_l + 2 * trio_l + ext_l + acc_l) * int64_t(P.n);
+int64_t ProductSpace::others(const fhe_context *ctx, int count,
+                             int moduli_id) {
+  const int64_t limbs = ctx->params.limbs_at(moduli_id);
+  return count * (10 * limbs * ctx->n() + 2 * ctx->ext_poly_words(moduli_id));
 }
 
-// The batched HMult + relinearize (+ rescale) pipeline on the workspace ws
-// (hmult_workspace_words) and, when given, the digits buffer (the staged
-// ModUp's Garner digits; else the context's second buffer).  Arguments are
-// checked by the caller.
+ProductSpace ProductSpace::at(const fhe_context *ctx, int count,
+                              int moduli_id, const fhe_context::KsPlan &plan,
+                              int64_t *ws, int64_t *digits) {
+  const int64_t poly = count * int64_t(ctx->params.limbs_at(moduli_id)) *
+                       ctx->n();
+  return {plan,          ws, ws + 4 * poly, ws + 7 * poly, ws + 10 * poly,
+          ws + 10 * poly + plan.ext_words, digits};
+}
+
+// The batched HMult + relinearize (+ rescale) pipeline on the given space
+// (without digits: the context's second buffer).  Arguments are checked by
+// the caller.
 void hmult_relin_into(fhe_context *ctx, int count, int moduli_id,
                       const int64_t *a, bool a_ntt, const int64_t *b,
                       bool b_ntt, const int64_t *key, int key_moduli_id,
-                      bool rescale, int64_t *out, int64_t *ws,
-                      int64_t *digits) {
+                      bool rescale, int64_t *out, const ProductSpace &space) {
     const auto &P = ctx->params;
     const int limbs = P.limbs_at(moduli_id);
-    const int ext_limbs = limbs + P.alpha;
     const int64_t N = ctx->n();
     const int64_t duo_l = int64_t(count) * 2 * limbs;
     const int64_t trio_l = int64_t(count) * 3 * limbs;
-    const int64_t ext_l =
-        int64_t(count) * ctx->ext_slots(moduli_id) * ext_limbs;
     // trio_c: the coefficient form of the trio; trio keeps the NTT form,
     // whose d2 limbs serve the partitions' own extended limbs
-    int64_t *an = ws, *bn = an + duo_l * N, *trio = bn + duo_l * N;
-    int64_t *trio_c = trio + trio_l * N;
-    int64_t *ext = trio_c + trio_l * N, *acc = ext + ext_l * N;
+    int64_t *an = space.factors, *bn = an + duo_l * N, *trio = space.trio;
+    int64_t *trio_c = space.trio_c, *ext = space.ext, *acc = space.acc;
     // prepare_for_multiply: to NTT form (src/ckks/engine_multiply.cpp:13-27).
     // Lazy throughout: d0 and d1 are canonicalized by the relinearization
     // add, and d2's inverse feeds the representative-sensitive ModUp
@@ -398,7 +395,8 @@ void hmult_relin_into(fhe_context *ctx, int count, int moduli_id,
     });
     ctx->key_switch(count, moduli_id, key, key_moduli_id,
                     trio_c + 2 * limbs * N, 3 * limbs * N, ext, acc,
-                    trio + 2 * limbs * N, 3 * limbs * N, false, digits);
+                    space.plan, trio + 2 * limbs * N, 3 * limbs * N, false,
+                    space.digits);
     if (!rescale) {
       ctx->stage("moddown_relin", [&] {
         fhe::launch_moddown_relin(ctx->tables, acc, trio_c, out, count, limbs,
@@ -423,10 +421,13 @@ int fhe_hmult_relin_rescale(fhe_context *ctx, int count, int moduli_id,
     require(count > 0, "Multiply: empty batch");
     ctx->check_moduli(moduli_id, 3, "Multiply");
     ctx->check_key(moduli_id, key_moduli_id, "Multiply");
-    int64_t *ws = ctx->scratch(
-        size_t(hmult_workspace_words(ctx, count, moduli_id)) * 8);
+    fhe_context::KsPlan plan;
+    int64_t *ws = ctx->ks_scratch(
+        count, moduli_id, ProductSpace::others(ctx, count, moduli_id), plan);
     hmult_relin_into(ctx, count, moduli_id, a, false, b, false, key,
-                     key_moduli_id, true, out, ws, nullptr);
+                     key_moduli_id, true, out,
+                     ProductSpace::at(ctx, count, moduli_id, plan, ws,
+                                      nullptr));
     ctx->check_launch("Multiply");
   });
 }
@@ -459,13 +460,15 @@ static void multiply_texts(fhe_context *ctx, int count, const int64_t *a,
   const int prod_polys = b_polys == 2 ? 3 : a_polys;
   if (key)
     ctx->check_key(mid, key_moduli_id, op);
-  // prepared inputs in the stash; the preparation's temporaries in the
-  // scratch workspace, which the product reuses
+  // prepared inputs and, before a relinearization, the product in the stash;
+  // the preparation's temporaries in the scratch workspace, which the
+  // relinearization reuses
   const int64_t an_l = int64_t(count) * a_polys * poly;
   const int64_t bn_l = int64_t(count) * b_polys * poly;
-  int64_t *an = ctx->stash(size_t(an_l + bn_l) * 8);
+  const int64_t prod_l = int64_t(count) * prod_polys * poly;
+  int64_t *an = ctx->stash(size_t(an_l + bn_l + (key ? prod_l : 0)) * 8);
   int64_t *bn = an + an_l;
-  int64_t *prod = out;
+  int64_t *prod = key ? bn + bn_l : out;
   auto limbs_of = [&](int l, int f) {
     return int64_t(P.limbs_at(ctx->moduli_id_of(l, f & FHE_FLAG_RESCALED)));
   };
@@ -473,10 +476,28 @@ static void multiply_texts(fhe_context *ctx, int count, const int64_t *a,
       std::max(int64_t(count) * a_polys * limbs_of(a_level, a_flags),
                int64_t(count) * b_polys * limbs_of(b_level, b_flags)) *
       N;
-  const int64_t ws_l = key ? hmult_workspace_words(ctx, count, mid) : 0;
-  int64_t *t0 = ctx->scratch(size_t(std::max(2 * t_l, ws_l)) * 8);
-  int64_t *t1 = t0 + t_l;
+  int64_t ws_l = 2 * t_l;
+  ProductSpace space{};
+  bool pipeline = false;
   if (key) {
+    // the space of relinearizing the product, which is in the stash: the
+    // factors' transforms, done with before the key switching, share the
+    // extended limbs' and the accumulators' words.  (The exact recomputation
+    // of zero residues takes the first half of them, with the flags in the
+    // accumulators.)
+    const int64_t acc_w = 2 * count * ctx->ext_poly_words(mid);
+    (void)ctx->ks_scratch(count, mid, 3 * count * poly + acc_w, space.plan);
+    pipeline = space.plan.ext_words >= 2 * count * poly &&
+               space.plan.ext_words + acc_w >= 4 * count * poly;
+    ws_l = std::max(ws_l, 3 * count * poly + space.plan.ext_words + acc_w);
+  }
+  int64_t *t0 = ctx->scratch(size_t(ws_l) * 8);
+  int64_t *t1 = t0 + t_l;
+  if (pipeline) {
+    space.trio = prod;
+    space.trio_c = t0;
+    space.ext = space.factors = t0 + 3 * count * poly;
+    space.acc = space.ext + space.plan.ext_words;
     // rescaled at the lower level, in the coefficient domain unless the text
     // is there in NTT form already; the product's pipeline transforms it
     auto prepared = [&](const int64_t *in, int level_in, int flags,
@@ -495,7 +516,7 @@ static void multiply_texts(fhe_context *ctx, int count, const int64_t *a,
     const int64_t *bp =
         same ? ap : prepared(b, b_level, b_flags, bn, b_ntt);
     hmult_relin_into(ctx, count, mid, ap, a_ntt, bp, b_ntt, key, key_moduli_id,
-                     false, out, t0, nullptr);
+                     false, out, space);
     return;
   }
   const int64_t *ap = ctx->prepare_for_multiply_into(
@@ -525,6 +546,8 @@ static void multiply_texts(fhe_context *ctx, int count, const int64_t *a,
                                 limbs, mid, ctx->stream);
     });
   }
+  if (key)
+    ctx->relinearize_into(count, mid, prod, key, key_moduli_id, out);
 }
 
 int fhe_multiply(fhe_context *ctx, int count, const int64_t *a, int a_level,
@@ -1063,19 +1086,18 @@ int fhe_rotate(fhe_context *ctx, int count, int moduli_id, const int64_t *in,
     ctx->check_key(moduli_id, key_moduli_id, "Rotate");
     const auto &P = ctx->params;
     const int limbs = P.limbs_at(moduli_id);
-    const int ext_limbs = limbs + P.alpha;
     const int64_t N = ctx->n();
     const int64_t duo_l = int64_t(count) * 2 * limbs;
-    const int64_t ext_l =
-        int64_t(count) * ctx->ext_slots(moduli_id) * ext_limbs;
-    const int64_t acc_l = int64_t(count) * 2 * ext_limbs;
-    int64_t *ws = ctx->scratch(size_t(duo_l + ext_l + acc_l) * N * 8);
-    int64_t *sw = ws, *ext = sw + duo_l * N, *acc = ext + ext_l * N;
+    fhe_context::KsPlan plan;
+    int64_t *sw = ctx->ks_scratch(
+        count, moduli_id,
+        duo_l * N + 2 * count * ctx->ext_poly_words(moduli_id), plan);
+    int64_t *ext = sw + duo_l * N, *acc = ext + plan.ext_words;
     // key switch of c1; c0 joins after ModDown, where the reference adds
     // c0 * P before it (src/ckks/core_key_switch.cpp:509-548): both give
     // floor((X + c0 P) / P) = floor(X / P) + c0
     ctx->key_switch(count, moduli_id, key, key_moduli_id, in + limbs * N,
-                    2 * limbs * N, ext, acc);
+                    2 * limbs * N, ext, acc, plan);
     ctx->stage("moddown_add", [&] {
       fhe::launch_moddown_add(ctx->tables, acc, in, 2 * limbs * N, 1, sw,
                               count, limbs, moduli_id, ctx->stream);
@@ -1107,36 +1129,43 @@ int fhe_rotate_batch(fhe_context *ctx, int count, int moduli_id,
     }
     const auto &P = ctx->params;
     const int limbs = P.limbs_at(moduli_id);
-    const int ext_limbs = limbs + P.alpha;
     const int64_t N = ctx->n();
     const int64_t duo_l = int64_t(count) * 2 * limbs;
-    const int64_t ext_l =
-        int64_t(count) * ctx->ext_slots(moduli_id) * ext_limbs;
-    const int64_t acc_l = int64_t(count) * 2 * ext_limbs;
-    int64_t *ws = ctx->scratch(size_t(duo_l + ext_l + acc_l) * N * 8);
-    int64_t *sw = ws, *ext = sw + duo_l * N, *acc = ext + ext_l * N;
-    const bool hoist = ctx->ks_fused(moduli_id);
+    fhe_context::KsPlan plan;
+    int64_t *sw = ctx->ks_scratch(
+        count, moduli_id,
+        duo_l * N + 2 * count * ctx->ext_poly_words(moduli_id), plan);
+    int64_t *ext = sw + duo_l * N, *acc = ext + plan.ext_words;
     // CKKSEngine::rotate_batch (src/ckks/engine_rotate.cpp:262-300): one
-    // decomposition of c1, then the key-dependent part per key
-    if (hoist)
-      ctx->ks_decompose(count, moduli_id, key_moduli_ids[0], in + limbs * N,
-                        2 * limbs * N, ext);
-    for (int k = 0; k < key_count; k++) {
+    // decomposition of c1, then the key-dependent part per key; group by
+    // group of ciphertexts, or with key switching one partition at a time
+    const bool hoist = plan.group > 0;
+    const int group = hoist ? plan.group : count;
+    const int64_t duo = 2 * limbs * N;
+    for (int c = 0; c < count; c += group) {
+      const int here = std::min(group, count - c);
+      const int64_t *duos = in + c * duo;
       if (hoist)
-        ctx->ks_apply(count, moduli_id, keys[k], key_moduli_ids[k], ext, acc);
-      else
-        ctx->key_switch(count, moduli_id, keys[k], key_moduli_ids[k],
-                        in + limbs * N, 2 * limbs * N, ext, acc);
-      ctx->stage("moddown_add", [&] {
-        fhe::launch_moddown_add(ctx->tables, acc, in, 2 * limbs * N, 1, sw,
-                                count, limbs, moduli_id, ctx->stream);
-      });
-      ctx->stage("automorphism", [&] {
-        fhe::launch_automorphism(ctx->tables, sw, outs[k], duo_l, limbs,
-                                 moduli_id,
-                                 automorphism_exponent(P.log_n, deltas[k]),
-                                 ctx->stream);
-      });
+        ctx->ks_decompose(here, moduli_id, key_moduli_ids[0],
+                          duos + limbs * N, duo, ext);
+      for (int k = 0; k < key_count; k++) {
+        if (hoist)
+          ctx->ks_apply(here, moduli_id, keys[k], key_moduli_ids[k], ext, acc);
+        else
+          ctx->key_switch(here, moduli_id, keys[k], key_moduli_ids[k],
+                          duos + limbs * N, duo, ext, acc, plan);
+        ctx->stage("moddown_add", [&] {
+          fhe::launch_moddown_add(ctx->tables, acc, duos, duo, 1, sw, here,
+                                  limbs, moduli_id, ctx->stream);
+        });
+        ctx->stage("automorphism", [&] {
+          fhe::launch_automorphism(ctx->tables, sw, outs[k] + c * duo,
+                                   int64_t(here) * 2 * limbs, limbs,
+                                   moduli_id,
+                                   automorphism_exponent(P.log_n, deltas[k]),
+                                   ctx->stream);
+        });
+      }
     }
     ctx->check_launch("Rotate");
   });
@@ -1252,14 +1281,13 @@ int fhe_conjugate(fhe_context *ctx, int count, int moduli_id,
     ctx->check_key(moduli_id, key_moduli_id, "Conjugate");
     const auto &P = ctx->params;
     const int limbs = P.limbs_at(moduli_id);
-    const int ext_limbs = limbs + P.alpha;
     const int64_t N = ctx->n();
     const int64_t duo_l = int64_t(count) * 2 * limbs;
-    const int64_t ext_l =
-        int64_t(count) * ctx->ext_slots(moduli_id) * ext_limbs;
-    const int64_t acc_l = int64_t(count) * 2 * ext_limbs;
-    int64_t *ws = ctx->scratch(size_t(duo_l + ext_l + acc_l) * N * 8);
-    int64_t *perm = ws, *ext = perm + duo_l * N, *acc = ext + ext_l * N;
+    fhe_context::KsPlan plan;
+    int64_t *perm = ctx->ks_scratch(
+        count, moduli_id,
+        duo_l * N + 2 * count * ctx->ext_poly_words(moduli_id), plan);
+    int64_t *ext = perm + duo_l * N, *acc = ext + plan.ext_words;
     // CKKSCore::conjugate (src/ckks/core.cpp:1035-1056): automorphism
     // first, then key switching of the permuted c1 plus the permuted c0
     ctx->stage("automorphism", [&] {
@@ -1268,7 +1296,7 @@ int fhe_conjugate(fhe_context *ctx, int count, int moduli_id,
                                ctx->stream);
     });
     ctx->key_switch(count, moduli_id, key, key_moduli_id, perm + limbs * N,
-                    2 * limbs * N, ext, acc);
+                    2 * limbs * N, ext, acc, plan);
     ctx->stage("moddown_add", [&] {
       fhe::launch_moddown_add(ctx->tables, acc, perm, 2 * limbs * N, 1, out,
                               count, limbs, moduli_id, ctx->stream);

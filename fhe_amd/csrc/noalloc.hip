@@ -58,29 +58,38 @@ extern "C" int fhe_hmult_relin_rescale_noalloc(fhe_context *ctx, int count,
     // runs (N != 2^16); batches it holds are accepted, and run in the fused
     // form in as many parts as the fused form's workspace asks for, or, when
     // that holds not even one pair, one partition at a time
-    const bool fused = ctx->fused_key_switch;
-    struct Restore {
-      fhe_context *ctx;
-      bool fused;
-      ~Restore() { ctx->fused_key_switch = fused; }
-    } restore{ctx, fused};
-    auto words = [&](int n) {
-      return hmult_workspace_words(ctx, n, moduli_id) +
+    using Plan = fhe_context::KsPlan;
+    auto words = [&](int n, const Plan &plan) {
+      return ProductSpace::others(ctx, n, moduli_id) + plan.ext_words +
              ctx->ks_digits_words(n, moduli_id);
     };
-    ctx->fused_key_switch = false;
-    const int64_t least = words(count);
+    const bool whole = ctx->tables.log_n == 16;
+    Plan plan = whole ? ctx->ks_groups_of(count, moduli_id)
+                      : ctx->ks_one_partition(count, moduli_id);
+    const int64_t least = words(count, plan);
     require(size_t(least) <= kScratchWords,
             "Multiply (no allocation): the batch needs " +
                 std::to_string(least * 8) +
                 " bytes of workspace, above the " +
                 std::to_string(kScratchBytes) +
                 "-byte scratch; split the batch");
-    ctx->fused_key_switch = fused;
-    int part = std::min<int64_t>(count, kScratchWords / words(1));
-    if (part == 0) {
-      ctx->fused_key_switch = false;
-      part = count;
+    const int64_t in = int64_t(2) * ctx->params.limbs_at(moduli_id) * ctx->n();
+    const int64_t res = in - 2 * ctx->n();
+    int part = count;
+    if (!whole && ctx->ks_fused(moduli_id)) {
+      const Plan one = ctx->ks_groups_of(1, moduli_id);
+      const int fit = int(std::min<int64_t>(
+          count, int64_t(kScratchWords) / words(1, one)));
+      // a part's results may not reach the factors of a later part: an output
+      // is never ahead of a factor that starts at or after it (a result is
+      // shorter than a factor)
+      auto apart = [&](const int64_t *x) {
+        return out <= x || out >= x + count * in;
+      };
+      if (fit >= count || (fit > 0 && apart(a) && apart(b))) {
+        part = fit;
+        plan = ctx->ks_groups_of(part, moduli_id);
+      }
     }
     require(ctx->modup_cache.count({moduli_id, key_moduli_id}) != 0,
             "Multiply (no allocation): no ModUp constants for this key "
@@ -94,13 +103,14 @@ extern "C" int fhe_hmult_relin_rescale_noalloc(fhe_context *ctx, int count,
     }
     require(base != nullptr, "Multiply (no allocation): no scratch address "
                              "for this device");
-    const int64_t in = int64_t(2) * ctx->params.limbs_at(moduli_id) * ctx->n();
-    const int64_t res = in - 2 * ctx->n();
     for (int c = 0; c < count; c += part) {
       const int n = std::min(part, count - c);
-      hmult_relin_into(ctx, n, moduli_id, a + c * in, false, b + c * in, false,
-                       key, key_moduli_id, true, out + c * res, base,
-                       base + hmult_workspace_words(ctx, n, moduli_id));
+      hmult_relin_into(
+          ctx, n, moduli_id, a + c * in, false, b + c * in, false, key,
+          key_moduli_id, true, out + c * res,
+          ProductSpace::at(ctx, n, moduli_id, plan, base,
+                           base + ProductSpace::others(ctx, n, moduli_id) +
+                               plan.ext_words));
     }
     ctx->check_launch("Multiply");
   });
