@@ -34,16 +34,25 @@ struct Batch {
 };
 
 // Device bytes a batch of `count` jobs at `limbs` limbs may take beyond its
-// inputs: the key switch's extended limbs, accumulators and trio for each
-// ciphertext, and the texts of the composition (power basis or the
-// rotation chain), in limbs of N words.
-size_t batch_bytes(const fhe_context *ctx, int kind, int count, int limbs) {
+// inputs: the key switch's extended limbs, digits, accumulators, partial sums
+// and coefficient-form trio, the prepared factors and NTT-form trio of its
+// products, and the texts of the composition (`degree` powers and the weighted
+// sum's, or the rotation chain).
+size_t batch_bytes(const fhe_context *ctx, int kind, int degree, int count,
+                   int limbs) {
   const auto &P = ctx->params;
-  const int ext = limbs + P.alpha;
-  const int parts = (limbs + P.alpha - 1) / P.alpha;
-  const int64_t ks = int64_t(parts) * ext + 2 * ext + 3 * limbs;
-  const int64_t texts = kind == FHE_JOB_POLY ? 9 * 2 * limbs : 6 * 2 * limbs;
-  return size_t(count) * size_t(ks + texts) * size_t(P.n) * 8;
+  const int mid = P.chain_count - limbs;
+  const int64_t acc = 2 * ctx->ext_poly_words(mid);
+  const auto plan =
+      ctx->ks_plan(count, mid, count * (3 * int64_t(limbs) * P.n + acc));
+  const auto split =
+      fhe::ks_split(ctx->tables, P.partition_count(mid), count,
+                    limbs + P.alpha, ctx->lazy_key_switch);
+  const int64_t texts = (kind == FHE_JOB_POLY ? degree + 5 : 6) * 2 * limbs;
+  return size_t(plan.ext_words + ctx->ks_digits_words(plan.group, mid) +
+                count * split.groups * acc +
+                count * (10 * int64_t(limbs) + texts) * P.n) *
+         8;
 }
 
 } // namespace
@@ -149,7 +158,8 @@ extern "C" int fhe_serve(const fhe_serve_engine *engines, int engine_count,
           size_t free_b = 0, total_b = 0;
           hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
           stats->min_free_bytes = std::min(stats->min_free_bytes, free_b);
-          const size_t need = fhe_host::batch_bytes(ctx, kind, count, limbs);
+          const size_t need = fhe_host::batch_bytes(
+              ctx, kind, E.coefficient_count - 1, count, limbs);
           if (free_b < need + options->reserve_bytes) {
             // wait for memory: only when something can free it
             stats->deferred_admissions++;
