@@ -34,10 +34,13 @@ struct Batch {
 };
 
 // Device bytes a batch of `count` jobs at `limbs` limbs may take beyond its
-// inputs: the key switch's extended limbs, digits, accumulators, partial sums
-// and coefficient-form trio, the prepared factors and NTT-form trio of its
+// inputs: the key switch's extended limbs, digits, accumulators and
+// coefficient-form trio, the prepared factors and NTT-form trio of its
 // products, and the texts of the composition (`degree` powers and the weighted
-// sum's, or the rotation chain).
+// sum's, or the rotation chain).  kFixedBytes: the partial sums, which only
+// batches of less than 256 blocks of 2 x 32 KiB have (ks_split), and as much
+// for the allocations' granularity.
+constexpr size_t kFixedBytes = size_t(32) << 20;
 size_t batch_bytes(const fhe_context *ctx, int kind, int degree, int count,
                    int limbs) {
   const auto &P = ctx->params;
@@ -45,14 +48,11 @@ size_t batch_bytes(const fhe_context *ctx, int kind, int degree, int count,
   const int64_t acc = 2 * ctx->ext_poly_words(mid);
   const auto plan =
       ctx->ks_plan(count, mid, count * (3 * int64_t(limbs) * P.n + acc));
-  const auto split =
-      fhe::ks_split(ctx->tables, P.partition_count(mid), count,
-                    limbs + P.alpha, ctx->lazy_key_switch);
   const int64_t texts = (kind == FHE_JOB_POLY ? degree + 5 : 6) * 2 * limbs;
   return size_t(plan.ext_words + ctx->ks_digits_words(plan.group, mid) +
-                count * split.groups * acc +
-                count * (10 * int64_t(limbs) + texts) * P.n) *
-         8;
+                count * (acc + (10 * int64_t(limbs) + texts) * P.n)) *
+             8 +
+         kFixedBytes;
 }
 
 } // namespace
