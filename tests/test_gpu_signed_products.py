@@ -78,3 +78,42 @@ def test_signed_products(gpu_lib, log_n, alpha, limbs):
         for lazy in (1, 0):
             same = np.array_equal(got[1 - lazy][c], want)
             assert same, (c, lazy)
+
+
+@pytest.mark.parametrize("log_n,alpha", [(13, 1), (14, 2), (16, 4)])
+def test_signed_values_elsewhere(gpu_lib, log_n, alpha):
+    """Transforms, decryption and key switching of values in (-q, q)."""
+    primes = fhe_amd.resolve_primes(log_n, alpha)
+    rng = np.random.Generator(np.random.PCG64(60 + log_n))
+    orc = Oracle(log_n, primes, alpha)
+    with fhe_amd.Context(log_n, alpha) as ctx:
+        n, mid = ctx.n, 1
+        limbs, key_mid = ctx.limbs_at(mid), ctx.key_moduli_id()
+        x = negate_some(rng, primes, mid,
+                        uniform(rng, primes, mid, (2, limbs, n)))
+        assert (x < 0).any()
+        same = []
+        for enter in (True, False):
+            d = ctx.to_device(x)
+            ctx.ntt(d, mid, enter=enter)
+            y = d.download()
+            same.append(np.array_equal(y, orc.ntt(x, mid, enter=enter)))
+            d.free()
+        for z in (y, x):
+            d = ctx.to_device(z)
+            ctx.intt(d, mid, post=1)
+            same.append(np.array_equal(d.download(), orc.intt(z, mid, post=1)))
+            d.free()
+        key = uniform(rng, primes, key_mid, ctx.key_shape(key_mid))
+        sk = uniform(rng, primes, 0, (ctx.chain_count, n))
+        dx, dk, ds = (ctx.to_device(v) for v in (x[None], key, sk))
+        pt, out = ctx.array((1, limbs, n)), ctx.array((1, 2, limbs, n))
+        ctx.decrypt(dx, ds, 0, pt, mid)
+        ctx.switch_key(dx, dk, key_mid, out, mid)
+        same.append(np.array_equal(pt.download()[0],
+                                   orc.decrypt(x, sk, 0, mid)))
+        same.append(np.array_equal(out.download()[0],
+                                   orc.switch_key(x, key, mid, key_mid)))
+        for arr in (dx, dk, ds, pt, out):
+            arr.free()
+    assert same == [True] * 6

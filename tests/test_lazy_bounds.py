@@ -1,10 +1,9 @@
-"""Bounds of the lazy transform arithmetic used by the representative-free
-stages (fhe_amd/csrc/ntt_r16.h): a model of the kLazySmall and kLazyLarge
-butterflies in exact integers checks, for worst-case inputs just below 2q,
-that every intermediate stays inside the stated bounds (so no 64-bit
-wrap-around can occur on the device) and that the residues equal the exact
-transform's.  The device results themselves are checked bit-exact against
-the oracle by the GPU tests."""
+"""Lazy arithmetic outside the butterflies (test_f64_bounds.py and
+test_lazy_large_bounds.py model those): ModDown's Shoup steps
+(fhe_amd/csrc/moddown.h) and the epilogue of the 64-bit lazy inverse
+transform (fhe_amd/csrc/ntt_r16.h), in exact integers against the reference's
+formulas.  The device results themselves are checked bit-exact against the
+oracle by the GPU tests."""
 import random
 
 import pytest
@@ -44,73 +43,6 @@ def root(q, n):
 
 def brev(x, b):
     return int(format(x, f"0{b}b")[::-1], 2)
-
-
-def forward(x, q, log_n, mode):
-    n = 1 << log_n
-    psi = root(q, n)
-    x, q2, top = list(x), 2 * q, 0
-    for s in range(log_n):
-        half = n >> (s + 1)
-        for g in range(1 << s):
-            w = pow(psi, brev((1 << s) + g, log_n), q)
-            wq = (w << 64) // q
-            for j in range(2 * g * half, 2 * g * half + half):
-                a, b = x[j], x[j + half]
-                if mode == "exact":
-                    t = w * b % q
-                    x[j], x[j + half] = (a + t) % q, (a - t) % q
-                    continue
-                if mode == "large" and a >= q2:
-                    a -= q2
-                t = shoup(b, w, wq, q)
-                x[j], x[j + half] = a + t, a + q2 - t
-                top = max(top, x[j], x[j + half])
-    return x, top
-
-
-def inverse(x, q, log_n, mode):
-    n = 1 << log_n
-    psi_inv = pow(root(q, n), -1, q)
-    x, q2, top = list(x), 2 * q, 0
-    for t in range(log_n):
-        half = 1 << t
-        for g in range(n >> (t + 1)):
-            w = pow(psi_inv, brev((n >> (t + 1)) + g, log_n), q)
-            wq = (w << 64) // q
-            for j in range(2 * g * half, 2 * g * half + half):
-                a, b = x[j], x[j + half]
-                if mode == "exact":
-                    x[j], x[j + half] = (a + b) % q, (a - b) * w % q
-                    continue
-                total, off = a + b, q2
-                if mode == "large":
-                    total = total - q2 if total >= q2 else total
-                else:
-                    off = q << (1 + t)
-                    assert b < off
-                x[j], x[j + half] = total, shoup(a + off - b, w, wq, q)
-                top = max(top, x[j], x[j + half])
-    return x, top
-
-
-@pytest.mark.parametrize("bits,mode", [(40, "small"), (41, "small"),
-                                       (60, "large"), (54, "large")])
-def test_lazy_butterflies_bounds_and_residues(bits, mode):
-    log_n = 8
-    q = ntt_prime(bits, 1 << log_n)
-    rng = random.Random(bits)
-    x = [2 * q - 1 - rng.randrange(64) for _ in range(1 << log_n)]
-    exact, _ = forward([v % q for v in x], q, log_n, "exact")
-    lazy, top = forward(x, q, log_n, mode)
-    assert [v % q for v in lazy] == exact
-    # forward: below 2q + 2q per stage (small), below 4q (large)
-    assert top < ((2 + 2 * log_n) * q if mode == "small" else 4 * q)
-    exact, _ = inverse([v % q for v in x], q, log_n, "exact")
-    lazy, top = inverse(x, q, log_n, mode)
-    assert [v % q for v in lazy] == exact
-    # inverse: below 2q * 2^stages (small; 2^59 after 16 stages for q < 2^42)
-    assert top < ((2 * q) << log_n if mode == "small" else 2 * q)
 
 
 @pytest.mark.parametrize("bits", [40, 54, 60])
@@ -153,14 +85,12 @@ def test_lazy_moddown_step_matches_reference_formula(bits):
         assert got == expect, (trial, v, steps)
 
 
-@pytest.mark.parametrize("bits,mode", [(40, "small"), (41, "small"),
-                                       (60, "large"), (54, "large")])
-def test_lazy_inverse_epilogue_folds_the_exit(bits, mode):
-    """The lazy inverse transforms' epilogue: one Montgomery product with
-    N^-1 R^-1 (mont_exit of the table's N^-1 R) in place of the product
-    with N^-1 R and the exit.  Over inputs up to the lazy bounds (2^59 for
-    primes below 2^42 after 16 stages, 2q otherwise) the result is below
-    2q and has the residue of the two-step form."""
+@pytest.mark.parametrize("bits", [43, 54, 60, 61])
+def test_lazy_inverse_epilogue_folds_the_exit(bits):
+    """The 64-bit lazy inverse transform's epilogue: one Montgomery product
+    with N^-1 R^-1 (mont_exit of the table's N^-1 R) in place of the product
+    with N^-1 R and the exit.  Over values below 4q, brought below 2q first,
+    the result is below 2q and has the residue of the two-step form."""
     log_n = 16
     q = ntt_prime(bits, 1 << log_n)
     r_bits = 62
@@ -174,10 +104,11 @@ def test_lazy_inverse_epilogue_folds_the_exit(bits, mode):
 
     ninv = pow(1 << log_n, -1, q) * (1 << r_bits) % q  # N^-1 R
     folded = mont(ninv, 1)                             # mont_exit: N^-1
-    top = (1 << 59) if mode == "small" else 2 * q
+    top = 4 * q
     rng = random.Random(bits + 1)
-    for v in [0, 1, q - 1, q, 2 * q - 1, top - 1] + \
+    for v in [0, 1, q - 1, q, 2 * q - 1, 2 * q, top - 1] + \
             [rng.randrange(top) for _ in range(2000)]:
+        v = v - 2 * q if v >= 2 * q else v
         y = mont(v, folded)
         assert y < 2 * q
         assert y % q == mont(mont(v, ninv), 1) % q
