@@ -859,7 +859,7 @@ def stage_report(stages, step_ms, prof_steps, shape, peaks):
         valu["kernel_achieved"] = round(k, 0)
         valu["kernel_frac"] = round(k / peaks[0], 4)
     roofline = {
-        "bound": "valu",
+        "bound": "hbm",
         "kernel": name,
         "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": round(gbs / HBM_PEAK_GBS, 4),
@@ -873,12 +873,16 @@ def stage_report(stages, step_ms, prof_steps, shape, peaks):
         "step_frac": round(step_gbs / HBM_PEAK_GBS, 4),
         "valu": valu,
         "valu_issue": valu_issue(name, batch, avg),
-        "binding": "VALU: 62-bit modular products from 32-bit multiply-adds; "
-                   "the HBM fractions are of the algorithmic bytes, the "
-                   "product fractions of the Shoup-product rate measured "
-                   "on this device (fhe_modmul_peak), valu_issue the "
-                   "kernel's VALU instructions (rocprofv3 SQ_INSTS_VALU) "
-                   "against the issue rate of the product probe",
+        "binding": "memory traffic first: the step's transforms pass through "
+                   "HBM twice; the key inner product (24 of 29 limbs in "
+                   "FP64, 5 in 64-bit integers) saturates neither HBM nor "
+                   "VALU issue and waits on its loads.  The HBM fractions "
+                   "are of the algorithmic bytes, the product fractions of "
+                   "the Shoup-product rate measured on this device "
+                   "(fhe_modmul_peak; FP64 products exceed it), valu_issue "
+                   "the kernel's VALU instructions (rocprofv3 "
+                   "SQ_INSTS_VALU) against the issue rate of the product "
+                   "probe",
     }
     return breakdown, roofline
 

@@ -803,7 +803,8 @@ struct fhe_context {
                      ext_limbs, moduli_id, fhe::kInttExitReduce, stream);
   }
 
-  // The key-independent half of key switching on the fused path (N = 2^13 .. 2^16):
+  // The key-independent half of key switching on the fused path
+  // (N = 2^13 .. 2^16; any N for a bootstrap key's stages):
   // ModUp of every partition and the first forward NTT pass of every
   // extended limb into ext [count][parts][ext][N] (CKKSCore::decompose,
   // src/ckks/core_key_switch.cpp:434-460, up to its second NTT pass).

@@ -8,8 +8,8 @@
 namespace fhe {
 
 // Whether a batched transform may use the lazy arithmetic (ntt_r16.h; the
-// radix-16 sizes): its outputs are other representatives of the same
-// residues, forward outputs below 2q, inverse outputs with the exit
+// radix-16 sizes, exact elsewhere): its outputs are other representatives of
+// the same residues, forward outputs below 2q, inverse outputs with the exit
 // canonical.
 //
 // The exact inverse with the exit (kInttExit) is canonical too but for zero
@@ -94,8 +94,8 @@ void ntt_forward_second(const DeviceTables &t, const int64_t *src,
                         int moduli_id, hipStream_t stream,
                         LazySpec lazy = LazySpec());
 
-// Fused key-switching core for N = 2^13 .. 2^16: for each tile of each extended limb
-// and ciphertext, the low-bit forward NTT pass of every partition's
+// Fused key-switching core for N = 2^13 .. 2^16: for each tile of each
+// extended limb and ciphertext, the low-bit forward NTT pass of every partition's
 // extended polynomial, the key inner product over all partitions
 // (src/ckks/core_key_switch.cpp:318-336) and the low-bit inverse NTT pass of
 // both accumulators.  ext: [count][parts][ext_limbs][N] after

@@ -8,8 +8,10 @@
 // finishes the forward NTT of that tile (the high-bit pass ran before),
 // multiplies by both key halves and accumulates in registers; it then runs
 // the first (low-bit) pass of the inverse NTT on both accumulators before a
-// single write.  Each coefficient sees the reference's exact sequence of
-// butterflies, products and guards.
+// single write.  With lazy = false each coefficient sees the reference's exact
+// sequence of butterflies, products and guards; the lazy forms (ntt_r16.h),
+// partial sums and transforms taken from the source's NTT form keep the
+// residues only, which is what the canonical accumulators depend on.
 #include <algorithm>
 
 #include "kernels.h"
@@ -396,6 +398,13 @@ void launch_staged_modup(const DeviceTables &t, const int64_t *x,
 // 464 blocks, 423 -> 468 us with three groups, whose sums then cost more than
 // the idle slots did).
 constexpr int64_t kSplitTarget = 256;
+
+// The second inverse pass adds the groups' kF64 values as they are, each below
+// 2^8 (q / 2 + 2) after eight stages from centred sums: integers below 2^53.
+// (kLazyLarge sums are brought below 4q at every step.)
+static_assert(uint64_t(kKsMaxGroups) * 256 * (kF64Bound / 2 + 2) <
+                  uint64_t(1) << 53,
+              "the partial sums must stay exact in doubles");
 
 KsSplit ks_split(const DeviceTables &t, int parts, int count, int ext_limbs,
                  bool lazy) {

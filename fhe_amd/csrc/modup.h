@@ -82,8 +82,9 @@ __device__ __forceinline__ int64_t extend_limb(const int64_t (&d)[MAXZ],
 // canonicalizing INTT): Shoup products with the standard-form constants
 // (pairs {c, floor(c 2^64 / q)} at es + 2 (j ext + i)).  Primes below 2^42
 // keep the plain sum (below 4 * size * q); larger primes keep the sum below
-// 4q (short Shoup products), below the forward transform's 8q.  nq = 2^64 - q, opaque to the
-// compiler (opaque_neg), for the products and the subtraction of 4q.
+// 4q (short Shoup products), below the forward transform's 8q.
+// nq = 2^64 - q, opaque to the compiler (opaque_neg), for the products and
+// the subtraction of 4q.
 template <int MAXZ>
 __device__ __forceinline__ int64_t extend_limb_lazy(const int64_t (&d)[MAXZ],
                                                     int size, int i,

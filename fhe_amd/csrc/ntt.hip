@@ -1,11 +1,14 @@
 // Batched negacyclic NTT / INTT for gfx950.
 //
-// Butterflies are exactly the reference's radix-2 formulas
-// (src/operation/ntt.cpp:46-134 Cooley-Tukey, :177-272 Gentleman-Sande), so
-// every lazy representative in [0, 2q) matches.  The transform of one limb is
-// split into at most two passes over HBM: each pass owns a contiguous range of
-// index bits, loads a 4096-element tile of independent sub-transforms into
-// LDS and runs all of that range's radix-2 stages there.
+// Without lazy arithmetic the butterflies are exactly the reference's radix-2
+// formulas (src/operation/ntt.cpp:46-134 Cooley-Tukey, :177-272
+// Gentleman-Sande), so every lazy representative in [0, 2q) matches; the lazy
+// forms (ntt_r16.h) give other representatives of the same residues, and
+// where a zero residue's representative matters its limb is recomputed exactly
+// (repair_zero_kernel).  The transform of one limb is split into at most two
+// passes over HBM: each pass owns a contiguous range of index bits and runs
+// all of that range's radix-2 stages on 4096-element tiles of independent
+// sub-transforms, in registers for N = 2^13 .. 2^16 and in LDS otherwise.
 //
 //   forward  stage s flips index bit log_n-1-s; group of element i uses
 //            root[2^s - 1 + (i >> (log_n - s))]
@@ -410,7 +413,7 @@ namespace {
 // (the rule: a zero residue comes up once in 2^40 coefficients).  The block
 // walks the limb's tiles pass by pass; its own stores of one pass are what
 // it reads in the next, behind a block barrier.  bound: latency of the
-// launch, 3 us; a flagged limb takes about 0.2 ms.
+// launch, 5 us for 800 limbs; a flagged limb takes about 0.2 ms.
 struct RepairArgs {
   const uint32_t *zero; // [count][limbs]
   // the NTT-form source polynomial of ciphertext c at z + c * z_stride, or,

@@ -379,8 +379,10 @@ __device__ __forceinline__ void r16_exchange_words(V (&x)[16], uint32_t *lds,
 // (prime p); the pass covers index bits [b, b + L); COLS is b > 0.  pre
 // (forward, per prime) multiplies every loaded value first; post (inverse)
 // is the InttPost epilogue; last = the pass completes a forward transform.
+// The first pass of a lazy inverse takes any representatives, that of a lazy
+// forward transform any with pre or in kF64, else values in [0, 8q).
 // zero (lazy inverse): a flag word of the limb, cleared by the first pass and
-// set by the last one where a canonical result is zero (repair_zero_limb).
+// set by the last one where a canonical result is zero (repair_zero_kernel).
 // more (lazy second inverse pass): this limb of the first of more_count
 // buffers, more_stride words apart, that are added to the source.
 // OPAQUE: the pass runs inside a persistent loop (opaque_tid).
