@@ -274,10 +274,13 @@ void for_class_runs(const DeviceTables &t, int moduli_id, int limbs, F &&f) {
 }
 
 // Launches with fewer blocks than this choose the arithmetic per block (four
-// blocks per CU: above it the smaller kernel's extra waves have work).  One
-// launch per class against one mixed launch: 8.28 against 11.27 ms for 32
-// Gold HMults (14848 blocks), 1020 against 1183 us for 8 at N = 2^15 (1280);
-// below, the second launch would wait for the last blocks of the first.
+// blocks per CU: above it the extra waves of the smaller extension kernel have
+// work, and the key product's FP64 blocks do not carry the 64-bit form's code
+// and registers).  One launch per class against one mixed launch, both
+// kernels together and before the key product's range checks: 8.28 against
+// 11.27 ms for 32 Gold HMults (14848 blocks), 1020 against 1183 us for 8 at
+// N = 2^15 (1280); below, the second launch would wait for the last blocks of
+// the first.
 constexpr int64_t kSplitBlocks = 1024;
 
 } // namespace
